@@ -137,12 +137,4 @@ int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int resca
                       const float* w, int max_rows, float* out, void* workspace, size_t workspace_bytes,
                       mm_stream_t stream, const char* who, int accumulate = 0);
 
-// Decode workspace of n routes whose sorted positions lie below npos, and the decode path over such a
-// permutation (routes of experts above cap left out) added to / written into out; no argument checks.
-size_t decode_ws_bytes(int n, int npos, int E, int H, int I);
-int decode_perm_launch(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids,
-                       const float* w, const int32_t* offsets, const int32_t* order, const int32_t* active,
-                       const int32_t* nactive, int npos, int cap, float* out, int accumulate, void* workspace,
-                       hipStream_t s);
-
 }  // namespace mm

@@ -3,12 +3,15 @@
 // patches/vllm-exl3-host-dma.patch:182-201, runtime/dma_gemm.py:5-26, which reconstruct fp16 weights and run a
 // 128x128 GEMM).
 //
-// Launches: mm_permute (sorted positions) -> k_fat_prep (transformed inputs per sorted position) -> k_fat_plan
-// (expert records and the two tile lists) -> k_fat<0, 8>, k_fat16<0, 2> (gate/up) -> k_fat16<1, 4>, k_fat16<1, 2>
-// (down) -> k_fat_combine.
+// Launches: mm_permute (sorted positions) -> k_fat_plan (expert records, row groups, tile lists) -> k_fat_prep
+// (transformed inputs per row group) -> k_fat<0, 8>, k_mid<0> (gate/up) -> k_fat16<1, 4>, k_mid<1> (down) -> k_fat_combine.
 //
-// A workgroup (k_fat: 8 waves, two per SIMD; k_fat16: 16 waves, four per SIMD) owns a tile of 256 routes (sorted
-// positions of one expert; 128 for an expert's last <= 128 routes) x 256 output columns:
+// An expert's routes (sorted positions) are taken in row groups of 32, whose inputs are stored in MFMA operand order: per
+// matrix and 32-element step one contiguous 2 KB, chunk g (8 elements: tile rows 0 and 1 of decode window g) of row r at
+// 16 (32 g + r). A wave's operand load is then one contiguous KB, whichever kernel reads it.
+//
+// k_mid takes tiles of at most 96 routes (below). k_fat (8 waves, two per SIMD) and k_fat16 (16 waves) own a tile of 256
+// routes of one expert x 256 output columns, for calls with many of them:
 //   gate/up (MODE 0): gate columns 128 c .. 128 c + 127 and the same up columns, so the epilogue holds both and
 //                     applies the output transforms, SwiGLU and the down-input transform of that 128-block (the
 //                     transforms act within 128-blocks);
@@ -28,7 +31,27 @@ namespace mm {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int FT_BIG = 256;         // routes per tile (8 row blocks per row-wave)
-constexpr int FT_SMALL = 128;       // routes per tile for an expert's remainder of at most 128 routes
+constexpr int FT_MID = 96;          // routes per tile of k_mid
+constexpr int FT_BIG_MIN = 193;     // smallest remainder of c / 256 that takes a 256-route tile (two FT_MID tiles hold 192)
+
+// Where 256-route tiles are used. The kernels of the two tile sizes add an expert's products in different orders.
+//   a fused call: where it has workgroups of 256-route tiles for at least three rounds of the GPU (one fits a CU). Fewer
+//     leave CUs idle that FT_MID-route tiles fill: 3 tiles (48 workgroups) of a 512-token call took 214 us of its 1,540
+//     where FT_MID-route tiles took 60; at 64 tiles (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at
+//     297 (16,384 tokens) 8.25 and 8.65.
+//   the other entry points, whose rows must have the same bits whichever other experts a call computes (a layer in one call
+//     or in staging batches): by the expert's own routes, from four such tiles on. Staging batches hold few experts: 12
+//     tiles of a batch of 16 experts took 189 us of its 470, as FT_MID-route tiles 50.
+struct BigRule
+{
+    int min_tiles;      // of the call
+    int min_rows;       // of the expert
+};
+constexpr int FT_BIG_WORK = 3 * 256;
+constexpr int FT_BIG_ROWS = 1024;
+constexpr int GRP_ROWS = 32;        // rows of a row group
+constexpr int GRP_HALVES = 1024;    // one matrix's 32-element step of a row group
+constexpr int PREP_BLOCKS = 4;      // 128-blocks per input transform workgroup
 constexpr int FT_BN = 256;          // output columns per tile
 constexpr int FT_WAVES = 8;
 constexpr int FT_THREADS = 64 * FT_WAVES;
@@ -38,20 +61,27 @@ constexpr int FT_PT = 5;            // trellis steps in flight
 constexpr int FT_TS = FT_PT + 1;    // trellis ring slots
 constexpr int FT_PLAN_MAX = 1024;   // active experts the plan kernel handles
 
+// A tile of routes of one expert: rows row0 .. of record ai, whose inputs start at row group `group`.
+struct FatTile
+{
+    int32_t ai, row0, group, pad;
+};
+
 struct FatArgs
 {
     const ExpertRec* rec;         // [max_active] active experts (permutation order)
-    const int32_t* nactive;       // [1]
-    const int32_t* tile_off;      // [max_active + 1] first tile of each active expert in this launch's list
-    const int32_t* big_off;       // [max_active + 1] 256-route tiles (a 128-route tile follows them)
-    const uint16_t* xa;           // mode 0: [n][H/32][gate 32, up 32]; mode 1: [n][I] (operand order)
+    const FatTile* tiles;         // this launch's tiles
+    const int32_t* ntiles;        // [1]
+    const uint16_t* xa;           // inputs in row groups: mode 0 [groups][H/32][gate, up][1024], mode 1 [groups][I/32][1024]
     const uint16_t* svh13;        // [E][2][I]
     const uint16_t* suh2;         // [E][I]
     const uint16_t* svh2;         // [E][H]
     const int32_t* route_at;      // [n] flat route index of each sorted position
-    uint16_t* xd;                 // mode 0 output [n][I] (operand order)
+    uint16_t* xd;                 // mode 0 output: the down inputs, in row groups
     float* Y;                     // mode 1 output [n_routes][H] (per route), fp32 or (YH) fp16 bits
-    int H, I, K, N, nunits, max_active;
+    const float* xs;              // input sums [groups][nxs][NA][32] (affine decode), NA = 2 in mode 0, 1 in mode 1
+    float* xds;                   // mode 0 output: sums of the down inputs [groups][nxds = I / 128][32]
+    int H, I, K, N, nunits, nxs, nxds;
     float limit;
 };
 
@@ -130,31 +160,25 @@ __device__ __forceinline__ int lane8_k(int lane, int i)
     return 32 * ((lane >> 2) & 3) + 2 * (lane & 3) + (i & 1) + 8 * ((i >> 1) & 1) + 16 * (i >> 2);
 }
 
+// One 16-lane group transforms row `rl` of a row group: blocks b0 .. b1 - 1 of the token's row, both matrices (the
+// input is read once), two blocks per pass, all loaded before any is used.
 template <int XD>
-// cnt_e (optional): the expert's route count, read with the row and compared only before the stores (rows of
-// experts with cnt_e[0] <= cap are not stored), so it costs no round trip of its own.
-__device__ __forceinline__ void fat_prep_row_t(const void* x, size_t row, int e, int pos, const uint16_t* suh13,
-                                               uint16_t* xa, int H, const int32_t* cnt_e, int cap)
+__device__ __forceinline__ void fat_prep_row(const void* x, size_t row, const uint16_t* su0, uint16_t* dst, int H,
+                                             int b0, int b1, float (&sum)[2])
 {
-    int ce = cnt_e ? cnt_e[0] : cap + 1;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane & 3, q = (lane >> 2) & 3, bl = lane >> 4;
-    const int nb = H / 128;
+    const int lane = threadIdx.x & 63;
+    const int g = lane & 3, q = (lane >> 2) & 3;
     const Lane8Signs sg = lane8_signs(lane);
-    const uint16_t* su0 = suh13 + (size_t)e * 2 * H;       // gate; up follows
-    uint16_t* dst = xa + (size_t)pos * 2 * H + 8 * g;
     // raw words of element pair (t, h): fp16 / bf16 input as one dword, fp32 as two
     using Raw = typename std::conditional<XD == MM_DTYPE_F32, uint2, uint32_t>::type;
-    // lane group bl of wave w takes blocks w + 4 bl + 16 i of the row, both matrices (the input is read once): two
-    // blocks per pass, all loaded before any is used (blocks past the row reload its last block and are not stored)
-    for (int f0 = wave + 4 * bl; f0 < nb; f0 += 32)
+    for (int f0 = b0; f0 < b1; f0 += 2)
     {
         Raw xr[2][4];
         uint32_t sr[2][2][4];
 #pragma unroll
         for (int it = 0; it < 2; ++it)
         {
-            const int k0 = min(f0 + 16 * it, nb - 1) * 128 + 32 * q + 2 * g;
+            const int k0 = min(f0 + it, b1 - 1) * 128 + 32 * q + 2 * g;
 #pragma unroll
             for (int th = 0; th < 4; ++th)
             {
@@ -167,13 +191,11 @@ __device__ __forceinline__ void fat_prep_row_t(const void* x, size_t row, int e,
                 sr[it][1][th] = *reinterpret_cast<const uint32_t*>(su0 + H + k);
             }
         }
-        asm volatile("" : "+v"(ce));       // the count is first used here, after the row's loads
-        if (ce <= cap) return;
 #pragma unroll
         for (int it = 0; it < 2; ++it)
         {
-            const int b = f0 + 16 * it;
-            if (b >= nb) break;
+            const int b = f0 + it;
+            if (b >= b1) break;
             // th = 2 t + h: elements 8 h + 16 t (+ 0, 1) of the lane's column pair go to xv[4 t + 2 h + j]
             float xv[8];
 #pragma unroll
@@ -208,77 +230,73 @@ __device__ __forceinline__ void fat_prep_row_t(const void* x, size_t row, int e,
                     v[i + 1] = xv[i + 1] * h2f((uint16_t)(sr[it][m][th] >> 16));
                 }
                 fwht128_lane8(v, sg);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) sum[m] += r16(v[i] * HAD);
                 uint4 o;
                 o.x = (uint32_t)f2h(v[0] * HAD) | ((uint32_t)f2h(v[1] * HAD) << 16);
                 o.y = (uint32_t)f2h(v[2] * HAD) | ((uint32_t)f2h(v[3] * HAD) << 16);
                 o.z = (uint32_t)f2h(v[4] * HAD) | ((uint32_t)f2h(v[5] * HAD) << 16);
                 o.w = (uint32_t)f2h(v[6] * HAD) | ((uint32_t)f2h(v[7] * HAD) << 16);
-                // a nontemporal store: the 16 KB per route (2 GB at 16k tokens) stream past the caches, which
-                // their readers' tiles would otherwise lose to them (16k layer 9.67-9.79 -> 9.50-9.52 ms)
-                __builtin_nontemporal_store(u32x4{ o.x, o.y, o.z, o.w },
-                                            reinterpret_cast<u32x4*>(dst + (size_t)(4 * b + q) * 64 + m * 32));
+                *reinterpret_cast<uint4*>(dst + ((size_t)(4 * b + q) * 2 + m) * GRP_HALVES + g * 256) = o;
             }
         }
     }
 }
 
-__device__ __forceinline__ void fat_prep_row(const void* x, int x_dtype, size_t row, int e, int pos,
-                                             const uint16_t* suh13, uint16_t* xa, int H, const int32_t* cnt_e, int cap)
+// One workgroup per (row group, PREP_BLOCKS 128-blocks of the input row): wave w transforms rows 4 w .. 4 w + 3, so the
+// workgroup's waves together write whole 512-byte runs of the row group. The token of a position is token_sorted's
+// (a position of a token outside [0, T) is left unwritten), or order[pos] / topk.
+__global__ __launch_bounds__(512) void k_fat_prep(const void* x, int x_dtype, const int32_t* order,
+                                                  const int64_t* token_sorted, const ExpertRec* rec, const int2* groups,
+                                                  const int32_t* ngroups, const uint16_t* suh13, uint16_t* xa, float* xs,
+                                                  int topk, int T, int H)
 {
-    if (x_dtype == MM_DTYPE_F16)
-        fat_prep_row_t<MM_DTYPE_F16>(x, row, e, pos, suh13, xa, H, cnt_e, cap);
-    else if (x_dtype == MM_DTYPE_BF16)
-        fat_prep_row_t<MM_DTYPE_BF16>(x, row, e, pos, suh13, xa, H, cnt_e, cap);
-    else
-        fat_prep_row_t<MM_DTYPE_F32>(x, row, e, pos, suh13, xa, H, cnt_e, cap);
-}
-
-__global__ __launch_bounds__(256) void k_fat_prep(const void* x, int x_dtype, const int32_t* e_sorted,
-                                                  const int32_t* counts, const int32_t* offsets, const int32_t* order,
-                                                  const uint16_t* suh13, uint16_t* xa, int topk, int E, int H, int cap)
-{
-    const int pos = blockIdx.x;
-    // round trip 1: the routed count, the route and its expert (pos < n: in range past the routed count too)
-    const int nvalid = offsets[E];
-    const int s = order[pos], e = e_sorted[pos];
-    if (pos >= nvalid || (s | e) < 0) return;        // s, e >= 0: the test only keeps their loads before the branch
-    // round trip 2: the expert's route count with the row's loads; rows of experts at or below cap are not stored
-    fat_prep_row(x, x_dtype, (size_t)(s / topk) * H, e, pos, suh13, xa, H, counts + e, cap);
-}
-
-// Sorted-route form: position pos belongs to the expert e with offsets[e] <= pos < offsets[e + 1] (binary search
-// over the E + 1 offsets) and to token token_sorted[pos]; only positions of experts with counts[e] > 0 (the
-// selected fat experts) are transformed.
-__global__ __launch_bounds__(256) void k_fatb_prep(const void* x, int x_dtype, const int64_t* token_sorted,
-                                                   const int32_t* counts, const int32_t* offsets,
-                                                   const uint16_t* suh13, uint16_t* xa, int T, int E, int H)
-{
-    const int pos = blockIdx.x;
-    if (pos >= offsets[E]) return;
-    int lo = 0, hi = E;                 // largest e with offsets[e] <= pos
-    while (hi - lo > 1)
-    {
-        const int mid = (lo + hi) >> 1;
-        if (offsets[mid] <= pos) lo = mid; else hi = mid;
-    }
-    const int e = lo;
-    if (counts[e] <= 0 || pos >= offsets[e] + counts[e]) return;
-    const int64_t t = token_sorted[pos];
+    const int G = blockIdx.x, rl = threadIdx.x >> 4;
+    if (G >= ngroups[0]) return;
+    const int2 gi = groups[G];                       // record and first row
+    const ExpertRec* r = rec + gi.x;
+    if (gi.y + rl >= r->cnt) return;
+    const int pos = r->first + gi.y + rl;
+    const int64_t t = token_sorted ? token_sorted[pos] : (int64_t)(order[pos] / topk);
     if (t < 0 || t >= T) return;
-    fat_prep_row(x, x_dtype, (size_t)t * H, e, pos, suh13, xa, H, nullptr, 0);
+    const int nb = H / 128, b0 = blockIdx.y * PREP_BLOCKS, b1 = min(nb, b0 + PREP_BLOCKS);
+    const uint16_t* su0 = suh13 + (size_t)r->e * 2 * H;       // gate; up follows
+    uint16_t* dst = xa + (size_t)G * 64 * H + rl * 8;          // a row group: 32 rows x 2 matrices x H
+    float sum[2] = { 0.0f, 0.0f };
+    if (x_dtype == MM_DTYPE_F16)
+        fat_prep_row<MM_DTYPE_F16>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+    else if (x_dtype == MM_DTYPE_BF16)
+        fat_prep_row<MM_DTYPE_BF16>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+    else
+        fat_prep_row<MM_DTYPE_F32>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+    {
+        sum[m] += xor_lane<1>(sum[m]);
+        sum[m] += xor_lane<2>(sum[m]);
+        sum[m] += xor_lane<4>(sum[m]);
+        sum[m] += xor_lane<8>(sum[m]);
+        if ((threadIdx.x & 15) == 0) xs[(((size_t)G * gridDim.y + blockIdx.y) * 2 + m) * GRP_ROWS + rl] = sum[m];
+    }
 }
 
-// Expert records and the tile lists of the experts with more than cap routes. An expert of c routes gets
-// c / 256 tiles of 256 routes; a remainder r = c % 256 takes one more 256-route tile if r > 128 (a 256-route step
-// costs less than two 128-route steps), else one 128-route tile. off_big / off_small = tiles of active experts
-// 0 .. a-1 in each list.
+// 256-route tiles of an expert with c routes; the rest (at most FT_BIG_MIN - 1 routes) goes to FT_MID-route tiles.
+__device__ __forceinline__ int fat_big_tiles(int c) { return c / FT_BIG + (c % FT_BIG >= FT_BIG_MIN ? 1 : 0); }
+
+// Expert records, row groups and the tile lists of the experts with more than cap routes, one workgroup: thread a counts
+// expert a's tiles and groups, the lists are then filled by all threads, each entry finding its expert by a binary search
+// over the sums in LDS. totals = 256-route tiles, FT_MID-route tiles, row groups. The FT_MID-route list holds the tiles of
+// three row groups first, then those of two, then those of one: the longest start first.
 __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts, const int32_t* offsets,
                                                          const int32_t* active, const int32_t* nactive,
                                                          const int64_t* gate, const int64_t* up, const int64_t* down,
-                                                         ExpertRec* rec, int32_t* off_big, int32_t* off_small,
-                                                         int max_active, int cap)
+                                                         ExpertRec* rec, FatTile* big, FatTile* mid, int2* groups,
+                                                         int32_t* totals, int max_active, int cap, BigRule rule)
 {
-    __shared__ int s_w[2][FT_PLAN_MAX / 64];
+    // lists: 256-route tiles; tiles of three, two and one row groups; row groups
+    constexpr int NL = 5;
+    __shared__ int s_w[NL][FT_PLAN_MAX / 64];
+    __shared__ int s_off[NL][FT_PLAN_MAX + 1];             // exclusive sums
     const int a = threadIdx.x, lane = a & 63, wave = a >> 6;
     const int nact = min(nactive[0], max_active);
     int c = 0;
@@ -289,60 +307,103 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
         ExpertRec r{ e, c, offsets[e], 0, { gate[e], up[e], down[e] }, 0 };
         rec[a] = r;
     }
-    int tb = 0, ts = 0;
-    if (c > cap)
-    {
-        const int r = c % FT_BIG;
-        tb = c / FT_BIG + (r > FT_SMALL ? 1 : 0);
-        ts = (r > 0 && r <= FT_SMALL) ? 1 : 0;
-    }
-    const int ib = wave_incl_scan(tb), is = wave_incl_scan(ts);
-    if (lane == 63)
-    {
-        s_w[0][wave] = ib;
-        s_w[1][wave] = is;
-    }
-    __syncthreads();
-    int bb = 0, bs = 0, nb = 0, ns = 0;
-    for (int w = 0; w < FT_PLAN_MAX / 64; ++w)
-    {
-        if (w < wave)
+    if (c <= cap) c = 0;
+    // exclusive sums of list i into s_off[i]
+    auto scan = [&](int i, int v) {
+        const int incl = wave_incl_scan(v);
+        if (lane == 63) s_w[i][wave] = incl;
+        __syncthreads();
+        int base = 0, total = 0;
+        for (int w = 0; w < FT_PLAN_MAX / 64; ++w)
         {
-            bb += s_w[0][w];
-            bs += s_w[1][w];
+            if (w < wave) base += s_w[i][w];
+            total += s_w[i][w];
         }
-        nb += s_w[0][w];
-        ns += s_w[1][w];
-    }
-    if (a < max_active)
+        s_off[i][a] = base + incl - v;
+        if (a == 0) s_off[i][FT_PLAN_MAX] = total;
+        return total;
+    };
+    int nbig = c >= rule.min_rows ? fat_big_tiles(c) : 0;
+    int tbig = scan(0, nbig);
+    if (tbig < rule.min_tiles)                                    // uniform: too few to fill the GPU
     {
-        off_big[a] = bb + ib - tb;
-        off_small[a] = bs + is - ts;
+        __syncthreads();
+        nbig = 0;
+        tbig = scan(0, 0);
     }
+    const int rest = max(c - nbig * FT_BIG, 0), full = rest / FT_MID, r = rest % FT_MID;
+    const int t3 = scan(1, full + (r > 2 * GRP_ROWS ? 1 : 0));
+    const int t2 = scan(2, r > GRP_ROWS && r <= 2 * GRP_ROWS ? 1 : 0);
+    const int t1 = scan(3, r > 0 && r <= GRP_ROWS ? 1 : 0);
+    const int tg = scan(4, (c + GRP_ROWS - 1) / GRP_ROWS);
     if (a == 0)
     {
-        off_big[max_active] = nb;
-        off_small[max_active] = ns;
+        totals[0] = tbig;
+        totals[1] = t3 + t2 + t1;
+        totals[2] = tg;
+    }
+    __syncthreads();
+    // entry j of list i belongs to the last expert whose sum is at most j (later experts without entries share it)
+    auto owner = [&](int i, int j) {
+        int lo = 0, hi = FT_PLAN_MAX;
+        while (hi - lo > 1)
+        {
+            const int m = (lo + hi) >> 1;
+            if (s_off[i][m] <= j) lo = m; else hi = m;
+        }
+        return lo;
+    };
+    for (int j = a; j < tbig; j += FT_PLAN_MAX)
+    {
+        const int o = owner(0, j), row0 = (j - s_off[0][o]) * FT_BIG;
+        big[j] = FatTile{ o, row0, s_off[4][o] + row0 / GRP_ROWS, 0 };
+    }
+    for (int j = a; j < t3 + t2 + t1; j += FT_PLAN_MAX)
+    {
+        const int i = j < t3 ? 1 : j < t3 + t2 ? 2 : 3, k = j - (i == 1 ? 0 : i == 2 ? t3 : t3 + t2);
+        const int o = owner(i, k);
+        // the tiles of three row groups come first within an expert's rest; a shorter one follows them
+        const int before = i == 1 ? k - s_off[1][o] : s_off[1][o + 1] - s_off[1][o];
+        const int row0 = (s_off[0][o + 1] - s_off[0][o]) * FT_BIG + before * FT_MID;
+        mid[j] = FatTile{ o, row0, s_off[4][o] + row0 / GRP_ROWS, 0 };
+    }
+    for (int j = a; j < tg; j += FT_PLAN_MAX)
+    {
+        const int o = owner(4, j);
+        groups[j] = make_int2(o, (j - s_off[4][o]) * GRP_ROWS);
     }
 }
 
-// LDS slot of 16-byte chunk q of row r of an input stage whose rows hold NA x 64 bytes (NA = 2: gate chunks 0 .. 3,
-// up chunks 4 .. 7): the 16 rows one MFMA operand read covers fall in distinct 16-byte bank groups both for 8
-// lanes over 32 banks and for 16 lanes over 64 banks.
-template <int NA>
-__device__ __forceinline__ int chunk_slot(int q, int r)
+// Work item of this workgroup. The grid is sized for the most tiles a call can have; the work = tiles x column units of
+// this call is spread evenly over the 8 XCDs (workgroup b runs on XCD b % 8), and consecutive work items (the column
+// units of one tile, then the next tile of the same expert) stay on one XCD, so they share its L2 for the inputs and
+// the trellis.
+__device__ __forceinline__ bool fat_work(const FatArgs& a, int& mt, int& nu)
 {
-    if constexpr (NA == 2) return q ^ (((r >> 1) & 7) ^ ((r & 1) << 2));
-    else return q ^ (((r >> 1) ^ (r >> 2)) & 3);
+    const int work = a.ntiles[0] * a.nunits, per_xcd = (work + 7) >> 3;
+    const int L = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || L >= work) return false;
+    mt = L / a.nunits;
+    nu = L % a.nunits;
+    return true;
+}
+
+// A wave-uniform pointer for a buffer descriptor (each half widened as uint32_t: readfirstlane returns int).
+__device__ __forceinline__ void* uniform_ptr(const void* p)
+{
+    const uint64_t v = (uint64_t)(uintptr_t)p;
+    const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return reinterpret_cast<void*>((uintptr_t)((uint64_t)l | ((uint64_t)h << 32)));
 }
 
 // Epilogue of a fat tile from the transposed fp16 C tile in LDS (column c at c * CS halves, the raw GEMM outputs
 // rounded to fp16): gate/up (MODE 0) applies the output transforms, SwiGLU and the down-input transform of the
 // tile's 128-block and writes the down input in operand order; down (MODE 1) applies the output transform of its
 // two 128-blocks and writes per-route rows. The C tile is complete (the caller's barrier) when this runs.
-template <int MODE, int CS, bool YH, int NW = FT_WAVES>
+template <int MODE, int CS, bool YH, int NW = FT_WAVES, bool SUMS = false>
 __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16_t* C, int rows, int pos0, int e,
-                                                  int nu, int wave, int lane)
+                                                  int nu, size_t grp, int wave, int lane)
 {
     // Transforms in the layout of fwht128_lane8: per pass a wave takes 8 rows; lane (rpair, q, g) = (lane >> 4,
     // (lane >> 2) & 3, lane & 3) holds rows r0 + 2 rpair and r0 + 2 rpair + 1 (one dword of the transposed tile per
@@ -373,8 +434,8 @@ __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16
             suv[i] = h2f(svu[kk[i]]);
             sdv[i] = h2f(sd[kk[i]]);
         }
-        // operand order: the lane's 8 elements are positions 32 q + 8 g .. + 7 of the block, v[i] at + i
-        const int od = c0 + 32 * ((lane >> 2) & 3) + 8 * (lane & 3);
+        // the lane's 8 elements are chunk g of step c0 / 32 + q of its row's group
+        uint16_t* od = a.xd + (size_t)(c0 / 32 + ((lane >> 2) & 3)) * GRP_HALVES + 256 * (lane & 3);
         for (int r0 = 8 * wave; r0 < rows; r0 += 8 * NW)
         {
             const int r = r0 + 2 * rpair;
@@ -400,6 +461,20 @@ __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16
                     xv[i] = r16(act_gu(gg, uu, a.limit)) * sdv[i];
                 }
                 fwht128_lane8(xv, sg);
+                if constexpr (SUMS)
+                {
+                    // sum of the block's 128 rounded values over its 16 lanes
+                    float sum = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) sum += r16(xv[i] * HAD);
+                    sum += xor_lane<1>(sum);
+                    sum += xor_lane<2>(sum);
+                    sum += xor_lane<4>(sum);
+                    sum += xor_lane<8>(sum);
+                    const int rr = r + h2;
+                    if ((lane & 15) == 0 && rr < rows)
+                        a.xds[((grp + (rr >> 5)) * a.nxds + nu) * GRP_ROWS + (rr & 31)] = sum;
+                }
                 if (r + h2 < rows)
                 {
                     uint4 o;
@@ -407,7 +482,8 @@ __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16
                     o.y = (uint32_t)f2h(xv[2] * HAD) | ((uint32_t)f2h(xv[3] * HAD) << 16);
                     o.z = (uint32_t)f2h(xv[4] * HAD) | ((uint32_t)f2h(xv[5] * HAD) << 16);
                     o.w = (uint32_t)f2h(xv[6] * HAD) | ((uint32_t)f2h(xv[7] * HAD) << 16);
-                    *reinterpret_cast<uint4*>(a.xd + (size_t)(pos0 + r + h2) * a.I + od) = o;
+                    const int rr = r + h2;
+                    *reinterpret_cast<uint4*>(od + (grp + (rr >> 5)) * 32 * a.I + 8 * (rr & 31)) = o;
                 }
             }
         }
@@ -497,37 +573,17 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
     uint8_t* Bdec = smem + A_BYTES + T_BYTES;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // ---- tile. The grid is sized for the most tiles a call can have; the work = tiles x column blocks of this
-    // call is spread evenly over the 8 XCDs (workgroup b runs on XCD b % 8), and consecutive work items (the
-    // column blocks of one route block, then the next block of the same expert) stay on one XCD, so they share
-    // its L2 for the inputs and the trellis.
-    const int nact = min(a.nactive[0], a.max_active);
-    const int total = a.tile_off[nact];
-    const int work = total * a.nunits, per_xcd = (work + 7) >> 3;
-    const int L = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || L >= work) return;
-    const int mt = L / a.nunits, nu = L % a.nunits;
-    int lo = 0, hi = nact - 1;
-    while (lo < hi)
-    {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.tile_off[mid] <= mt) lo = mid; else hi = mid - 1;
-    }
-    const ExpertRec* rp = a.rec + lo;
-    // an expert's 256-route tiles come first; its 128-route tile (if any) follows them
-    const int row0 = BM == FT_BIG ? (mt - a.tile_off[lo]) * BM : (a.big_off[lo + 1] - a.big_off[lo]) * FT_BIG;
+    int mt, nu;
+    if (!fat_work(a, mt, nu)) return;
+    const FatTile* tp = a.tiles + mt;
+    const ExpertRec* rp = a.rec + tp->ai;
+    const int row0 = tp->row0;
     const int rows = __builtin_amdgcn_readfirstlane(min(BM, rp->cnt - row0));
     const int pos0 = __builtin_amdgcn_readfirstlane(rp->first + row0);
     const int e = __builtin_amdgcn_readfirstlane(rp->e);
+    const size_t grp = (size_t)__builtin_amdgcn_readfirstlane(tp->group);
     const int S = a.K / 32;
 
-    // ---- buffer descriptors (wave-uniform bases through readfirstlane, each half widened as uint32_t)
-    auto uniform_ptr = [](const void* p) {
-        const uint64_t v = (uint64_t)(uintptr_t)p;
-        const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-        const uint32_t h = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-        return reinterpret_cast<void*>((uintptr_t)((uint64_t)l | ((uint64_t)h << 32)));
-    };
     const bool tloader = wave < 4;
     // trellis loader (waves 0 .. 3): chunk q = wave of step s is tile row 2 s + (q >> 1) of matrix q & 1 (gate/up)
     // or of column block 2 nu + (q & 1) (down), 8 tiles = 768 bytes, 12 bytes per lane stored 16 bytes apart.
@@ -543,19 +599,17 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, Tring + (size_t)(s % FT_TS) * T_SLOT + (size_t)tq * 1024, 12,
                                                  tr * row_bytes + wcol + (uint32_t)lane * 12, 0, 0, 0);
     };
-    // inputs (every wave): LA loads of 1 KB = 1024 / SEG rows each (SEG / 16 lanes per row step); chunk q of row r
-    // goes to slot chunk_slot(q, r). Rows past the tile's routes and steps past the end read out of range (zero,
-    // no memory access).
-    const uint32_t a_row = (uint32_t)NA * a.K * 2;                       // bytes per route of the inputs
+    // inputs (every wave): LA loads of 1 KB each (half of one matrix's step of a row group). Row groups past the tile's
+    // routes and steps past the end read out of range (zero, no memory access).
+    const uint32_t gbytes = (uint32_t)NA * a.K * GRP_ROWS * 2;          // a row group
     const __amdgpu_buffer_rsrc_t ares = __builtin_amdgcn_make_buffer_rsrc(
-        uniform_ptr(a.xa + (size_t)pos0 * NA * a.K), (short)0, (int)((uint32_t)rows * a_row), 0x00020000);
+        uniform_ptr(a.xa + grp * (gbytes / 2)), (short)0, (int)((uint32_t)((rows + 31) / GRP_ROWS) * gbytes), 0x00020000);
     auto load_input = [&](int s, int u) {
         const int st = s % FT_PA;
-        const uint32_t ks = s < S ? (uint32_t)s * SEG : 0x40000000u; // the range is below 2^30
+        const uint32_t ks = s < S ? (uint32_t)s * (NA * 2048) : 0x40000000u; // the range is below 2^30
         const int li = wave * LA + u;                                  // 0 .. A_STAGE / 1024 - 1
-        const int r = li * (1024 / SEG) + lane / (SEG / 16), slot = lane % (SEG / 16);
-        const uint32_t voff = (uint32_t)r * a_row + (uint32_t)chunk_slot<NA>(slot, r) * 16 + ks;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, Aring + (size_t)st * A_STAGE + (size_t)li * 1024, 16, voff, 0, 0, 0);
+        const uint32_t voff = (uint32_t)(li / (2 * NA)) * gbytes + (uint32_t)(li % (2 * NA)) * 1024 + (uint32_t)lane * 16;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, Aring + (size_t)st * A_STAGE + (size_t)li * 1024, 16, voff + ks, 0, 0, 0);
     };
 
     // ---- decode: lane (col, g) decodes states i0 .. i0+3 of column col in a tile
@@ -581,7 +635,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
     for (int i = 0; i < MB; ++i)
     {
         const int r = 16 * (2 * i + wm) + col;
-        aoff[i] = r * SEG + chunk_slot<NA>((MODE == 0 ? (wn >> 1) : 0) * 4 + g, r) * 16;
+        aoff[i] = ((r >> 5) * NA + (MODE == 0 ? (wn >> 1) : 0)) * 2048 + (g * 32 + (r & 31)) * 16;
     }
     float4_t acc[MB][4];
 #pragma unroll
@@ -712,7 +766,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
             d[1] = (uint32_t)f2h(acc[i][j][2]) | ((uint32_t)f2h(acc[i][j][3]) << 16);
         }
     __syncthreads();
-    fat_tile_epilogue<MODE, CS, YH>(a, C, rows, pos0, e, nu, wave, lane);
+    fat_tile_epilogue<MODE, CS, YH>(a, C, rows, pos0, e, nu, grp, wave, lane);
 }
 
 // Sixteen-wave form of the tile (four waves per SIMD, 64 accumulators per lane): MBW = row blocks per wave, BM =
@@ -745,31 +799,17 @@ __global__ __launch_bounds__(FT16_THREADS, 1) void k_fat16(FatArgs a)
     uint8_t* Bdec = smem + A_BYTES + T_BYTES;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nact = min(a.nactive[0], a.max_active);
-    const int total = a.tile_off[nact];
-    const int work = total * a.nunits, per_xcd = (work + 7) >> 3;
-    const int L = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || L >= work) return;
-    const int mt = L / a.nunits, nu = L % a.nunits;
-    int lo = 0, hi = nact - 1;
-    while (lo < hi)
-    {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.tile_off[mid] <= mt) lo = mid; else hi = mid - 1;
-    }
-    const ExpertRec* rp = a.rec + lo;
-    const int row0 = BM == FT_BIG ? (mt - a.tile_off[lo]) * BM : (a.big_off[lo + 1] - a.big_off[lo]) * FT_BIG;
+    int mt, nu;
+    if (!fat_work(a, mt, nu)) return;
+    const FatTile* tp = a.tiles + mt;
+    const ExpertRec* rp = a.rec + tp->ai;
+    const int row0 = tp->row0;
     const int rows = __builtin_amdgcn_readfirstlane(min(BM, rp->cnt - row0));
     const int pos0 = __builtin_amdgcn_readfirstlane(rp->first + row0);
     const int e = __builtin_amdgcn_readfirstlane(rp->e);
+    const size_t grp = (size_t)__builtin_amdgcn_readfirstlane(tp->group);
     const int S = a.K / 32;
 
-    auto uniform_ptr = [](const void* p) {
-        const uint64_t v = (uint64_t)(uintptr_t)p;
-        const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-        const uint32_t h = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-        return reinterpret_cast<void*>((uintptr_t)((uint64_t)l | ((uint64_t)h << 32)));
-    };
     const bool tloader = wave < 4;
     const int tq = wave & 3;
     const uint32_t row_bytes = (uint32_t)(a.N / 16) * 96, wbytes = (uint32_t)(a.K / 16) * row_bytes;
@@ -782,18 +822,17 @@ __global__ __launch_bounds__(FT16_THREADS, 1) void k_fat16(FatArgs a)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, Tring + (size_t)(s % FT_TS) * T_SLOT + (size_t)tq * 1024, 12,
                                                  tr * row_bytes + wcol + (uint32_t)lane * 12, 0, 0, 0);
     };
-    const uint32_t a_row = (uint32_t)NA * a.K * 2;
+    const uint32_t gbytes = (uint32_t)NA * a.K * GRP_ROWS * 2;
     const __amdgpu_buffer_rsrc_t ares = __builtin_amdgcn_make_buffer_rsrc(
-        uniform_ptr(a.xa + (size_t)pos0 * NA * a.K), (short)0, (int)((uint32_t)rows * a_row), 0x00020000);
+        uniform_ptr(a.xa + grp * (gbytes / 2)), (short)0, (int)((uint32_t)((rows + 31) / GRP_ROWS) * gbytes), 0x00020000);
     // input load li = wave + 16 u of a step; this wave issues na of them (uniform)
     const int na = wave < NL ? (wave + NW < NL ? 2 : 1) : 0;
     auto load_input = [&](int s, int u) {
         const int st = s % FT_PA;
-        const uint32_t ks = s < S ? (uint32_t)s * SEG : 0x40000000u;
+        const uint32_t ks = s < S ? (uint32_t)s * (NA * 2048) : 0x40000000u;
         const int li = wave + NW * u;
-        const int r = li * (1024 / SEG) + lane / (SEG / 16), slot = lane % (SEG / 16);
-        const uint32_t voff = (uint32_t)r * a_row + (uint32_t)chunk_slot<NA>(slot, r) * 16 + ks;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, Aring + (size_t)st * A_STAGE + (size_t)li * 1024, 16, voff, 0, 0, 0);
+        const uint32_t voff = (uint32_t)(li / (2 * NA)) * gbytes + (uint32_t)(li % (2 * NA)) * 1024 + (uint32_t)lane * 16;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, Aring + (size_t)st * A_STAGE + (size_t)li * 1024, 16, voff + ks, 0, 0, 0);
     };
     auto load_inputs = [&](int s) {
         if (na > 0) load_input(s, 0);
@@ -816,7 +855,7 @@ __global__ __launch_bounds__(FT16_THREADS, 1) void k_fat16(FatArgs a)
     for (int i = 0; i < MBW; ++i)
     {
         const int r = 16 * (4 * i + wm) + col;
-        aoff[i] = r * SEG + chunk_slot<NA>((MODE == 0 ? (wn >> 1) : 0) * 4 + g, r) * 16;
+        aoff[i] = ((r >> 5) * NA + (MODE == 0 ? (wn >> 1) : 0)) * 2048 + (g * 32 + (r & 31)) * 16;
     }
     float4_t acc[MBW][4];
 #pragma unroll
@@ -923,7 +962,225 @@ __global__ __launch_bounds__(FT16_THREADS, 1) void k_fat16(FatArgs a)
             d[1] = (uint32_t)f2h(acc[i][j][2]) | ((uint32_t)f2h(acc[i][j][3]) << 16);
         }
     __syncthreads();
-    fat_tile_epilogue<MODE, CS, YH, NW>(a, C, rows, pos0, e, nu, wave, lane);
+    fat_tile_epilogue<MODE, CS, YH, NW>(a, C, rows, pos0, e, nu, grp, wave, lane);
+}
+
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+// k_mid's LDS: the four waves' rings (mid_depth steps of the trellis and the inputs), then, over them, the partial sums of
+// one row group, its C tile and the input sums (affine decode). One array: with a second one the compiler gives their accesses alias
+// scopes and then waits for every load to LDS (vmcnt 0) before each read.
+constexpr int mid_depth(int rb) { return rb == 3 ? 2 : 3; }
+constexpr int mid_slot(int rb) { return 2048 + rb * 2048; }
+constexpr int MID_C_AT = 2 * 32 * 128 * 4;
+constexpr int MID_XS_AT = MID_C_AT + FT_BN * (GRP_ROWS + 2) * 2;
+constexpr int MID_SMEM = std::max({ 4 * mid_depth(1) * mid_slot(1), 4 * mid_depth(2) * mid_slot(2),
+                                    4 * mid_depth(3) * mid_slot(3), MID_XS_AT + 2 * FT_MID * 4 });
+static_assert(2 * MID_SMEM <= 160 * 1024, "two workgroups (two waves per SIMD) share a CU's LDS");
+
+// Tiles of up to FT_MID = 96 routes x 256 output columns, for experts (and remainders of experts) with too few routes to
+// fill a 256-route tile. A workgroup is four waves: two column blocks of 128 (MODE 0: gate and up of one block, MODE
+// 1: two blocks) x two halves of K, and no barrier until the epilogue, which adds the halves. A wave streams its trellis rows (768 bytes) and
+// its inputs (a row group's step is one contiguous KB per operand) into a private LDS ring, and decodes each tile once,
+// in registers, for all its routes: v_mfma_f32_32x32x16_f16 over 32 routes x 32 columns, whose k-half h of operand mm
+// holds decode window 2 mm + h of both tile rows of the step, so the operand chunks are those of the row groups.
+template <int MODE, int RB, bool EXACT, bool YH>
+__device__ __forceinline__ void mid_tile(const FatArgs& a, uint8_t* smem, int rows, int pos0, int e, size_t grp, int nu,
+                                         const ExpertRec* rp)
+{
+    constexpr int BM = RB * GRP_ROWS;
+    constexpr int NA = MODE == 0 ? 2 : 1;
+    constexpr int DEPTH = mid_depth(RB);
+    constexpr int T_SLOT = 2048, SLOT = mid_slot(RB);
+    constexpr int NL = 2 + 2 * RB;                                // loads of a step
+    constexpr int CS = GRP_ROWS + 2;                              // C tile of one row group (fat_tile_epilogue)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = wave & 1, kh = wave >> 1;
+    const int S = a.K / 64, step0 = kh * S;                       // steps of this wave's half of K (a.K / 32 is even)
+
+    const uint32_t row_bytes = (uint32_t)(a.N / 16) * 96, wbytes = (uint32_t)(a.K / 16) * row_bytes;
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+        uniform_ptr((const void*)(uintptr_t)rp->w[MODE == 0 ? sub : 2]), (short)0, (int)wbytes, 0x00020000);
+    const uint32_t wcol = MODE == 0 ? (uint32_t)nu * 768 : (uint32_t)(2 * nu + sub) * 768;
+    const uint32_t gbytes = (uint32_t)NA * a.K * GRP_ROWS * 2;
+    const __amdgpu_buffer_rsrc_t ares = __builtin_amdgcn_make_buffer_rsrc(
+        uniform_ptr(a.xa + grp * (gbytes / 2)), (short)0, (int)((uint32_t)((rows + 31) / GRP_ROWS) * gbytes), 0x00020000);
+    uint8_t* ring = smem + wave * (DEPTH * SLOT);
+    // step s into a slot (past the end: the last step again, into a free slot): both trellis rows, 12 bytes per lane 16
+    // apart, then the operands mm of each row group (one past the tile's routes reads zeros)
+    auto load_step = [&](int s, int slot) {
+        uint8_t* d = ring + slot * SLOT;
+        s = step0 + min(s, S - 1);
+        const uint32_t o = (uint32_t)(2 * s) * row_bytes + wcol;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, d, 12, (uint32_t)lane * 12, o, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, d + 1024, 12, (uint32_t)lane * 12, o + row_bytes, 0, 0);
+        const uint32_t ao = (uint32_t)s * (NA * 2048) + (MODE == 0 ? (uint32_t)sub * 2048 : 0);
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+        {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, d + T_SLOT + r * 2048, 16, (uint32_t)lane * 16, ao + r * gbytes, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, d + T_SLOT + r * 2048 + 1024, 16, (uint32_t)lane * 16 + 1024,
+                                                     ao + r * gbytes, 0, 0);
+        }
+    };
+
+    // decode: lane (n = lane & 15, ct = (lane >> 4) & 1, h = lane >> 5) decodes window 2 mm + h of column n of tile
+    // 2 cp + ct
+    const int n = lane & 15, h = lane >> 5;
+    int llo[2], lhi[2];
+    uint32_t sh[2];
+#pragma unroll
+    for (int mm = 0; mm < 2; ++mm)
+    {
+        const int i0 = 32 * (n & 7) + 8 * (2 * mm + h) + 4 * (n >> 3), eb = 3 * i0 + 11;
+        const int blo = eb >> 5, bhi = (blo + 23) % 24;
+        llo[mm] = 4 * (4 * (blo / 3) + blo % 3) + 128 * ((lane >> 4) & 1);
+        lhi[mm] = 4 * (4 * (bhi / 3) + bhi % 3) + 128 * ((lane >> 4) & 1);
+        sh[mm] = 31u - (uint32_t)(eb & 31);
+    }
+
+    float16_t acc[RB][4];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[r][c][v] = 0.0f;
+    // trellis words and operands of half mm of the step in a slot
+    uint32_t W[2][4][2][2];
+    half8_t A[2][RB];
+    auto read_half = [&](int slot, auto mm_tag) {
+        constexpr int mm = decltype(mm_tag)::value;
+        const uint8_t* t0 = ring + slot * SLOT;
+#pragma unroll
+        for (int cp = 0; cp < 4; ++cp)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+            {
+                W[mm][cp][t][0] = *reinterpret_cast<const uint32_t*>(t0 + lhi[mm] + cp * 256 + t * 1024);
+                W[mm][cp][t][1] = *reinterpret_cast<const uint32_t*>(t0 + llo[mm] + cp * 256 + t * 1024);
+            }
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+            A[mm][r] = *reinterpret_cast<const half8_t*>(t0 + T_SLOT + r * 2048 + mm * 1024 + lane * 16);
+    };
+    auto compute_half = [&](auto mm_tag) {
+        constexpr int mm = decltype(mm_tag)::value;
+#pragma unroll
+        for (int cp = 0; cp < 4; ++cp)
+        {
+            const half4_t b0 = decode4<EXACT>(W[mm][cp][0][0], W[mm][cp][0][1], sh[mm]);
+            const half4_t b1 = decode4<EXACT>(W[mm][cp][1][0], W[mm][cp][1][1], sh[mm]);
+            const half8_t B = { b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3] };
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+                acc[r][cp] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[mm][r], B, acc[r][cp], 0, 0, 0);
+        }
+    };
+    const std::integral_constant<int, 0> h0;
+    const std::integral_constant<int, 1> h1;
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) load_step(j, j);
+    wait_vmcnt<(DEPTH - 1) * NL>();
+    constexpr bool PIPE = RB < 3;
+    if constexpr (PIPE) read_half(0, h0);
+    int slot = 0;
+    for (int s = 0; s < S; ++s)
+    {
+        // the second half's reads run during the first half's decode, the next step's first reads during the second's
+        if constexpr (PIPE) read_half(slot, h1);
+        else read_half(slot, h0);
+        compute_half(h0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!PIPE) read_half(slot, h1);
+        // step s + 1 is complete once at most the loads of the steps after it are outstanding; this step's reads are
+        // complete before its slot is filled again
+        wait_vmcnt<(DEPTH - 2) * NL>();
+        wait_lgkm0();
+        load_step(s + DEPTH, slot);
+        slot = slot + 1 == DEPTH ? 0 : slot + 1;
+        if constexpr (PIPE) read_half(slot, h0);
+        compute_half(h1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    wait_vmcnt<0>();
+    __syncthreads();
+    float4_t* red = reinterpret_cast<float4_t*>(smem) + sub * 1024 + lane;
+    uint16_t* C = reinterpret_cast<uint16_t*>(smem + MID_C_AT);
+    float* xs_row = reinterpret_cast<float*>(smem + MID_XS_AT) + sub * BM;
+    if (!EXACT && kh == 0)
+        for (int r = lane; r < BM; r += 64)
+        {
+            float v = 0.0f;
+            if (r < rows)
+                for (int b = 0; b < a.nxs; ++b)
+                    v += a.xs[(((grp + (r >> 5)) * a.nxs + b) * NA + (MODE == 0 ? sub : 0)) * GRP_ROWS + (r & 31)];
+            xs_row[r] = v * kbias_f();
+        }
+    // one row group at a time: the second half's sums through LDS, then the C tile (lane (column lane & 31, h) of a 32 x
+    // 32 block holds rows 8 (v >> 2) + 4 h + (v & 3); the affine decode's sums become KINV S + KBIAS (sum of the row's
+    // inputs)), then the epilogue, 8 rows per wave
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+    {
+        if (r * GRP_ROWS >= rows) break;
+        if (kh == 1)
+#pragma unroll
+            for (int cp = 0; cp < 4; ++cp)
+#pragma unroll
+                for (int v = 0; v < 16; v += 4)
+                    red[(cp * 4 + v / 4) * 64] = float4_t{ acc[r][cp][v], acc[r][cp][v + 1], acc[r][cp][v + 2], acc[r][cp][v + 3] };
+        __syncthreads();
+        if (kh == 0)
+#pragma unroll
+            for (int v = 0; v < 16; v += 4)
+            {
+                const int rr = 2 * v + 4 * h;
+                float4_t xs = { 0.f, 0.f, 0.f, 0.f };
+                if constexpr (!EXACT) xs = *reinterpret_cast<const float4_t*>(&xs_row[r * GRP_ROWS + rr]);
+#pragma unroll
+                for (int cp = 0; cp < 4; ++cp)
+                {
+                    const float4_t o = red[(cp * 4 + v / 4) * 64];
+                    uint32_t* d = reinterpret_cast<uint32_t*>(C + (size_t)(sub * 128 + cp * 32 + (lane & 31)) * CS + rr);
+                    float y[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        const float sum = acc[r][cp][v + i] + o[i];
+                        y[i] = EXACT ? sum : fmaf(kinv_f(), sum, xs[i]);
+                    }
+                    d[0] = (uint32_t)f2h(y[0]) | ((uint32_t)f2h(y[1]) << 16);
+                    d[1] = (uint32_t)f2h(y[2]) | ((uint32_t)f2h(y[3]) << 16);
+                }
+            }
+        __syncthreads();
+        fat_tile_epilogue<MODE, CS, YH, 4, !EXACT>(a, C, min(rows - r * GRP_ROWS, GRP_ROWS), pos0 + r * GRP_ROWS, e, nu,
+                                                   grp + r, wave, lane);
+    }
+}
+
+template <int MODE, bool EXACT, bool YH = false>
+__global__ __launch_bounds__(256, 2) void k_mid(FatArgs a)
+{
+    __shared__ __align__(16) uint8_t smem[MID_SMEM];
+    // workgroup b runs on XCD b % 8: tile t's column units go to XCD t % 8 one after another (they share the inputs), so the
+    // XCDs get the same mix of long and short tiles
+    const int b = blockIdx.x >> 3, mt = b / a.nunits * 8 + (int)(blockIdx.x & 7), nu = b % a.nunits;
+    if (mt >= a.ntiles[0]) return;
+    const FatTile* tp = a.tiles + mt;
+    const ExpertRec* rp = a.rec + tp->ai;
+    const int row0 = tp->row0;
+    const int rows = __builtin_amdgcn_readfirstlane(min(FT_MID, rp->cnt - row0));
+    const int pos0 = __builtin_amdgcn_readfirstlane(rp->first + row0);
+    const int e = __builtin_amdgcn_readfirstlane(rp->e);
+    const size_t grp = (size_t)__builtin_amdgcn_readfirstlane(tp->group);
+    if (rows > 2 * GRP_ROWS)
+        mid_tile<MODE, 3, EXACT, YH>(a, smem, rows, pos0, e, grp, nu, rp);
+    else if (rows > GRP_ROWS)
+        mid_tile<MODE, 2, EXACT, YH>(a, smem, rows, pos0, e, grp, nu, rp);
+    else
+        mid_tile<MODE, 1, EXACT, YH>(a, smem, rows, pos0, e, grp, nu, rp);
 }
 
 // Weighted combine of the fat routes: out[t] = (accumulate ? out[t] : 0) + sum_j w_j y_j over the routes j of
@@ -1115,12 +1372,17 @@ struct FatWs
     void* pws;            // permutation workspace
     size_t pws_bytes;
     ExpertRec* rec;       // [min(n, E)]
-    int32_t* off_big;     // [min(n, E) + 1]
-    int32_t* off_small;   // [min(n, E) + 1]
-    uint16_t* xa;         // [n][2][H]
-    uint16_t* xd;         // [n][I]
+    FatTile* big;         // 256-route tiles
+    FatTile* mid;         // FT_MID-route tiles
+    int2* groups;         // row groups: record, first row
+    int32_t* totals;      // [3] entries of the three lists
+    int max_big, max_mid, max_groups;
+    uint16_t* xa;         // [max_groups][H / 32][2][GRP_HALVES]
+    uint16_t* xd;         // [max_groups][I / 32][GRP_HALVES]
+    float* xs;            // [max_groups][prep slices][2][GRP_ROWS] input sums
+    float* xds;           // [max_groups][I / 128][GRP_ROWS] down-input sums
+    int nxs;
     float* Y;             // [n][H]
-    int32_t* e_sorted;    // [n] expert bin of each sorted position
     size_t bytes;
 };
 
@@ -1129,11 +1391,20 @@ static FatWs fat_carve(void* base, int n, int E, int H, int I)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t na = (size_t)(n < E ? n : E);
     const size_t pwsb = mm_permute_workspace(n, E);
-    constexpr int NS = 13;
+    // an expert of c routes has at most c / FT_BIG_MIN 256-route tiles, c / FT_MID + 1 others and c / GRP_ROWS + 1 row
+    // groups
+    FatWs w;
+    w.max_big = n / FT_BIG_MIN;
+    w.max_mid = n / FT_MID + (int)na;
+    w.max_groups = n / GRP_ROWS + (int)na;
+    const size_t ng = (size_t)w.max_groups;
+    w.nxs = (H / 128 + PREP_BLOCKS - 1) / PREP_BLOCKS;
+    constexpr int NS = 16;
     const size_t sizes[NS] = { al((size_t)(E + 1) * 4), al((size_t)(E + 2) * 4), al((size_t)n * 4), al((size_t)E * 4),
-                               al(4), al(pwsb), al(na * sizeof(ExpertRec)), al((na + 1) * 4), al((na + 1) * 4),
-                               al((size_t)n * 2 * H * 2), al((size_t)n * I * 2), al((size_t)n * H * 4),
-                               al((size_t)n * 4) };
+                               al(4), al(pwsb), al(na * sizeof(ExpertRec)), al(w.max_big * sizeof(FatTile)),
+                               al(w.max_mid * sizeof(FatTile)), al(ng * sizeof(int2)), al(12),
+                               al(ng * GRP_ROWS * 2 * H * 2), al(ng * GRP_ROWS * I * 2), al((size_t)n * H * 4),
+                               al(ng * w.nxs * 2 * GRP_ROWS * 4), al(ng * (I / 128) * GRP_ROWS * 4) };
     char* p = static_cast<char*>(base);
     char* at[NS];
     size_t off = 0;
@@ -1142,11 +1413,11 @@ static FatWs fat_carve(void* base, int n, int E, int H, int I)
         at[i] = p ? p + off : nullptr;
         off += sizes[i];
     }
-    FatWs w;
     w.counts = (int32_t*)at[0]; w.offsets = (int32_t*)at[1]; w.order = (int32_t*)at[2]; w.active = (int32_t*)at[3];
     w.nactive = (int32_t*)at[4]; w.pws = at[5]; w.pws_bytes = pwsb; w.rec = (ExpertRec*)at[6];
-    w.off_big = (int32_t*)at[7]; w.off_small = (int32_t*)at[8]; w.xa = (uint16_t*)at[9]; w.xd = (uint16_t*)at[10];
-    w.Y = (float*)at[11]; w.e_sorted = (int32_t*)at[12];
+    w.big = (FatTile*)at[7]; w.mid = (FatTile*)at[8]; w.groups = (int2*)at[9]; w.totals = (int32_t*)at[10];
+    w.xa = (uint16_t*)at[11]; w.xd = (uint16_t*)at[12]; w.Y = (float*)at[13];
+    w.xs = (float*)at[14]; w.xds = (float*)at[15];
     w.bytes = off;
     return w;
 }
@@ -1170,55 +1441,77 @@ static int fat_check(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     return MM_OK;
 }
 
-// Plan and both GEMMs over the sorted positions in ws (counts, offsets, order, active, nactive filled): Y rows of
-// every position of an active expert with more than cap routes.
-static int fat_gemms(const mm_layer_t* L, int n, int cap, const FatWs& ws, hipStream_t s, bool yh)
+// Plan, input transform and both GEMMs over the sorted positions in ws (counts, offsets, order, active, nactive filled):
+// Y rows of every position of an active expert with more than cap routes. token_sorted: the positions' tokens, or null
+// (order[pos] / topk).
+static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* token_sorted, int n,
+                     int cap, const FatWs& ws, hipStream_t s, bool yh, bool fused)
 {
+    // the fused call takes the layer's codebook evaluation; the others round the weights to fp16
+    const bool exact = !fused || (L->flags & MM_LAYER_EXACT) != 0;
+    const BigRule rule = fused ? BigRule{ (FT_BIG_WORK + L->I / 128 - 1) / (L->I / 128), 0 } : BigRule{ 0, FT_BIG_ROWS };
     const int E = L->E, na = n < E ? n : E;
     hipLaunchKernelGGL(k_fat_plan, dim3(1), dim3(FT_PLAN_MAX), 0, s, ws.counts, ws.offsets, ws.active, ws.nactive,
-                       L->gate_ptr, L->up_ptr, L->down_ptr, ws.rec, ws.off_big, ws.off_small, na, cap);
-    // a 256-route tile holds more than 128 routes: at most n / 129 of them; one 128-route tile per active expert
-    const int max_big = n / (FT_SMALL + 1), max_small = na;
+                       L->gate_ptr, L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.mid, ws.groups, ws.totals, na, cap, rule);
+    hipLaunchKernelGGL(k_fat_prep, dim3((unsigned)ws.max_groups, (unsigned)ws.nxs),
+                       dim3(512), 0, s, x, x_dtype, ws.order, token_sorted, ws.rec, ws.groups, ws.totals + 2, L->suh13,
+                       ws.xa, ws.xs, topk, T, L->H);
     auto grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles * units + 7) & ~(size_t)7)); };    // >= 8 per_xcd
-    FatArgs g{ ws.rec, ws.nactive, ws.off_big, ws.off_big, ws.xa, L->svh13, L->suh2, L->svh2, ws.order, ws.xd, ws.Y,
-               L->H, L->I, L->H, L->I, L->I / 128, na, L->limit };
-    FatArgs gs = g;
-    gs.tile_off = ws.off_small;
+    auto mid_grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles + 7) / 8 * 8 * units)); };
+    FatArgs g{ ws.rec, ws.big, ws.totals, ws.xa, L->svh13, L->suh2, L->svh2, ws.order, ws.xd, ws.Y,
+               ws.xs, ws.xds, L->H, L->I, L->H, L->I, L->I / 128, ws.nxs, L->I / 128, L->limit };
+    FatArgs gm = g;
+    gm.tiles = ws.mid;
+    gm.ntiles = ws.totals + 1;
     FatArgs d = g;
     d.xa = ws.xd; d.K = L->I; d.N = L->H; d.nunits = L->H / 256;
-    FatArgs ds = d;
-    ds.tile_off = ws.off_small;
-    // gate/up: 256-route tiles on the 8-wave kernel, 128-route tiles and the down GEMM on the 16-wave kernel (same
-    // bits; measured on the 16k layer: gate/up 256-route tiles equal, 128-route tiles 97 against 111 us, down
-    // 2.76-2.85 against 2.92-2.94 ms)
-    if (max_big > 0) hipLaunchKernelGGL((k_fat<0, FT_BIG / 32>), grid(max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
-    hipLaunchKernelGGL((k_fat16<0, FT_SMALL / 64>), grid(max_small, g.nunits), dim3(FT16_THREADS), 0, s, gs);
+    d.xs = ws.xds; d.nxs = g.nxds;
+    FatArgs dm = d;
+    dm.tiles = ws.mid;
+    dm.ntiles = ws.totals + 1;
+    // gate/up: 256-route tiles on the 8-wave kernel, down on the 16-wave kernel (same bits; measured on the 16k layer:
+    // gate/up equal, down 2.76-2.85 against 2.92-2.94 ms)
+    if (ws.max_big > 0) hipLaunchKernelGGL((k_fat<0, FT_BIG / 32>), grid(ws.max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
+    if (exact) hipLaunchKernelGGL((k_mid<0, true>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
+    else hipLaunchKernelGGL((k_mid<0, false>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
     if (yh)
     {
-        if (max_big > 0)
-            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64, true>), grid(max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
-        hipLaunchKernelGGL((k_fat16<1, FT_SMALL / 64, true>), grid(max_small, d.nunits), dim3(FT16_THREADS), 0, s, ds);
+        if (ws.max_big > 0)
+            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64, true>), grid(ws.max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
+        if (exact) hipLaunchKernelGGL((k_mid<1, true, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
+        else hipLaunchKernelGGL((k_mid<1, false, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
     }
     else
     {
-        if (max_big > 0)
-            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64>), grid(max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
-        hipLaunchKernelGGL((k_fat16<1, FT_SMALL / 64>), grid(max_small, d.nunits), dim3(FT16_THREADS), 0, s, ds);
+        if (ws.max_big > 0)
+            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64>), grid(ws.max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
+        if (exact) hipLaunchKernelGGL((k_mid<1, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
+        else hipLaunchKernelGGL((k_mid<1, false>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
     }
     return check_launch("fat path");
 }
 
-// Permutation, input prep, plan and both GEMMs: Y rows of every route whose expert has more than cap routes.
+// Permutation, input transform, plan and both GEMMs: Y rows of every route whose expert has more than cap routes.
 static int fat_run(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, int cap,
-                   const FatWs& ws, hipStream_t s, bool yh)
+                   const FatWs& ws, hipStream_t s, bool yh, bool fused)
 {
     const int n = T * topk, E = L->E;
     int rc = permute_launch(ids, nullptr, n, topk, E, ws.counts, ws.offsets, ws.order, nullptr, nullptr, nullptr,
-                            ws.active, ws.nactive, ws.e_sorted, ws.pws, ws.pws_bytes, s);
+                            ws.active, ws.nactive, nullptr, ws.pws, ws.pws_bytes, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_fat_prep, dim3(n), dim3(256), 0, s, x, x_dtype, ws.e_sorted, ws.counts, ws.offsets, ws.order,
-                       L->suh13, ws.xa, topk, E, L->H, cap);
-    return fat_gemms(L, n, cap, ws, s, yh);
+    return fat_gemms(L, x, x_dtype, T, topk, nullptr, n, cap, ws, s, yh, fused);
+}
+
+// fat_run and the weighted combine of its rows.
+static int fat_layer(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
+                     int cap, int accumulate, float* out, const FatWs& ws, hipStream_t s, bool fused)
+{
+    const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true, fused);
+    if (r) return r;
+    const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
+    hipLaunchKernelGGL(k_fat_combine, grid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.Y), ids, w,
+                       ws.counts, T, topk, L->H, L->E, cap, accumulate);
+    return check_launch("fat layer");
 }
 
 // Workspace of the sorted-route form: the fat sections for n positions, then the token lists.
@@ -1247,6 +1540,12 @@ static FatbWs fatb_carve(void* base, int n, int T, int E, int H, int I)
 
 // ------------------------------------------------------------------------------------ the fused-MoE call
 
+// Calls of more routes than the decode path routes in-kernel run every expert on the grouped GEMM: k_mid decodes a tile as
+// fast for one route as for 32, so an expert with few routes costs it what the decode path pays per 16 (34 against 33 ns per
+// 16 x 16 tile and SIMD), and the decode path's launches over all tokens, for the few routes it is left with, go (at 4,096
+// tokens its combine alone took 0.64 ms, at 16,384 tokens 2.0 ms).
+constexpr int FUSED_SPLIT_MAX = 1024;
+
 // ids_small[s] = ids[s] when its expert has at most cap routes in the call (counts from the fat pass's
 // permutation), else -1: the routes the decode path takes.
 __global__ __launch_bounds__(256) void k_small_ids(const int64_t* __restrict__ ids, const int32_t* __restrict__ counts,
@@ -1259,48 +1558,34 @@ __global__ __launch_bounds__(256) void k_small_ids(const int64_t* __restrict__ i
     }
 }
 
-// Workspace of mm_fused_moe: the fat pass over all n routes, the decode path's ids and permutation, then the
-// decode workspace with positions bounded by npos.
+// Workspace of mm_fused_moe: the fat pass over all n routes, then (calls of at most FUSED_SPLIT_MAX routes) the decode
+// path's ids and workspace.
 struct FusedWs
 {
     FatWs fat;
     int64_t* ids_small;   // [n]
-    int32_t* counts;      // [E + 1]  permutation of ids_small
-    int32_t* offsets;     // [E + 2]
-    int32_t* order;       // [n]
-    int32_t* active;      // [E]
-    int32_t* nactive;     // [1]
-    void* pws;
-    size_t pws_bytes;
     void* dws;            // decode workspace
-    int npos;
-    bool in_kernel;       // decode routing found in-kernel (n <= 1024, topk <= 16)
-    size_t bytes;
+    size_t dws_bytes, bytes;
 };
 
-static FusedWs fused_carve(void* base, int T, int topk, int E, int H, int I, int cap)
+static FusedWs fused_carve(void* base, int T, int topk, int E, int H, int I)
 {
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const int n = T * topk;
     FusedWs w;
     w.fat = fat_carve(base, n, E, H, I);
-    w.in_kernel = n <= 1024 && topk <= 16;
-    // every decode-path expert has at most cap routes, so their positions lie below E x cap
-    w.npos = w.in_kernel ? n : (int)std::min<int64_t>(n, (int64_t)E * std::max(cap, 1));
-    w.pws_bytes = mm_permute_workspace(n, E);
-    const size_t sizes[8] = { al((size_t)n * 8), al((size_t)(E + 1) * 4), al((size_t)(E + 2) * 4), al((size_t)n * 4),
-                              al((size_t)E * 4), al(4), al(w.pws_bytes), decode_ws_bytes(n, w.npos, E, H, I) };
-    char* p = base ? static_cast<char*>(base) + w.fat.bytes : nullptr;
-    char* at[8];
-    size_t off = 0;
-    for (int i = 0; i < 8; ++i)
+    w.ids_small = nullptr;
+    w.dws = nullptr;
+    w.dws_bytes = 0;
+    w.bytes = w.fat.bytes;
+    if (n > FUSED_SPLIT_MAX) return w;
+    const size_t ids = ((size_t)n * 8 + 255) & ~(size_t)255;
+    w.dws_bytes = mm_gemv_workspace(n, E, H, I);
+    if (base)
     {
-        at[i] = p ? p + off : nullptr;
-        off += sizes[i];
+        w.ids_small = reinterpret_cast<int64_t*>(static_cast<char*>(base) + w.bytes);
+        w.dws = static_cast<char*>(base) + w.bytes + ids;
     }
-    w.ids_small = (int64_t*)at[0]; w.counts = (int32_t*)at[1]; w.offsets = (int32_t*)at[2]; w.order = (int32_t*)at[3];
-    w.active = (int32_t*)at[4]; w.nactive = (int32_t*)at[5]; w.pws = at[6]; w.dws = at[7];
-    w.bytes = w.fat.bytes + off;
+    w.bytes += ids + w.dws_bytes;
     return w;
 }
 
@@ -1313,7 +1598,7 @@ extern "C" {
 size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap)
 {
     if (T <= 0 || topk <= 0 || E <= 0 || H <= 0 || I <= 0 || cap < 0) return 0;
-    return fused_carve(nullptr, T, topk, E, H, I, cap).bytes;
+    return fused_carve(nullptr, T, topk, E, H, I).bytes;
 }
 
 int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1324,30 +1609,23 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
     MM_CHECK_ARG(w && out && cap >= 1, "mm_fused_moe: null pointer or cap < 1");
     MM_CHECK_ARG(topk <= 16, "mm_fused_moe: topk must be at most 16");
     const int n = T * topk, E = L->E;
-    const FusedWs ws = fused_carve(workspace, T, topk, E, L->H, L->I, cap);
-    // the decode path's per-position inputs are addressed with 32-bit buffer offsets
-    MM_CHECK_ARG((size_t)ws.npos * 2 * std::max(L->H, L->I) * 2 < ((size_t)1 << 31),
-                 "mm_fused_moe: too many decode-path positions (%d)", ws.npos);
+    const FusedWs ws = fused_carve(workspace, T, topk, E, L->H, L->I);
+    // a limit of the interface: n, or E x cap for larger n, transformed inputs within 32-bit byte offsets
+    const size_t npos = n <= FUSED_SPLIT_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
+    MM_CHECK_ARG(npos * 2 * std::max(L->H, L->I) * 2 < ((size_t)1 << 31),
+                 "mm_fused_moe: too many decode-path positions (%zu)", npos);
     MM_CHECK_ARG(workspace && workspace_bytes >= ws.bytes, "mm_fused_moe: workspace too small (%zu < %zu)",
                  workspace_bytes, ws.bytes);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (n > FUSED_SPLIT_MAX) return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, ws.fat, s, true);
     // 1. experts above cap on the grouped GEMM: out = their weighted sum (every token written)
-    int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws.fat, s, true);
+    int r = fat_layer(L, x, x_dtype, T, topk, ids, w, cap, 0, out, ws.fat, s, true);
     if (r) return r;
-    const dim3 cgrid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
-    hipLaunchKernelGGL(k_fat_combine, cgrid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.fat.Y), ids, w,
-                       ws.fat.counts, T, topk, L->H, E, cap, 0);
     // 2. the others on the decode path, added per token in ascending route order
     hipLaunchKernelGGL(k_small_ids, dim3((unsigned)std::min((n + 255) / 256, 1024)), dim3(256), 0, s, ids,
                        ws.fat.counts, n, E, cap, ws.ids_small);
-    if (ws.in_kernel)
-        return moe_decode_launch(L, x, x_dtype, 0, T, topk, ws.ids_small, w, cap, out, ws.dws,
-                                 decode_ws_bytes(n, n, E, L->H, L->I), stream, "mm_fused_moe", 1);
-    r = permute_launch(ws.ids_small, nullptr, n, topk, E, ws.counts, ws.offsets, ws.order, nullptr, nullptr, nullptr,
-                       ws.active, ws.nactive, nullptr, ws.pws, ws.pws_bytes, s);
-    if (r) return r;
-    return decode_perm_launch(L, x, x_dtype, T, topk, ws.ids_small, w, ws.offsets, ws.order, ws.active, ws.nactive,
-                              ws.npos, cap, out, 1, ws.dws, s);
+    return moe_decode_launch(L, x, x_dtype, 0, T, topk, ws.ids_small, w, cap, out, ws.dws, ws.dws_bytes, stream,
+                             "mm_fused_moe", 1);
 }
 
 size_t mm_prefill_workspace(int n, int E, int H, int I)
@@ -1365,7 +1643,7 @@ int mm_grouped_gemm(const mm_layer_t* L, const void* x, int x_dtype, int T, int 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     FatWs ws = fat_carve(workspace, T * topk, L->E, L->H, L->I);
     ws.Y = Y;
-    return fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, false);
+    return fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, false, false);
 }
 
 int mm_moe_prefill(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1374,15 +1652,8 @@ int mm_moe_prefill(const mm_layer_t* L, const void* x, int x_dtype, int T, int t
     const int rc = fat_check(L, x, x_dtype, T, topk, ids, workspace, workspace_bytes, "mm_moe_prefill");
     if (rc) return rc;
     MM_CHECK_ARG(w && out && cap >= 0, "mm_moe_prefill: null pointer or negative cap");
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const FatWs ws = fat_carve(workspace, T * topk, L->E, L->H, L->I);
-    const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true);
-    if (r) return r;
-    const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
-    hipLaunchKernelGGL(k_fat_combine, grid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.Y), ids, w,
-                       ws.counts, T, topk, L->H, L->E, cap,
-                       accumulate);
-    return check_launch("mm_moe_prefill");
+    return fat_layer(L, x, x_dtype, T, topk, ids, w, cap, accumulate, out, fat_carve(workspace, T * topk, L->E, L->H, L->I),
+                     reinterpret_cast<hipStream_t>(stream), false);
 }
 
 size_t mm_fat_batched_workspace(int n, int T, int E, int H, int I)
@@ -1420,9 +1691,7 @@ int mm_fat_batched(const mm_layer_t* L, const void* x, int x_dtype, int T, int n
     hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)std::min((T + 255) / 256, 1024)), dim3(256), 0, s, ws.tcount, T, 0);
     hipLaunchKernelGGL(k_fatb_tokens<1>, dim3(pg), dim3(256), 0, s, token_sorted, ws.f.counts, ws.f.offsets, ws.f.order,
                        ws.tcount, ws.toff, ws.tpos, T, E, n);
-    hipLaunchKernelGGL(k_fatb_prep, dim3(n), dim3(256), 0, s, x, x_dtype, token_sorted, ws.f.counts, ws.f.offsets,
-                       L->suh13, ws.f.xa, T, E, L->H);
-    int r = fat_gemms(L, n, cap, ws.f, s, true);
+    int r = fat_gemms(L, x, x_dtype, T, 1, token_sorted, n, cap, ws.f, s, true, false);
     if (r) return r;
     const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
     hipLaunchKernelGGL(k_fatb_combine, grid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.f.Y),

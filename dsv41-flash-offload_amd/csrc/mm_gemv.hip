@@ -889,18 +889,11 @@ static int check_common(const mm_layer_t* L, const void* x, int x_dtype, int T, 
     return MM_OK;
 }
 
-__global__ __launch_bounds__(256) void k_fill_pos(int32_t* p, int n)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = -1;
-}
-
 static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_dtype, int rescale, int n, int npos,
                         int topk, const int64_t* ids, const int32_t* offsets, const int32_t* order,
                         const int32_t* active, const int32_t* nactive, int cap, hipStream_t s)
 {
     const int nb = prep_blocks(L->H);
-    // positions past npos are not visited: their routes' pos_of must read "no position"
-    if (npos < n) hipLaunchKernelGGL(k_fill_pos, dim3((unsigned)min((n + 255) / 256, 1024)), dim3(256), 0, s, w.pos_of, n);
     PrepArgs p{ x, ids, offsets, order, active, nactive, L->gate_ptr, L->up_ptr, L->down_ptr, L->suh13,
                 w.rec, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, w.xa, w.xsum, n, topk, L->E, L->H, nb,
                 x_dtype, rescale, cap, npos };
@@ -955,27 +948,6 @@ int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int resca
     hipLaunchKernelGGL(k_down_combine, dim3(T * (L->H / GV_COLS)), dim3(threads), 0, s,
                        down_args(L, ws, n, topk, ids, w, nullptr, out, accumulate));
     return check_launch(who);
-}
-
-size_t decode_ws_bytes(int n, int npos, int E, int H, int I) { return carve(nullptr, n, npos, E, H, I).bytes; }
-
-// The decode path of a call on a permutation whose valid positions lie below npos (every expert <= cap routes
-// there), summed per token into out (out += with accumulate). Arguments are checked by the caller.
-int decode_perm_launch(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids,
-                       const float* w, const int32_t* offsets, const int32_t* order, const int32_t* active,
-                       const int32_t* nactive, int npos, int cap, float* out, int accumulate, void* workspace,
-                       hipStream_t s)
-{
-    const int n = T * topk;
-    const Ws ws = carve(workspace, n, npos, L->E, L->H, L->I);
-    launch_prep(L, ws, x, x_dtype, 0, n, npos, topk, ids, offsets, order, active, nactive, cap, s);
-    launch_partial<0>(L, ws, npos, s);
-    launch_gu_epilogue(L, ws, npos, s);
-    launch_partial<1>(L, ws, npos, s);
-    const int threads = 64 * (topk < 2 ? 2 : topk);
-    hipLaunchKernelGGL(k_down_combine, dim3(T * (L->H / GV_COLS)), dim3(threads), 0, s,
-                       down_args(L, ws, npos, topk, ids, w, nullptr, out, accumulate));
-    return check_launch("decode path");
 }
 
 }  // namespace mm

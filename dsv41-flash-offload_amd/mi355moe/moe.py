@@ -134,7 +134,8 @@ def moe_forward(store, x, ids, w, shared_expert=None, fat_threshold=FAT_THRESHOL
 
 def fused_moe(store, x, ids, w, cap, stream=None):
     """mm_fused_moe: out fp32 [T, H] over ids [T, k] / w [T, k], experts with more than `cap` routes on the
-    grouped GEMM and the others on the decode path, split on the device."""
+    grouped GEMM and the others on the decode path, split on the device (calls of more than 1,024 routes run every
+    expert on the grouped GEMM)."""
     T, k = ids.shape
     x = x.contiguous()
     ids = ids.contiguous().long()

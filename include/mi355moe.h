@@ -187,7 +187,7 @@ size_t mm_prefill_workspace(int n, int E, int H, int I);
  * patches/vllm-exl3-host-dma.patch:182-201, and runtime/dma_gemm.py:5-26 run_batch, which feeds it): for every
  * route s < T*topk whose expert (0 <= ids[s] < E) has more than cap routes in the call, computes the expert
  * SwiGLU MLP and writes Y fp32 [T*topk][H] row s; other rows are left untouched. The weights are decoded into LDS
- * as fp16 (the reconstruct's rounding, ft_core.h:75-83) once per 128 routes and multiplied on MFMA; fp16
+ * as fp16 (the reconstruct's rounding, ft_core.h:75-83) once per 96 or 256 routes and multiplied on MFMA; fp16
  * activations, fp32 accumulation, fp16 rounding at the reference's points. x, x_dtype as for mm_expert_gemv
  * (no rescale). Needs H a multiple of 256, I of 128, E <= 1024. */
 int mm_grouped_gemm(const mm_layer_t* layer, const void* x, int x_dtype, int T, int topk, const int64_t* ids, int cap,
@@ -204,9 +204,10 @@ int mm_moe_prefill(const mm_layer_t* layer, const void* x, int x_dtype, int T, i
 /* The fused-MoE call of a prefill-sized batch (patches/vllm-exl3-host-dma.patch:241-449: experts with more than
  * the fat threshold routes through the fat-expert GEMM, patch:286-291,450-460, the others through the fused
  * group kernel), with the split made on the device: out fp32 [T][H] = sum_j w[t,j] * expert_{ids[t,j]}(x_t) over
- * the valid routes, where experts with more than cap routes run on the grouped GEMM (fp16-rounded weights, as the
- * reference's reconstruct) and the others on the decode path (the layer's codebook evaluation), each token's
- * decode-path routes added in ascending j onto its fat-expert sum. No host synchronisation: the call can be
+ * the valid routes. Up to 1,024 routes, experts with more than cap routes run on the grouped GEMM and the others on
+ * the decode path, each token's decode-path routes added in ascending j onto its fat-expert sum; larger calls run every
+ * expert on the grouped GEMM, added in ascending j. Weights follow the layer's codebook evaluation (MM_LAYER_EXACT or
+ * not), except in tiles of 256 routes, which round them to fp16 as the reference's reconstruct does. No host synchronisation: the call can be
  * captured. ids int64 [T*topk], w fp32 [T*topk], topk <= 16, cap >= 1; x as for mm_moe_prefill. Workspace:
  * mm_fused_moe_workspace(T, topk, E, H, I, cap) bytes. */
 size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap);

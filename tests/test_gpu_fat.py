@@ -223,3 +223,56 @@ def test_fused_moe_device_split_vs_oracle(dev, T, k, E, cap):
     ref = OracleLayer(st, seed).forward(x16.astype(np.float32), ids, w)
     ok, m = within_tolerance(out.cpu().numpy(), ref)
     assert ok, m
+
+
+@pytest.mark.parametrize("exact", [True, False])
+def test_row_group_tiles_at_their_edges(dev, exact):
+    """Experts whose routes end on either side of the row groups of 32, of the tiles of 96 and of 192, through the grouped
+    GEMM (fp16-rounded weights) and through a fused call of more than 1,024 routes (the layer's evaluation), down GEMM
+    of four steps (two per half of K)."""
+    import torch
+    from mi355moe import moe
+    H, I, seed = 512, 128, 8181
+    counts = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256, 289]
+    E = len(counts)
+    st = make_store(E, H, I, seed, device=dev, exact=exact)
+    rng = np.random.default_rng(13)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
+    T = ids.shape[0]
+    w = np.ones((T, 1), np.float32)
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    print(f"row group tiles T={T} exact={exact}", flush=True)
+    assert T > 1024
+    Y = moe.grouped_gemm(st, _t(x16, dev), _t(ids, dev), cap=0)
+    out = moe.fused_moe(st, _t(x16, dev), _t(ids, dev), _t(w, dev), 32)
+    torch.cuda.synchronize()
+    ref = OracleLayer(st, seed).forward(x16.astype(np.float32), ids, w)
+    for e in range(E):
+        rows = ids[:, 0] == e
+        for name, got in (("grouped", Y), ("fused", out)):
+            ok, m = within_tolerance(got.cpu().numpy()[rows], ref[rows])
+            assert ok, (name, counts[e], m)
+
+
+def test_full_tiles_of_a_large_call(dev):
+    """Enough 256-route tiles to take their own kernels (at least three rounds of 256 workgroups of them), with remainders
+    of one route, of one and of two row groups, and partial tiles of 193 and 255 routes: sampled rows of every expert."""
+    import torch
+    from mi355moe import moe
+    H, I, seed = 256, 2048, 8282
+    counts = [193, 255, 256, 257, 290, 330] * 9
+    E = len(counts)
+    assert sum(c // 256 + (c % 256 >= 193) for c in counts) * (I // 128) >= 3 * 256
+    st = make_store(E, H, I, seed, device=dev, exact=True)
+    rng = np.random.default_rng(14)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
+    T = ids.shape[0]
+    w = np.ones((T, 1), np.float32)
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    print(f"full tiles T={T}", flush=True)
+    out = moe.fused_moe(st, _t(x16, dev), _t(ids, dev), _t(w, dev), 32)
+    torch.cuda.synchronize()
+    rows = np.concatenate([np.flatnonzero(ids[:, 0] == e)[[0, 100, 192, -1]] for e in range(E)])
+    ref = OracleLayer(st, seed).forward(x16[rows].astype(np.float32), ids[rows], w[rows])
+    ok, m = within_tolerance(out.cpu().numpy()[rows], ref)
+    assert ok, m
