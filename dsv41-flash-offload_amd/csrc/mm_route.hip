@@ -217,6 +217,18 @@ __device__ __forceinline__ int rm_at(int r, int q) { return r * RM_ROW + 8 * (q 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float rm_f4_t __attribute__((ext_vector_type(4)));
 
+// g = g1 + g2 + g3 as bf16 bits
+__device__ __forceinline__ void bf16_parts(float g, uint32_t& a, uint32_t& b, uint32_t& c)
+{
+    const uint32_t h1 = __float_as_uint(g) & 0xffff0000u;
+    const float r1 = g - __uint_as_float(h1);
+    const uint32_t h2 = __float_as_uint(r1) & 0xffff0000u;
+    const float r2 = r1 - __uint_as_float(h2);
+    a = h1 >> 16;
+    b = h2 >> 16;
+    c = __float_as_uint(r2) >> 16;
+}
+
 template <int TM, int TN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void k_router_mfma(const uint16_t* __restrict__ x, const float* __restrict__ G,
                                                               float* __restrict__ logits, int T, int H, int E)
@@ -264,15 +276,6 @@ __global__ __launch_bounds__(64 * WM * WN) void k_router_mfma(const uint16_t* __
 #pragma unroll
         for (int j = 0; j < GL; ++j) gv[j] = gin[j] ? *reinterpret_cast<const float4*>(gp[j] + k0) : make_float4(0, 0, 0, 0);
     };
-    auto split = [](float g, uint32_t& a, uint32_t& b, uint32_t& c) {
-        const uint32_t h1 = __float_as_uint(g) & 0xffff0000u;
-        const float r1 = g - __uint_as_float(h1);
-        const uint32_t h2 = __float_as_uint(r1) & 0xffff0000u;
-        const float r2 = r1 - __uint_as_float(h2);
-        a = h1 >> 16;
-        b = h2 >> 16;
-        c = __float_as_uint(r2) >> 16;
-    };
     rm_f4_t acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -289,10 +292,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_router_mfma(const uint16_t* __
         for (int j = 0; j < GL; ++j)
         {
             uint32_t a[4], b[4], c[4];
-            split(gv[j].x, a[0], b[0], c[0]);
-            split(gv[j].y, a[1], b[1], c[1]);
-            split(gv[j].z, a[2], b[2], c[2]);
-            split(gv[j].w, a[3], b[3], c[3]);
+            bf16_parts(gv[j].x, a[0], b[0], c[0]);
+            bf16_parts(gv[j].y, a[1], b[1], c[1]);
+            bf16_parts(gv[j].z, a[2], b[2], c[2]);
+            bf16_parts(gv[j].w, a[3], b[3], c[3]);
             const int o = rm_at(gr[j], gq[j] >> 1) + 4 * (gq[j] & 1);
             *reinterpret_cast<uint2*>(&gs[0][o]) = make_uint2(a[0] | (a[1] << 16), a[2] | (a[3] << 16));
             *reinterpret_cast<uint2*>(&gs[1][o]) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
@@ -331,6 +334,113 @@ __global__ __launch_bounds__(64 * WM * WN) void k_router_mfma(const uint16_t* __
                 if (t < T && e < E) logits[(size_t)t * E + e] = acc[i][j][r];
             }
         }
+}
+
+// The same products for calls too small to fill the GPU with 128 x 192 tiles: a workgroup takes 16 MI tokens x 16 NJ
+// experts and splits H over its NW waves, each with a contiguous run of 32-element steps whose operands it loads straight
+// into MFMA layout (two steps at a time, the next two in flight) and splits in registers; the waves' sums are added through
+// LDS in wave order. Rows past T or E repeat the last one and are not stored.
+//
+// What bounds it is the operand loads (each workgroup reads its rows from L2). The launch takes the smallest tile whose
+// workgroups still fit the GPU's CUs (RS_CUS) once, so every call of up to 512, 1,024 and, at two rounds, 4,096 tokens x 384
+// experts is one or two rounds deep. Router call, H 4096: 65 to 512 tokens 31 us (32 x 32 tiles), 700 and 1,024 tokens 40
+// (64 x 32; 55 with 32 x 32), 2,048 tokens 52 (64 x 48; 73 with 64 x 32), 4,096 tokens 96; the 128 x 192 tiles take 156 to
+// 162 us at all of these (12 to 64 workgroups) and 168 at 8,192 tokens, where 64 x 48 takes 181. Four steps in flight
+// instead of two: 34, 57 us.
+constexpr size_t RS_CUS = 256;
+template <int MI, int NJ, int NW>
+__global__ __launch_bounds__(64 * NW) void k_router_split(const uint16_t* __restrict__ x, const float* __restrict__ G,
+                                                          float* __restrict__ logits, int T, int H, int E)
+{
+    constexpr int TM = 16 * MI, TN = 16 * NJ, GS = 2;
+    __shared__ float part[NW][TM][TN + 1];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = blockIdx.y * TM, e0 = blockIdx.x * TN;
+    const int S = H / RM_K, s0 = S * wave / NW, s1 = S * (wave + 1) / NW;
+    const int r = lane & 15, q = lane >> 4;                   // operand row and k-group of 8
+    const uint16_t* xp[MI];
+    const float* gp[NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) xp[i] = x + (size_t)min(t0 + 16 * i + r, T - 1) * H + 8 * q;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) gp[j] = G + (size_t)min(e0 + 16 * j + r, E - 1) * H + 8 * q;
+    uint4 xv[2][GS][MI];
+    float4 gv[2][GS][NJ][2];
+    // steps s .. s + GS - 1 (past the run: its last step again, not multiplied)
+    auto load = [&](int s, int b) {
+#pragma unroll
+        for (int u = 0; u < GS; ++u)
+        {
+            const int k0 = max(min(s + u, s1 - 1), 0) * RM_K;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) xv[b][u][i] = *reinterpret_cast<const uint4*>(xp[i] + k0);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+            {
+                gv[b][u][j][0] = *reinterpret_cast<const float4*>(gp[j] + k0);
+                gv[b][u][j][1] = *reinterpret_cast<const float4*>(gp[j] + k0 + 4);
+            }
+        }
+    };
+    rm_f4_t acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = rm_f4_t{ 0.f, 0.f, 0.f, 0.f };
+    auto step = [&](int s, int b) {
+#pragma unroll
+        for (int u = 0; u < GS; ++u)
+        {
+            if (s + u >= s1) break;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+            {
+                const float* g = reinterpret_cast<const float*>(&gv[b][u][j][0]);
+                uint32_t w[3][4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                {
+                    uint32_t lo[3], hi[3];
+                    bf16_parts(g[2 * c], lo[0], lo[1], lo[2]);
+                    bf16_parts(g[2 * c + 1], hi[0], hi[1], hi[2]);
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) w[p][c] = lo[p] | (hi[p] << 16);
+                }
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                {
+                    const bf16x8_t B = __builtin_bit_cast(bf16x8_t, make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]));
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xv[b][u][i]), B,
+                                                                            acc[i][j], 0, 0, 0);
+                }
+            }
+        }
+    };
+    load(s0, 0);
+    for (int s = s0; s < s1; s += 2 * GS)
+    {
+        load(s + GS, 1);
+        step(s, 0);
+        load(s + 2 * GS, 0);
+        step(s + GS, 1);
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) part[wave][16 * i + 4 * q + v][16 * j + r] = acc[i][j][v];
+    __syncthreads();
+    for (int o = threadIdx.x; o < TM * TN; o += 64 * NW)
+    {
+        const int t = o / TN, e = o % TN;
+        float sum = part[0][t][e];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) sum += part[w][t][e];
+        if (t0 + t < T && e0 + e < E) logits[(size_t)(t0 + t) * E + e0 + e] = sum;
+    }
 }
 
 // One wave per token: k rounds of a wave-wide argmax (ties to the lower index), then softmax over the picks.
@@ -1043,9 +1153,20 @@ int mm_router_topk(const void* x_bf16, int T, int H, const float* gate, int E, i
         hipLaunchKernelGGL(k_router_gemv<16>, dim3(E, (T + 15) / 16), dim3(256), 0, S(stream), (const uint16_t*)x_bf16,
                            gate, logits, T, H, E);
     else if (H % RM_K == 0 && ((uintptr_t)x_bf16 & 15) == 0 && ((uintptr_t)gate & 15) == 0)
-        hipLaunchKernelGGL((k_router_mfma<RM_TM, RM_TN, RM_WM, RM_WN>), dim3((E + RM_TN - 1) / RM_TN,
-                           (T + RM_TM - 1) / RM_TM), dim3(64 * RM_WM * RM_WN), 0, S(stream),
-                           (const uint16_t*)x_bf16, gate, logits, T, H, E);
+    {
+        const uint16_t* xb = (const uint16_t*)x_bf16;
+        auto grid = [&](int tm, int tn) { return dim3((E + tn - 1) / tn, (T + tm - 1) / tm); };
+        auto blocks = [&](int tm, int tn) { const dim3 g = grid(tm, tn); return (size_t)g.x * g.y; };
+        if (blocks(32, 32) <= RS_CUS)
+            hipLaunchKernelGGL((k_router_split<2, 2, 8>), grid(32, 32), dim3(512), 0, S(stream), xb, gate, logits, T, H, E);
+        else if (blocks(64, 32) <= RS_CUS)
+            hipLaunchKernelGGL((k_router_split<4, 2, 8>), grid(64, 32), dim3(512), 0, S(stream), xb, gate, logits, T, H, E);
+        else if (blocks(64, 48) <= 2 * RS_CUS)
+            hipLaunchKernelGGL((k_router_split<4, 3, 8>), grid(64, 48), dim3(512), 0, S(stream), xb, gate, logits, T, H, E);
+        else
+            hipLaunchKernelGGL((k_router_mfma<RM_TM, RM_TN, RM_WM, RM_WN>), grid(RM_TM, RM_TN),
+                               dim3(64 * RM_WM * RM_WN), 0, S(stream), xb, gate, logits, T, H, E);
+    }
     else
         hipLaunchKernelGGL(k_router_logits, dim3((E + 63) / 64, (T + 63) / 64), dim3(256), 0, S(stream),
                            (const uint16_t*)x_bf16, gate, logits, T, H, E);

@@ -258,3 +258,31 @@ def test_router_at_prefill_size(dev):
         if not np.array_equal(gi[t], rid[t]):
             srt = np.sort(rl[t])[::-1]
             assert np.min(np.abs(np.diff(srt[: k + 1]))) < 1e-5, t
+
+
+@pytest.mark.parametrize("T,H,E,k", [(65, 96, 40, 4), (97, 4128, 33, 3), (513, 512, 384, 8), (682, 256, 385, 8), (683, 256, 384, 6),
+                                     (1025, 512, 384, 8), (1367, 224, 384, 8), (4097, 64, 384, 8), (300, 5120, 1024, 6)])
+def test_router_tile_choice(dev, T, H, E, k):
+    """Calls on either side of the lines between the router's tile shapes, with partial token and expert tiles and with
+    fewer 32-element steps than waves: logits within the worst case of an fp32 sum of H products in any order, picks the
+    top k of the logits themselves."""
+    import torch
+    from mi355moe import _lib
+    g = torch.Generator(device=dev)
+    g.manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=dev).bfloat16()
+    G = torch.randn((E, H), generator=g, device=dev) * 0.02
+    ids = torch.empty((T, k), dtype=torch.int64, device=dev)
+    w = torch.empty((T, k), dtype=torch.float32, device=dev)
+    logits = torch.full((T + 1, E), float("nan"), device=dev)
+    print(f"router tiles T={T} H={H} E={E}", flush=True)
+    _lib.call("mm_router_topk", x.data_ptr(), T, H, G.data_ptr(), E, k, logits.data_ptr(), ids.data_ptr(), w.data_ptr(),
+              _lib.stream_ptr())
+    torch.cuda.synchronize()
+    assert bool(logits[T].isnan().all())
+    xd, gd = x.double(), G.double()
+    bound = H * 2.0 ** -24 * (xd.abs() @ gd.abs().t())
+    assert bool(((logits[:T].double() - xd @ gd.t()).abs() <= bound).all())
+    sel = logits[:T].gather(1, ids)
+    assert torch.equal(sel, logits[:T].topk(k, dim=1).values)
+    assert torch.allclose(w, torch.softmax(sel.double(), dim=1).float(), rtol=1e-5, atol=1e-6)
