@@ -132,9 +132,8 @@ int prep_blocks(int H);
 void launch_route_prep(const PrepArgs& p, hipStream_t s);
 
 // The launches of mm_moe_decode on a given workspace (argument checks included); `who` names the caller in errors.
-// accumulate: out += the layer sum instead of out = the layer sum.
 int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int rescale, int T, int topk, const int64_t* ids,
                       const float* w, int max_rows, float* out, void* workspace, size_t workspace_bytes,
-                      mm_stream_t stream, const char* who, int accumulate = 0);
+                      mm_stream_t stream, const char* who);
 
 }  // namespace mm

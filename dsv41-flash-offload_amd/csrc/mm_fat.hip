@@ -1540,54 +1540,14 @@ static FatbWs fatb_carve(void* base, int n, int T, int E, int H, int I)
 
 // ------------------------------------------------------------------------------------ the fused-MoE call
 
-// Calls of more routes than the decode path routes in-kernel run every expert on the grouped GEMM: k_mid decodes a tile as
-// fast for one route as for 32, so an expert with few routes costs it what the decode path pays per 16 (34 against 33 ns per
-// 16 x 16 tile and SIMD), and the decode path's launches over all tokens, for the few routes it is left with, go (at 4,096
-// tokens its combine alone took 0.64 ms, at 16,384 tokens 2.0 ms).
-constexpr int FUSED_SPLIT_MAX = 1024;
-
-// ids_small[s] = ids[s] when its expert has at most cap routes in the call (counts from the fat pass's
-// permutation), else -1: the routes the decode path takes.
-__global__ __launch_bounds__(256) void k_small_ids(const int64_t* __restrict__ ids, const int32_t* __restrict__ counts,
-                                                   int n, int E, int cap, int64_t* __restrict__ ids_small)
-{
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x)
-    {
-        const int64_t e = ids[s];
-        ids_small[s] = (e >= 0 && e < E && counts[e] <= cap) ? e : -1;
-    }
-}
-
-// Workspace of mm_fused_moe: the fat pass over all n routes, then (calls of at most FUSED_SPLIT_MAX routes) the decode
-// path's ids and workspace.
-struct FusedWs
-{
-    FatWs fat;
-    int64_t* ids_small;   // [n]
-    void* dws;            // decode workspace
-    size_t dws_bytes, bytes;
-};
-
-static FusedWs fused_carve(void* base, int T, int topk, int E, int H, int I)
-{
-    const int n = T * topk;
-    FusedWs w;
-    w.fat = fat_carve(base, n, E, H, I);
-    w.ids_small = nullptr;
-    w.dws = nullptr;
-    w.dws_bytes = 0;
-    w.bytes = w.fat.bytes;
-    if (n > FUSED_SPLIT_MAX) return w;
-    const size_t ids = ((size_t)n * 8 + 255) & ~(size_t)255;
-    w.dws_bytes = mm_gemv_workspace(n, E, H, I);
-    if (base)
-    {
-        w.ids_small = reinterpret_cast<int64_t*>(static_cast<char*>(base) + w.bytes);
-        w.dws = static_cast<char*>(base) + w.bytes + ids;
-    }
-    w.bytes += ids + w.dws_bytes;
-    return w;
-}
+// A call runs as a whole on one path. Up to FUSED_DECODE_MAX routes it is the decode path, whose launches cut the experts'
+// rows into equal runs over the whole GPU; an expert with many routes costs it a pass per 16, which few experts of such a
+// call need. Above, it is the grouped GEMM: k_mid decodes a tile as fast for one route as for 32 (34 against 33 ns per 16 x 16
+// tile and SIMD), and the decode path's combine over all tokens grows with the call (at 4,096 tokens 0.64 ms). Whole calls on
+// the decode path / on the grouped GEMM, H 4096, top-8 of 384: 100 tokens 741 / 796 us (Zipf routing) and 856 / 970 (64 hot
+// experts), 128 tokens 854 / 897 and 957 / 1,068; beyond 1,024 routes the decode path needs the permutation. Against the
+// experts divided by cap over both paths: 884 and 879 us at 100 tokens.
+constexpr int FUSED_DECODE_MAX = 1024;
 
 }  // namespace mm
 
@@ -1598,7 +1558,8 @@ extern "C" {
 size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap)
 {
     if (T <= 0 || topk <= 0 || E <= 0 || H <= 0 || I <= 0 || cap < 0) return 0;
-    return fused_carve(nullptr, T, topk, E, H, I).bytes;
+    const int n = T * topk;
+    return n <= FUSED_DECODE_MAX ? mm_gemv_workspace(n, E, H, I) : fat_carve(nullptr, n, E, H, I).bytes;
 }
 
 int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1609,23 +1570,18 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
     MM_CHECK_ARG(w && out && cap >= 1, "mm_fused_moe: null pointer or cap < 1");
     MM_CHECK_ARG(topk <= 16, "mm_fused_moe: topk must be at most 16");
     const int n = T * topk, E = L->E;
-    const FusedWs ws = fused_carve(workspace, T, topk, E, L->H, L->I);
     // a limit of the interface: n, or E x cap for larger n, transformed inputs within 32-bit byte offsets
-    const size_t npos = n <= FUSED_SPLIT_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
+    const size_t npos = n <= FUSED_DECODE_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
     MM_CHECK_ARG(npos * 2 * std::max(L->H, L->I) * 2 < ((size_t)1 << 31),
                  "mm_fused_moe: too many decode-path positions (%zu)", npos);
-    MM_CHECK_ARG(workspace && workspace_bytes >= ws.bytes, "mm_fused_moe: workspace too small (%zu < %zu)",
-                 workspace_bytes, ws.bytes);
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (n > FUSED_SPLIT_MAX) return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, ws.fat, s, true);
-    // 1. experts above cap on the grouped GEMM: out = their weighted sum (every token written)
-    int r = fat_layer(L, x, x_dtype, T, topk, ids, w, cap, 0, out, ws.fat, s, true);
-    if (r) return r;
-    // 2. the others on the decode path, added per token in ascending route order
-    hipLaunchKernelGGL(k_small_ids, dim3((unsigned)std::min((n + 255) / 256, 1024)), dim3(256), 0, s, ids,
-                       ws.fat.counts, n, E, cap, ws.ids_small);
-    return moe_decode_launch(L, x, x_dtype, 0, T, topk, ws.ids_small, w, cap, out, ws.dws, ws.dws_bytes, stream,
-                             "mm_fused_moe", 1);
+    const size_t need = mm_fused_moe_workspace(T, topk, E, L->H, L->I, cap);
+    MM_CHECK_ARG(workspace && workspace_bytes >= need, "mm_fused_moe: workspace too small (%zu < %zu)", workspace_bytes,
+                 need);
+    if (n <= FUSED_DECODE_MAX)
+        return moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, workspace, workspace_bytes, stream,
+                                 "mm_fused_moe");
+    return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I),
+                     reinterpret_cast<hipStream_t>(stream), true);
 }
 
 size_t mm_prefill_workspace(int n, int E, int H, int I)

@@ -34,6 +34,13 @@ constexpr int GV_WAVES = 4;
 constexpr int GV_THREADS = 64 * GV_WAVES;
 constexpr int GV_COLS = 128;          // output columns per segment (8 tiles)
 constexpr int GV_ROUTE_MAX = 1024;    // in-kernel routing limit (routes per call)
+// Routes per record (one pass of a partial-sum wave) with in-kernel routing of more than this many tokens. A segment costs
+// its waves one pass over its rows, whatever its routes, so equal runs of rows are equal work: with one record per expert
+// the waves of an expert with more than 16 routes took twice as long as the others and the launch waited for them (24
+// tokens, top-8 and the shared expert: 357 -> 304 us a call; 100 tokens on the decode path alone 741 us, against 884 with its
+// busy experts on the grouped GEMM). Fewer tokens keep one record per expert, found from a bitmap (the counts cost the
+// one-token layer 1 %); a token that picks an expert twice only makes a longer record.
+constexpr int REC_ROUTES = 16;
 constexpr int GV_RING = 4;            // tile rows in flight per wave (even: rows go through MFMA in pairs)
 static_assert(GV_RING % 2 == 0, "row pairs");
 constexpr int ROW_BYTES = 8 * 96;     // one tile row of a segment
@@ -98,7 +105,8 @@ __device__ __forceinline__ float load_x_t(const void* x, size_t i)
 template <int XD>
 __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
 {
-    __shared__ uint32_t s_bm[32];
+    // in-kernel routing (E <= 1024): each expert's routes, or (one record per expert) a bitmap of the experts present
+    __shared__ __align__(16) int s_hist[GV_ROUTE_MAX];
     __shared__ int s_cnt[4][4];
     __shared__ float s_ss[4];
     __shared__ int s_ai;
@@ -106,6 +114,7 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     const int blk = blockIdx.x % a.nb, m = (blockIdx.x / a.nb) & 1, idx = blockIdx.x / (2 * a.nb);
     const bool writer = m == 0 && blk == 0;      // the one workgroup of a route that writes its routing data
     const bool perm = a.offsets != nullptr;
+    const bool split = !perm && a.n > REC_ROUTES * a.topk;   // more than REC_ROUTES tokens: records of REC_ROUTES routes
     // routing from the permutation: the workgroups of index idx own sorted position idx
     const int nvalid_perm = perm ? a.offsets[a.E] : 0;
     const int s = perm ? a.order[idx] : idx;
@@ -160,7 +169,10 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
             ss = fmaf(v, v, ss);
         }
     }
-    if (tid < 32) s_bm[tid] = 0;
+    if (split)
+        *reinterpret_cast<int4*>(&s_hist[4 * tid]) = make_int4(0, 0, 0, 0);
+    else if (tid < 32)
+        s_hist[tid] = 0;
     if (tid == 0) s_ai = -1;
     __syncthreads();
 #pragma unroll
@@ -174,7 +186,8 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
         const int64_t v = rid[k];
         const int i = tid + 256 * k;
         if (perm || i >= a.n || v < 0 || v >= a.E) continue;
-        atomicOr(&s_bm[v >> 5], 1u << (v & 31));
+        if (split) atomicAdd(&s_hist[v], 1);
+        else atomicOr(&s_hist[v >> 5], 1 << (v & 31));
         nv += 1;
         less += v < e;
         same += v == e;
@@ -202,15 +215,36 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     // an expert with more than cap routes belongs to the fat-expert path: its positions stay reserved, but it gets
     // an empty record and its routes no transformed inputs and no outputs
     const bool fat = valid && (perm ? pcnt : same) > a.cap;
-    // in-kernel routing: the experts present below the route's expert (its record index) and in all, from the
-    // bitmap by one reduction over the first wave
+    // in-kernel routing: the records of the experts below the route's expert and of all, by one reduction over the first
+    // wave (records of REC_ROUTES routes: lane l takes experts 16 l .. 16 l + 15)
     int below = 0, present = 0;
     if (!perm && wave == 0 && (writer || blockIdx.x == 0))
     {
-        const uint32_t wd = lane < 32 ? s_bm[lane] : 0u;
-        const int eb = valid ? (e >> 5) : -1;
-        below = wave_sum_int(lane < eb ? __popc(wd) : (lane == eb ? __popc(wd & ((1u << (e & 31)) - 1u)) : 0));
-        present = wave_sum_int(__popc(wd));
+        if (split)
+        {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                const int4 c = *reinterpret_cast<const int4*>(&s_hist[16 * lane + 4 * k]);
+                const int cc[4] = { c.x, c.y, c.z, c.w };
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                {
+                    const int nr = (cc[u] + REC_ROUTES - 1) / REC_ROUTES;
+                    present += nr;
+                    below += 16 * lane + 4 * k + u < e ? nr : 0;
+                }
+            }
+        }
+        else
+        {
+            const uint32_t wd = lane < 32 ? (uint32_t)s_hist[lane] : 0u;
+            const int eb = valid ? (e >> 5) : -1;
+            below = lane < eb ? __popc(wd) : (lane == eb ? __popc(wd & ((1u << (e & 31)) - 1u)) : 0);
+            present = __popc(wd);
+        }
+        below = wave_sum_int(below);
+        present = wave_sum_int(present);
     }
     if (tid == 0 && (writer || blockIdx.x == 0))
     {
@@ -221,9 +255,9 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
         }
         if (writer)
         {
-            // the expert's active index: experts present below it (in-kernel routing), or its place in the
-            // permutation's active list (-1 if absent there)
-            const int ai = !valid ? -1 : (perm ? s_ai : below);
+            // the route's record: an expert's come after those of the experts below it, one per REC_ROUTES routes or one in
+            // all; with a permutation it has one, at its place in the active list (-1 if absent there)
+            const int ai = !valid ? -1 : (perm ? s_ai : below + (split ? rank / REC_ROUTES : 0));
             a.pos_of[s] = valid && !fat ? pos : -1;
             a.ai_of[s] = valid && !fat ? ai : -1;
             if (valid)
@@ -231,11 +265,11 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
                 a.route_at[pos] = s;
                 a.e_at[pos] = fat ? -1 : e;
                 a.ai_at[pos] = fat ? -1 : ai;
-                // the expert's first route writes its record
-                const bool first_route = perm ? pos == a.offsets[e] : rank == 0;
+                // the record's first route writes it
+                const bool first_route = perm ? pos == a.offsets[e] : (split ? rank % REC_ROUTES : rank) == 0;
                 if (first_route && ai >= 0)
                 {
-                    const int cnt = perm ? a.offsets[e + 1] - pos : same;
+                    const int cnt = perm ? a.offsets[e + 1] - pos : split ? min(same - rank, REC_ROUTES) : same;
                     ExpertRec r{ e, fat ? 0 : cnt, pos, 0, { wt0, wt1, wt2 }, 0 };
                     a.rec[ai] = r;
                 }
@@ -660,7 +694,6 @@ struct DEpiArgs
     float* Y;                 // [n][H] (per-route rows)
     float* out;               // [T][H] (combine)
     int npos, H, I, topk, nwaves, cap, affine;
-    int accumulate;           // combine: out += the sum instead of out = the sum
 };
 
 // Down output of one (sorted position, 128-column block of H): pieces added in order (then the AFFINE
@@ -749,7 +782,7 @@ __global__ __launch_bounds__(1024) void k_down_combine(DEpiArgs a)
     for (int h = threadIdx.x; h < GV_COLS; h += blockDim.x)
     {
         float* dst = a.out + (size_t)t * a.H + c + h;
-        float o = a.accumulate ? *dst : 0.0f;
+        float o = 0.0f;
         for (int jj = 0; jj < a.topk; ++jj)
             if (ok[jj]) o = fmaf(wj[jj], ys[jj][h], o);
         *dst = o;
@@ -796,12 +829,15 @@ static int piece_cap(int n)
     return c > 32 ? 32 : (c < 4 ? 4 : c);
 }
 
+// Most records of n routes over E experts.
+static int max_records(int n, int E) { return (n < E ? n : E) + n / REC_ROUTES; }
+
 // Workspace of n routes whose sorted positions lie below npos (npos = n unless a caller bounds the positions).
 static Ws carve(void* base, int n, int npos, int E, int H, int I)
 {
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t m = (size_t)npos;
-    const size_t na = (size_t)(npos < E ? npos : E), cap = (size_t)piece_cap(npos);
+    const size_t na = (size_t)max_records(npos, E), cap = (size_t)piece_cap(npos);
     // the small routing arrays first and together (records, counts, pos_of, route_at, e_at, ai_at, ai_of), so the
     // epilogues' first loads fall in the same few pages
     const size_t sizes[13] = { al(na * sizeof(ExpertRec)), al(2 * 4), al((size_t)n * 4), al(m * 4),
@@ -879,7 +915,7 @@ static int check_common(const mm_layer_t* L, const void* x, int x_dtype, int T, 
     MM_CHECK_ARG(T > 0 && n > 0 && topk > 0 && n <= T * topk, "%s: bad T/n/topk", who);
     MM_CHECK_ARG((size_t)n * 2 * (L->H > L->I ? L->H : L->I) * 2 < ((size_t)1 << 31), "%s: too many routes", who);
     // tile rows of a partial launch (active experts x 2 matrices x column blocks x tile rows) count in int
-    MM_CHECK_ARG((size_t)(n < L->E ? n : L->E) * L->H / 1024 * L->I < ((size_t)1 << 31), "%s: too many routes", who);
+    MM_CHECK_ARG((size_t)max_records(n, L->E) * L->H / 1024 * L->I < ((size_t)1 << 31), "%s: too many routes", who);
     MM_CHECK_ARG(max_rows > 0, "%s: max_rows must be at least 1", who);
     const bool perm = offsets != nullptr;
     MM_CHECK_ARG(perm ? (order && active && nactive) : n <= GV_ROUTE_MAX,
@@ -921,16 +957,16 @@ static void launch_gu_epilogue(const mm_layer_t* L, const Ws& w, int npos, hipSt
 }
 
 static DEpiArgs down_args(const mm_layer_t* L, const Ws& w, int npos, int topk, const int64_t* ids, const float* wt,
-                          float* Y, float* out, int accumulate)
+                          float* Y, float* out)
 {
     return DEpiArgs{ w.part_d, w.xdsum, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, ids, wt, L->svh2, Y, out, npos, L->H,
-                     L->I, topk, partial_waves(seg_max(L, npos, 1)), piece_cap(npos), (L->flags & MM_LAYER_EXACT) ? 0 : 1, accumulate };
+                     L->I, topk, partial_waves(seg_max(L, npos, 1)), piece_cap(npos), (L->flags & MM_LAYER_EXACT) ? 0 : 1 };
 }
 
 // One decode layer (mm_moe_decode) on a caller-provided workspace; `who` names the entry point in errors.
 int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int rescale, int T, int topk, const int64_t* ids,
                       const float* w, int max_rows, float* out, void* workspace, size_t workspace_bytes,
-                      mm_stream_t stream, const char* who, int accumulate)
+                      mm_stream_t stream, const char* who)
 {
     MM_CHECK_ARG(topk > 0 && topk <= MAX_TOPK, "%s: topk must be in [1, %d]", who, MAX_TOPK);
     const int n = T * topk;
@@ -946,7 +982,7 @@ int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int resca
     launch_partial<1>(L, ws, n, s);
     const int threads = 64 * (topk < 2 ? 2 : topk);
     hipLaunchKernelGGL(k_down_combine, dim3(T * (L->H / GV_COLS)), dim3(threads), 0, s,
-                       down_args(L, ws, n, topk, ids, w, nullptr, out, accumulate));
+                       down_args(L, ws, n, topk, ids, w, nullptr, out));
     return check_launch(who);
 }
 
@@ -980,7 +1016,7 @@ int mm_expert_gemv(const mm_layer_t* L, const void* x, int x_dtype, int rescale,
     if (phases & 8) launch_partial<1>(L, w, n, s);
     if (phases & 16)
         hipLaunchKernelGGL(k_down_y, dim3((n * (L->H / GV_COLS) + 3) / 4), dim3(256), 0, s,
-                           down_args(L, w, n, topk, ids, nullptr, Y, nullptr, 0));
+                           down_args(L, w, n, topk, ids, nullptr, Y, nullptr));
     return check_launch("mm_expert_gemv");
 }
 
@@ -988,7 +1024,7 @@ int mm_moe_decode(const mm_layer_t* L, const void* x, int x_dtype, int rescale, 
                   const float* w, int max_rows, float* out, void* workspace, size_t workspace_bytes, mm_stream_t stream)
 {
     return mm::moe_decode_launch(L, x, x_dtype, rescale, T, topk, ids, w, max_rows, out, workspace, workspace_bytes,
-                                 stream, "mm_moe_decode", 0);
+                                 stream, "mm_moe_decode");
 }
 
 }  // extern "C"

@@ -1,9 +1,9 @@
 """The vllm_exl3 MoE entry points the reference patches (patches/vllm-exl3-host-dma.patch), over this library.
 
   apply_exl3_fused_moe(x2d, ids, weights, layer, inners, expert_map, limit) -> contiguous fp32 [T, H]
-      the fused-MoE call (patch:241-449): routes of experts with more than FAT_EXPERT_THRESHOLD rows go to the
-      fat-expert grouped GEMM, the rest to the decode path; with host-resident experts and at least
-      _DMA_MIN_TOKENS tokens, the experts not in HBM are streamed through staging slots (EXL3_HOST_DMA).
+      the fused-MoE call (patch:241-449), on the decode path or the fat-expert grouped GEMM by its size; with
+      host-resident experts and at least _DMA_MIN_TOKENS tokens, the experts not in HBM are streamed through staging
+      slots (EXL3_HOST_DMA).
   apply_exl3_batched_fat(xh, token_sorted, weight_sorted, counts_host, inners, limit, cap, out, use_kernel, skip)
       the fat-expert entry on expert-sorted routes (patch:182-201), accumulating into out.
   Exl3MoEMethod.process_weights_after_loading(layer)
@@ -298,9 +298,8 @@ def apply_exl3_fused_moe(x2d, ids, weights, layer, inners=None, expert_map=None,
     if (_EXL3_HOST_DMA_MODE > 0 and layer.host_home is not None and getattr(layer, "_exl3_dma", None) is not None
             and T >= _DMA_MIN_TOKENS and inners is None and not torch.cuda.is_current_stream_capturing()):
         return _dma_prefill(x2d, ids, w16, layer, limit, dev)
-    # at most FAT_EXPERT_THRESHOLD tokens: every route on the decode path (the reference's fat_possible test);
-    # above it the experts with more than FAT_EXPERT_THRESHOLD routes go to the fat-expert GEMM. Both are decided on
-    # the device, so no call synchronises the host and every call can be captured in a graph.
+    # at most FAT_EXPERT_THRESHOLD tokens: every route on the decode path (the reference's fat_possible test); above it
+    # the call's number of routes decides. No call synchronises the host, so every call can be captured in a graph.
     return moe.moe_forward(L, x2d, ids, w16, fat_threshold=FAT_EXPERT_THRESHOLD)
 
 

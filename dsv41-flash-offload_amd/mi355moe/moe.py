@@ -117,9 +117,8 @@ def moe_forward(store, x, ids, w, shared_expert=None, fat_threshold=FAT_THRESHOL
 
     Routes with ids outside [0, E) contribute nothing. As the reference's fused-MoE call does
     (patches/vllm-exl3-host-dma.patch:241-290), a call of at most `fat_threshold` tokens runs every route on the
-    decode path; a larger call sends the experts with more than `fat_threshold` routes to the fat-expert grouped
-    GEMM and the rest to the decode path. The split is made on the device (no host synchronisation), so every
-    call can be captured in a HIP graph."""
+    decode path. A larger call goes to mm_fused_moe, which takes the decode path or the grouped GEMM by its number of
+    routes. No call synchronises the host, so every call can be captured in a HIP graph."""
     T = x.shape[0]
     ids, w = _with_shared(ids, w, T, shared_expert)
     k = ids.shape[1]
@@ -133,9 +132,8 @@ def moe_forward(store, x, ids, w, shared_expert=None, fat_threshold=FAT_THRESHOL
 
 
 def fused_moe(store, x, ids, w, cap, stream=None):
-    """mm_fused_moe: out fp32 [T, H] over ids [T, k] / w [T, k], experts with more than `cap` routes on the
-    grouped GEMM and the others on the decode path, split on the device (calls of more than 1,024 routes run every
-    expert on the grouped GEMM)."""
+    """mm_fused_moe: out fp32 [T, H] over ids [T, k] / w [T, k], on the decode path (up to 1,024 routes) or the grouped
+    GEMM; `cap` is the reference's threshold between the two and only bounds the call's size."""
     T, k = ids.shape
     x = x.contiguous()
     ids = ids.contiguous().long()

@@ -204,10 +204,10 @@ int mm_moe_prefill(const mm_layer_t* layer, const void* x, int x_dtype, int T, i
 /* The fused-MoE call of a prefill-sized batch (patches/vllm-exl3-host-dma.patch:241-449: experts with more than
  * the fat threshold routes through the fat-expert GEMM, patch:286-291,450-460, the others through the fused
  * group kernel), with the split made on the device: out fp32 [T][H] = sum_j w[t,j] * expert_{ids[t,j]}(x_t) over
- * the valid routes. Up to 1,024 routes, experts with more than cap routes run on the grouped GEMM and the others on
- * the decode path, each token's decode-path routes added in ascending j onto its fat-expert sum; larger calls run every
- * expert on the grouped GEMM, added in ascending j. Weights follow the layer's codebook evaluation (MM_LAYER_EXACT or
- * not), except in tiles of 256 routes, which round them to fp16 as the reference's reconstruct does. No host synchronisation: the call can be
+ * the valid routes, added in ascending j. A call of up to 1,024 routes runs on the decode path, a larger one on the
+ * grouped GEMM; cap, the reference's threshold between its two paths, bounds the call's size (E x cap routes' inputs
+ * within 2 GiB) and chooses nothing. Weights follow the layer's codebook evaluation (MM_LAYER_EXACT or not), except in
+ * tiles of 256 routes, which round them to fp16 as the reference's reconstruct does. No host synchronisation: the call can be
  * captured. ids int64 [T*topk], w fp32 [T*topk], topk <= 16, cap >= 1; x as for mm_moe_prefill. Workspace:
  * mm_fused_moe_workspace(T, topk, E, H, I, cap) bytes. */
 size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap);

@@ -370,3 +370,30 @@ def test_decode_cap_leaves_fat_experts_out(dev):
     ref = OracleLayer(st, seed).forward(x16.astype(np.float32), np.where(ids == 0, -1, ids), w)
     ok, m = within_tolerance(out.cpu().numpy(), ref)
     assert ok, m
+
+
+@pytest.mark.parametrize("exact", [False, True])
+def test_decode_layer_with_experts_of_many_routes(dev, exact):
+    """More than 16 tokens on the decode path: experts with 1, 15, 16, 17 and 33 routes and one with every token (records
+    of 16 routes), tokens that pick an expert twice and masked routes, against the oracle."""
+    import torch
+    from mi355moe import moe
+    H, I, seed = 512, 256, 6161
+    counts = [1, 15, 16, 17, 33]
+    E, T = len(counts) + 2, sum(counts)
+    st = make_store(E, H, I, seed, device=dev, exact=exact)
+    rng = np.random.default_rng(21)
+    ids = np.full((T, 3), E - 1, np.int64)
+    ids[:, 0] = rng.permutation(np.repeat(np.arange(len(counts)), counts))
+    ids[:, 2] = -1
+    ids[::9, 2] = ids[::9, 0]
+    w = rng.uniform(0.1, 1.0, (T, 3)).astype(np.float32)
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    print(f"many routes per expert T={T} exact={exact}", flush=True)
+    out = moe.moe_forward(st, _t(x16, dev), _t(ids, dev), _t(w, dev), fat_threshold=T)
+    again = moe.fused_moe(st, _t(x16, dev), _t(ids, dev), _t(w, dev), 32)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    ref = OracleLayer(st, seed).forward(x16.astype(np.float32), ids, w)
+    ok, m = within_tolerance(out.cpu().numpy(), ref)
+    assert ok, m
