@@ -51,7 +51,9 @@ constexpr int FT_BIG_WORK = 3 * 256;
 constexpr int FT_BIG_ROWS = 1024;
 constexpr int GRP_ROWS = 32;        // rows of a row group
 constexpr int GRP_HALVES = 1024;    // one matrix's 32-element step of a row group
-constexpr int PREP_BLOCKS = 4;      // 128-blocks per input transform workgroup
+// 128-blocks per input transform workgroup (16,384 tokens, H 4096, 2.3 GB written: 783 us with 2, 844 with 4, 946 with 8;
+// nontemporal stores of 4: 828 us, and 225 against 204 us at 4,096 tokens)
+constexpr int PREP_BLOCKS = 2;
 constexpr int FT_BN = 256;          // output columns per tile
 constexpr int FT_WAVES = 8;
 constexpr int FT_THREADS = 64 * FT_WAVES;
@@ -400,10 +402,13 @@ __device__ __forceinline__ void* uniform_ptr(const void* p)
 // Epilogue of a fat tile from the transposed fp16 C tile in LDS (column c at c * CS halves, the raw GEMM outputs
 // rounded to fp16): gate/up (MODE 0) applies the output transforms, SwiGLU and the down-input transform of the
 // tile's 128-block and writes the down input in operand order; down (MODE 1) applies the output transform of its
-// two 128-blocks and writes per-route rows. The C tile is complete (the caller's barrier) when this runs.
+// two 128-blocks and writes per-route rows. The C tile is complete (the caller's barrier) when this runs. sc = the scales of
+// the tile's columns (gate/up: svh of gate, of up, suh of down, 128 each; down: svh of 256), route = the output rows of its
+// positions (down).
 template <int MODE, int CS, bool YH, int NW = FT_WAVES, bool SUMS = false>
-__device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16_t* C, int rows, int pos0, int e,
-                                                  int nu, size_t grp, int wave, int lane)
+__device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16_t* C, int rows,
+                                                  int nu, size_t grp, int wave, int lane, const uint16_t* const (&sc)[3],
+                                                  const int32_t* route)
 {
     // Transforms in the layout of fwht128_lane8: per pass a wave takes 8 rows; lane (rpair, q, g) = (lane >> 4,
     // (lane >> 2) & 3, lane & 3) holds rows r0 + 2 rpair and r0 + 2 rpair + 1 (one dword of the transposed tile per
@@ -423,16 +428,13 @@ __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16
     if constexpr (MODE == 0)
     {
         const int c0 = nu * 128;
-        const uint16_t* svg = a.svh13 + ((size_t)e * 2 + 0) * a.I + c0;
-        const uint16_t* svu = a.svh13 + ((size_t)e * 2 + 1) * a.I + c0;
-        const uint16_t* sd = a.suh2 + (size_t)e * a.I + c0;
         float sgv[8], suv[8], sdv[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
         {
-            sgv[i] = h2f(svg[kk[i]]);
-            suv[i] = h2f(svu[kk[i]]);
-            sdv[i] = h2f(sd[kk[i]]);
+            sgv[i] = h2f(sc[0][kk[i]]);
+            suv[i] = h2f(sc[1][kk[i]]);
+            sdv[i] = h2f(sc[2][kk[i]]);
         }
         // the lane's 8 elements are chunk g of step c0 / 32 + q of its row's group
         uint16_t* od = a.xd + (size_t)(c0 / 32 + ((lane >> 2) & 3)) * GRP_HALVES + 256 * (lane & 3);
@@ -493,17 +495,14 @@ __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16
         float svv[2][8];
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb)
-        {
-            const uint16_t* sv = a.svh2 + (size_t)e * a.H + (2 * nu + hb) * 128;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) svv[hb][i] = h2f(sv[kk[i]]);
-        }
+            for (int i = 0; i < 8; ++i) svv[hb][i] = h2f(sc[hb][kk[i]]);
         for (int r0 = 8 * wave; r0 < rows; r0 += 8 * NW)
         {
             const int r = r0 + 2 * rpair;
             // output rows of the lane's two routes (a row past the tile's routes is not stored)
-            const int y0 = r < rows ? a.route_at[pos0 + r] : 0;
-            const int y1 = r + 1 < rows ? a.route_at[pos0 + r + 1] : 0;
+            const int y0 = r < rows ? route[r] : 0;
+            const int y1 = r + 1 < rows ? route[r + 1] : 0;
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb)
             {
@@ -540,6 +539,23 @@ __device__ __forceinline__ void fat_tile_epilogue(const FatArgs& a, const uint16
                 }
             }
         }
+    }
+}
+
+// The scales of column unit nu of expert e (fat_tile_epilogue).
+template <int MODE>
+__device__ __forceinline__ void fat_scales(const FatArgs& a, int e, int nu, const uint16_t* (&sc)[3])
+{
+    if constexpr (MODE == 0)
+    {
+        sc[0] = a.svh13 + ((size_t)e * 2 + 0) * a.I + nu * 128;
+        sc[1] = a.svh13 + ((size_t)e * 2 + 1) * a.I + nu * 128;
+        sc[2] = a.suh2 + (size_t)e * a.I + nu * 128;
+    }
+    else
+    {
+        sc[0] = sc[2] = a.svh2 + (size_t)e * a.H + nu * 256;
+        sc[1] = sc[0] + 128;
     }
 }
 
@@ -766,7 +782,9 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
             d[1] = (uint32_t)f2h(acc[i][j][2]) | ((uint32_t)f2h(acc[i][j][3]) << 16);
         }
     __syncthreads();
-    fat_tile_epilogue<MODE, CS, YH>(a, C, rows, pos0, e, nu, grp, wave, lane);
+    const uint16_t* sc[3];
+    fat_scales<MODE>(a, e, nu, sc);
+    fat_tile_epilogue<MODE, CS, YH>(a, C, rows, nu, grp, wave, lane, sc, a.route_at + pos0);
 }
 
 // Sixteen-wave form of the tile (four waves per SIMD, 64 accumulators per lane): MBW = row blocks per wave, BM =
@@ -962,20 +980,24 @@ __global__ __launch_bounds__(FT16_THREADS, 1) void k_fat16(FatArgs a)
             d[1] = (uint32_t)f2h(acc[i][j][2]) | ((uint32_t)f2h(acc[i][j][3]) << 16);
         }
     __syncthreads();
-    fat_tile_epilogue<MODE, CS, YH, NW>(a, C, rows, pos0, e, nu, grp, wave, lane);
+    const uint16_t* sc[3];
+    fat_scales<MODE>(a, e, nu, sc);
+    fat_tile_epilogue<MODE, CS, YH, NW>(a, C, rows, nu, grp, wave, lane, sc, a.route_at + pos0);
 }
 
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
-// k_mid's LDS: the four waves' rings (mid_depth steps of the trellis and the inputs), then, over them, the partial sums of
-// one row group, its C tile and the input sums (affine decode). One array: with a second one the compiler gives their accesses alias
+// k_mid's LDS: the four waves' rings (mid_depth steps of the trellis and the inputs) and, over them once they are done, the
+// partial sums of one row group and its C tile. One array: with a second one the compiler gives their accesses alias
 // scopes and then waits for every load to LDS (vmcnt 0) before each read.
 constexpr int mid_depth(int rb) { return rb == 3 ? 2 : 3; }
 constexpr int mid_slot(int rb) { return 2048 + rb * 2048; }
 constexpr int MID_C_AT = 2 * 32 * 128 * 4;
-constexpr int MID_XS_AT = MID_C_AT + FT_BN * (GRP_ROWS + 2) * 2;
-constexpr int MID_SMEM = std::max({ 4 * mid_depth(1) * mid_slot(1), 4 * mid_depth(2) * mid_slot(2),
-                                    4 * mid_depth(3) * mid_slot(3), MID_XS_AT + 2 * FT_MID * 4 });
+constexpr int MID_RINGS = std::max({ 4 * mid_depth(1) * mid_slot(1), 4 * mid_depth(2) * mid_slot(2),
+                                     4 * mid_depth(3) * mid_slot(3), MID_C_AT + FT_BN * (GRP_ROWS + 2) * 2 });
+// what the epilogue needs from memory, loaded while the rings fill: scales [3][128], output rows, input sums [2]
+constexpr int MID_SC_AT = MID_RINGS, MID_ROUTE_AT = MID_SC_AT + 3 * 256, MID_XS_AT = MID_ROUTE_AT + FT_MID * 4;
+constexpr int MID_SMEM = MID_XS_AT + 2 * FT_MID * 4;
 static_assert(2 * MID_SMEM <= 160 * 1024, "two workgroups (two waves per SIMD) share a CU's LDS");
 
 // Tiles of up to FT_MID = 96 routes x 256 output columns, for experts (and remainders of experts) with too few routes to
@@ -1081,6 +1103,25 @@ __device__ __forceinline__ void mid_tile(const FatArgs& a, uint8_t* smem, int ro
     const std::integral_constant<int, 1> h1;
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) load_step(j, j);
+    {
+        // (every thread's loads in one round trip with the rings')
+        const int tid = threadIdx.x;
+        const uint16_t* sc[3];
+        fat_scales<MODE>(a, e, nu, sc);
+        constexpr int NSC = MODE == 0 ? 3 : 2;
+        uint32_t scw = 0;
+        if (tid < NSC * 64) scw = reinterpret_cast<const uint32_t*>(tid < 64 ? sc[0] : tid < 128 ? sc[1] : sc[2])[tid & 63];
+        int32_t ro = 0;
+        if (MODE == 1 && tid < rows) ro = a.route_at[pos0 + tid];
+        float xsum = 0.0f;
+        const int xr = tid & 127, xm = tid >> 7;               // row, column block
+        if (!EXACT && xr < rows)
+            for (int b = 0; b < a.nxs; ++b)
+                xsum += a.xs[(((grp + (xr >> 5)) * a.nxs + b) * NA + (MODE == 0 ? xm : 0)) * GRP_ROWS + (xr & 31)];
+        if (tid < NSC * 64) reinterpret_cast<uint32_t*>(smem + MID_SC_AT)[tid] = scw;
+        if (MODE == 1 && tid < rows) reinterpret_cast<int32_t*>(smem + MID_ROUTE_AT)[tid] = ro;
+        if (!EXACT && xr < BM) reinterpret_cast<float*>(smem + MID_XS_AT)[xm * FT_MID + xr] = xsum * kbias_f();
+    }
     wait_vmcnt<(DEPTH - 1) * NL>();
     constexpr bool PIPE = RB < 3;
     if constexpr (PIPE) read_half(0, h0);
@@ -1107,16 +1148,10 @@ __device__ __forceinline__ void mid_tile(const FatArgs& a, uint8_t* smem, int ro
     __syncthreads();
     float4_t* red = reinterpret_cast<float4_t*>(smem) + sub * 1024 + lane;
     uint16_t* C = reinterpret_cast<uint16_t*>(smem + MID_C_AT);
-    float* xs_row = reinterpret_cast<float*>(smem + MID_XS_AT) + sub * BM;
-    if (!EXACT && kh == 0)
-        for (int r = lane; r < BM; r += 64)
-        {
-            float v = 0.0f;
-            if (r < rows)
-                for (int b = 0; b < a.nxs; ++b)
-                    v += a.xs[(((grp + (r >> 5)) * a.nxs + b) * NA + (MODE == 0 ? sub : 0)) * GRP_ROWS + (r & 31)];
-            xs_row[r] = v * kbias_f();
-        }
+    const float* xs_row = reinterpret_cast<const float*>(smem + MID_XS_AT) + sub * FT_MID;
+    const uint16_t* sc0 = reinterpret_cast<const uint16_t*>(smem + MID_SC_AT);
+    const uint16_t* const sc[3] = { sc0, sc0 + 128, sc0 + 256 };
+    const int32_t* route = reinterpret_cast<const int32_t*>(smem + MID_ROUTE_AT);
     // one row group at a time: the second half's sums through LDS, then the C tile (lane (column lane & 31, h) of a 32 x
     // 32 block holds rows 8 (v >> 2) + 4 h + (v & 3); the affine decode's sums become KINV S + KBIAS (sum of the row's
     // inputs)), then the epilogue, 8 rows per wave
@@ -1155,8 +1190,8 @@ __device__ __forceinline__ void mid_tile(const FatArgs& a, uint8_t* smem, int ro
                 }
             }
         __syncthreads();
-        fat_tile_epilogue<MODE, CS, YH, 4, !EXACT>(a, C, min(rows - r * GRP_ROWS, GRP_ROWS), pos0 + r * GRP_ROWS, e, nu,
-                                                   grp + r, wave, lane);
+        fat_tile_epilogue<MODE, CS, YH, 4, !EXACT>(a, C, min(rows - r * GRP_ROWS, GRP_ROWS), nu, grp + r, wave, lane, sc,
+                                                   route + r * GRP_ROWS);
     }
 }
 

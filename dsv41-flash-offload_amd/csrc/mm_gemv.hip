@@ -102,11 +102,12 @@ __device__ __forceinline__ float load_x_t(const void* x, size_t i)
     return static_cast<const float*>(x)[i];
 }
 
-template <int XD>
+template <int XD, bool SPLIT>
 __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
 {
-    // in-kernel routing (E <= 1024): each expert's routes, or (one record per expert) a bitmap of the experts present
-    __shared__ __align__(16) int s_hist[GV_ROUTE_MAX];
+    // in-kernel routing (E <= 1024): each expert's routes (SPLIT: records of REC_ROUTES routes), or a bitmap of the experts
+    // present (one record per expert)
+    __shared__ __align__(16) int s_hist[SPLIT ? 1024 : 32];
     __shared__ int s_cnt[4][4];
     __shared__ float s_ss[4];
     __shared__ int s_ai;
@@ -114,7 +115,6 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     const int blk = blockIdx.x % a.nb, m = (blockIdx.x / a.nb) & 1, idx = blockIdx.x / (2 * a.nb);
     const bool writer = m == 0 && blk == 0;      // the one workgroup of a route that writes its routing data
     const bool perm = a.offsets != nullptr;
-    const bool split = !perm && a.n > REC_ROUTES * a.topk;   // more than REC_ROUTES tokens: records of REC_ROUTES routes
     // routing from the permutation: the workgroups of index idx own sorted position idx
     const int nvalid_perm = perm ? a.offsets[a.E] : 0;
     const int s = perm ? a.order[idx] : idx;
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
             ss = fmaf(v, v, ss);
         }
     }
-    if (split)
+    if constexpr (SPLIT)
         *reinterpret_cast<int4*>(&s_hist[4 * tid]) = make_int4(0, 0, 0, 0);
     else if (tid < 32)
         s_hist[tid] = 0;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
         const int64_t v = rid[k];
         const int i = tid + 256 * k;
         if (perm || i >= a.n || v < 0 || v >= a.E) continue;
-        if (split) atomicAdd(&s_hist[v], 1);
+        if constexpr (SPLIT) atomicAdd(&s_hist[v], 1);
         else atomicOr(&s_hist[v >> 5], 1 << (v & 31));
         nv += 1;
         less += v < e;
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     int below = 0, present = 0;
     if (!perm && wave == 0 && (writer || blockIdx.x == 0))
     {
-        if (split)
+        if constexpr (SPLIT)
         {
 #pragma unroll
             for (int k = 0; k < 4; ++k)
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
         {
             // the route's record: an expert's come after those of the experts below it, one per REC_ROUTES routes or one in
             // all; with a permutation it has one, at its place in the active list (-1 if absent there)
-            const int ai = !valid ? -1 : (perm ? s_ai : below + (split ? rank / REC_ROUTES : 0));
+            const int ai = !valid ? -1 : (perm ? s_ai : below + (SPLIT ? rank / REC_ROUTES : 0));
             a.pos_of[s] = valid && !fat ? pos : -1;
             a.ai_of[s] = valid && !fat ? ai : -1;
             if (valid)
@@ -266,10 +266,10 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
                 a.e_at[pos] = fat ? -1 : e;
                 a.ai_at[pos] = fat ? -1 : ai;
                 // the record's first route writes it
-                const bool first_route = perm ? pos == a.offsets[e] : (split ? rank % REC_ROUTES : rank) == 0;
+                const bool first_route = perm ? pos == a.offsets[e] : (SPLIT ? rank % REC_ROUTES : rank) == 0;
                 if (first_route && ai >= 0)
                 {
-                    const int cnt = perm ? a.offsets[e + 1] - pos : split ? min(same - rank, REC_ROUTES) : same;
+                    const int cnt = perm ? a.offsets[e + 1] - pos : SPLIT ? min(same - rank, REC_ROUTES) : same;
                     ExpertRec r{ e, fat ? 0 : cnt, pos, 0, { wt0, wt1, wt2 }, 0 };
                     a.rec[ai] = r;
                 }
@@ -811,15 +811,25 @@ struct Ws
 
 int prep_blocks(int H) { return (H + PREP_ROWS - 1) / PREP_ROWS; }
 
-void launch_route_prep(const PrepArgs& p, hipStream_t s)
+template <int XD>
+static void launch_route_prep_t(const PrepArgs& p, hipStream_t s)
 {
     const dim3 grid(2 * p.npos * p.nb), block(256);
-    if (p.x_dtype == MM_DTYPE_F16)
-        hipLaunchKernelGGL(k_route_prep<MM_DTYPE_F16>, grid, block, 0, s, p);
-    else if (p.x_dtype == MM_DTYPE_BF16)
-        hipLaunchKernelGGL(k_route_prep<MM_DTYPE_BF16>, grid, block, 0, s, p);
+    // more than REC_ROUTES tokens, routed in-kernel: records of REC_ROUTES routes
+    if (!p.offsets && p.n > REC_ROUTES * p.topk)
+        hipLaunchKernelGGL((k_route_prep<XD, true>), grid, block, 0, s, p);
     else
-        hipLaunchKernelGGL(k_route_prep<MM_DTYPE_F32>, grid, block, 0, s, p);
+        hipLaunchKernelGGL((k_route_prep<XD, false>), grid, block, 0, s, p);
+}
+
+void launch_route_prep(const PrepArgs& p, hipStream_t s)
+{
+    if (p.x_dtype == MM_DTYPE_F16)
+        launch_route_prep_t<MM_DTYPE_F16>(p, s);
+    else if (p.x_dtype == MM_DTYPE_BF16)
+        launch_route_prep_t<MM_DTYPE_BF16>(p, s);
+    else
+        launch_route_prep_t<MM_DTYPE_F32>(p, s);
 }
 
 // Most pieces per segment a partial launch may use: bounded so the partial sums stay a few MB.
