@@ -40,7 +40,7 @@ constexpr int FT_BIG_MIN = 193;     // smallest remainder of c / 256 that takes 
 //     where FT_MID-route tiles took 60; at 64 tiles (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at
 //     297 (16,384 tokens) 8.25 and 8.65.
 //   the other entry points, whose rows must have the same bits whichever other experts a call computes (a layer in one call
-//     or in staging batches): by the expert's own routes, from four such tiles on. Staging batches hold few experts: 12
+//     or in staging batches): by the expert's own routes, from three such tiles on. Staging batches hold few experts: 12
 //     tiles of a batch of 16 experts took 189 us of its 470, as FT_MID-route tiles 50.
 struct BigRule
 {
@@ -48,7 +48,7 @@ struct BigRule
     int min_rows;       // of the expert
 };
 constexpr int FT_BIG_WORK = 3 * 256;
-constexpr int FT_BIG_ROWS = 1024;
+constexpr int FT_BIG_ROWS = 3 * FT_BIG;
 constexpr int GRP_ROWS = 32;        // rows of a row group
 constexpr int GRP_HALVES = 1024;    // one matrix's 32-element step of a row group
 // 128-blocks per input transform workgroup (16,384 tokens, H 4096, 2.3 GB written: 783 us with 2, 844 with 4, 946 with 8;
