@@ -109,10 +109,12 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     // present (one record per expert)
     __shared__ __align__(16) int s_hist[SPLIT ? 1024 : 32];
     __shared__ int s_cnt[4][4];
-    __shared__ float s_ss[4];
+    __shared__ float s_ss[4], s_bs[2][4];
     __shared__ int s_ai;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int blk = blockIdx.x % a.nb, m = (blockIdx.x / a.nb) & 1, idx = blockIdx.x / (2 * a.nb);
+    // SPLIT: one workgroup per (route, matrix) walks the row's blocks (the routing is found once per row, not per block)
+    const int nbk = SPLIT ? 1 : a.nb;
+    const int blk = blockIdx.x % nbk, m = (blockIdx.x / nbk) & 1, idx = blockIdx.x / (2 * nbk);
     const bool writer = m == 0 && blk == 0;      // the one workgroup of a route that writes its routing data
     const bool perm = a.offsets != nullptr;
     // routing from the permutation: the workgroups of index idx own sorted position idx
@@ -286,24 +288,46 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
         const float tot = (s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3]);
         scale = tot > 0.0f ? 1.0f / sqrtf(tot / (float)a.H) : 1.0f;
     }
-    __syncthreads();      // s_ss is reused below
-    float bsum = 0.0f;
-    if (h0 < a.H)
+    uint16_t* dst = a.xa + ((size_t)pos * 2 + m) * a.H;
+    float* xsum = a.xsum + ((size_t)pos * 2 + m) * a.nb;
+    float wa = va, wb = vb, ra = sa, rb = sb;
+    for (int b = blk;; ++b)
     {
-        if (!(XD == MM_DTYPE_F16 && !a.rescale))
+        const int hb = b * PREP_ROWS + wave * 128;
+        const bool more = SPLIT && b + 1 < a.nb;
+        float na = 0.f, nb = 0.f, pa = 0.f, pb = 0.f;
+        if (more)
         {
-            va = r16(bf16_value(va * scale));
-            vb = r16(bf16_value(vb * scale));
+            // the next block, in flight during this one
+            const int hn = hb + PREP_ROWS < a.H ? hb + PREP_ROWS : 0;
+            na = load_x_t<XD>(a.x, row + hn + lane);
+            nb = load_x_t<XD>(a.x, row + hn + lane + 64);
+            pa = h2f(su[hn + lane]);
+            pb = h2f(su[hn + lane + 64]);
         }
-        prep_block_wave(va, vb, sa, sb);
-        uint16_t* dst = a.xa + ((size_t)pos * 2 + m) * a.H;
-        dst[operand_index(h0 + lane)] = f2h(va);
-        dst[operand_index(h0 + lane + 64)] = f2h(vb);
-        bsum = wave_sum(va + vb);
+        float bsum = 0.0f;
+        if (hb < a.H)
+        {
+            if (!(XD == MM_DTYPE_F16 && !a.rescale))
+            {
+                wa = r16(bf16_value(wa * scale));
+                wb = r16(bf16_value(wb * scale));
+            }
+            prep_block_wave(wa, wb, ra, rb);
+            dst[operand_index(hb + lane)] = f2h(wa);
+            dst[operand_index(hb + lane + 64)] = f2h(wb);
+            bsum = wave_sum(wa + wb);
+        }
+        float(&bs)[4] = s_bs[b & 1];      // two in turn: a block's sums are read before the block after the next writes
+        if (lane == 0) bs[wave] = bsum;
+        __syncthreads();
+        if (tid == 0) xsum[b] = (bs[0] + bs[1]) + (bs[2] + bs[3]);
+        if (!more) break;
+        wa = na;
+        wb = nb;
+        ra = pa;
+        rb = pb;
     }
-    if (lane == 0) s_ss[wave] = bsum;
-    __syncthreads();
-    if (tid == 0) a.xsum[((size_t)pos * 2 + m) * a.nb + blk] = (s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3]);
 }
 
 // ------------------------------------------------------------------------------------ 2/4. partial sums
@@ -814,12 +838,14 @@ int prep_blocks(int H) { return (H + PREP_ROWS - 1) / PREP_ROWS; }
 template <int XD>
 static void launch_route_prep_t(const PrepArgs& p, hipStream_t s)
 {
-    const dim3 grid(2 * p.npos * p.nb), block(256);
-    // more than REC_ROUTES tokens, routed in-kernel: records of REC_ROUTES routes
+    // more than REC_ROUTES tokens, routed in-kernel: records of REC_ROUTES routes, and one workgroup per route and matrix
+    // instead of one per 512 rows, each of which found the routing again (100 tokens, top-8: 39 us of a 790 us call; with
+    // this the call 962 -> 689 us where it went 925 -> 699 before; 24 tokens 1.21 x where it was 1.18). Fewer tokens have too
+    // few rows to fill the GPU with.
     if (!p.offsets && p.n > REC_ROUTES * p.topk)
-        hipLaunchKernelGGL((k_route_prep<XD, true>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((k_route_prep<XD, true>), dim3(2 * p.npos), dim3(256), 0, s, p);
     else
-        hipLaunchKernelGGL((k_route_prep<XD, false>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((k_route_prep<XD, false>), dim3(2 * p.npos * p.nb), dim3(256), 0, s, p);
 }
 
 void launch_route_prep(const PrepArgs& p, hipStream_t s)
