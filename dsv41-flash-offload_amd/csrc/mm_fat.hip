@@ -565,7 +565,8 @@ __device__ __forceinline__ void fat_scales(const FatArgs& a, int e, int nu, cons
 // (0.7 % off the 16k layer against contiguous halves); every wave loads an
 // eighth of the inputs and waves 0 .. 3 also the trellis (chunk w: tile row w >> 1 of matrix / block w & 1),
 // which runs further ahead; wave w decodes column tiles 2 (w & 3), 2 (w & 3) + 1 of sub-block w >> 2 in both tile
-// rows (chunks w >> 2 and 2 + (w >> 2)). Rows past the tile's routes read zero inputs.
+// rows (chunks w >> 2 and 2 + (w >> 2)). Rows past the tile's routes multiply what their row group holds (zeros past the
+// last group) and are not stored.
 template <int MODE, int MB, bool YH = false>
 __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
 {
