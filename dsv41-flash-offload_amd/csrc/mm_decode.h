@@ -111,6 +111,7 @@ struct PrepArgs
     float* xsum;              // [n][2][nb] sums of xa over each workgroup's rows
     int n, topk, E, H, nb, x_dtype, rescale;
     int cap;                  // experts with more than cap routes are left out (no record work, no outputs)
+    int walk;                 // records of 16 routes: one workgroup per route and matrix
     int npos;                 // sorted positions visited (n with in-kernel routing; the permutation's valid
                               // positions must lie below it)
 };

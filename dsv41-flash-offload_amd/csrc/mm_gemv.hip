@@ -34,7 +34,7 @@ constexpr int GV_WAVES = 4;
 constexpr int GV_THREADS = 64 * GV_WAVES;
 constexpr int GV_COLS = 128;          // output columns per segment (8 tiles)
 constexpr int GV_ROUTE_MAX = 1024;    // in-kernel routing limit (routes per call)
-// Routes per record (one pass of a partial-sum wave) with in-kernel routing of more than this many tokens. A segment costs
+// Routes per record (one pass of a partial-sum wave) in calls of more than this many tokens. A segment costs
 // its waves one pass over its rows, whatever its routes, so equal runs of rows are equal work: with one record per expert
 // the waves of an expert with more than 16 routes took twice as long as the others and the launch waited for them (24
 // tokens, top-8 and the shared expert: 357 -> 304 us a call; 100 tokens on the decode path alone 741 us, against 884 with its
@@ -46,6 +46,7 @@ static_assert(GV_RING % 2 == 0, "row pairs");
 constexpr int ROW_BYTES = 8 * 96;     // one tile row of a segment
 constexpr int WAVES_PER_CU = 24;      // partial kernels: 6 workgroups of 4 waves per CU (<= 80 VGPRs, 16 KB LDS)
 constexpr int PREP_ROWS = 512;        // input rows per route-prep workgroup
+constexpr int PREP_WALK_MIN = 384;    // routes from which a permutation's route prep walks the input rows
 constexpr int SS_LOADS = 16;          // route prep: row elements per thread loaded at once for the rescale
 constexpr int MAX_TOPK = 16;
 
@@ -106,17 +107,17 @@ template <int XD, bool SPLIT>
 __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
 {
     // in-kernel routing (E <= 1024): each expert's routes (SPLIT: records of REC_ROUTES routes), or a bitmap of the experts
-    // present (one record per expert)
+    // present (one record per expert); with a permutation the active experts' routes come from its offsets
     __shared__ __align__(16) int s_hist[SPLIT ? 1024 : 32];
     __shared__ int s_cnt[4][4];
     __shared__ float s_ss[4], s_bs[2][4];
     __shared__ int s_ai;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // SPLIT: one workgroup per (route, matrix) walks the row's blocks (the routing is found once per row, not per block)
-    const int nbk = SPLIT ? 1 : a.nb;
+    // walk: one workgroup per (route, matrix) takes the row's blocks one after another, instead of one each
+    const bool perm = a.offsets != nullptr, walk = SPLIT && a.walk;
+    const int nbk = walk ? 1 : a.nb;
     const int blk = blockIdx.x % nbk, m = (blockIdx.x / nbk) & 1, idx = blockIdx.x / (2 * nbk);
     const bool writer = m == 0 && blk == 0;      // the one workgroup of a route that writes its routing data
-    const bool perm = a.offsets != nullptr;
     // routing from the permutation: the workgroups of index idx own sorted position idx
     const int nvalid_perm = perm ? a.offsets[a.E] : 0;
     const int s = perm ? a.order[idx] : idx;
@@ -177,11 +178,21 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
         s_hist[tid] = 0;
     if (tid == 0) s_ai = -1;
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (tid + 256 * k < nact_perm && act[k] == e) s_ai = tid + 256 * k;     // one match at most
     // in-kernel routing: position = routes of lower experts + earlier routes of the same expert
     int less = 0, same = 0, rank = 0, nv = 0;
+    // with a permutation: the records of the active experts before the route's expert (less) and of all (nv)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        if (tid + 256 * k >= nact_perm) continue;
+        if (act[k] == e) s_ai = tid + 256 * k;     // one match at most
+        if constexpr (SPLIT)
+        {
+            const int nr = (a.offsets[act[k] + 1] - a.offsets[act[k]] + REC_ROUTES - 1) / REC_ROUTES;
+            nv += nr;
+            less += act[k] < e ? nr : 0;
+        }
+    }
 #pragma unroll
     for (int k = 0; k < GV_ROUTE_MAX / 256; ++k)
     {
@@ -214,9 +225,14 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     rank = s_cnt[0][2] + s_cnt[1][2] + s_cnt[2][2] + s_cnt[3][2];
     nv = s_cnt[0][3] + s_cnt[1][3] + s_cnt[2][3] + s_cnt[3][3];
     const int pos = perm ? idx : less + rank;
+    if (perm)
+    {
+        same = pcnt;
+        rank = idx - a.offsets[ec];
+    }
     // an expert with more than cap routes belongs to the fat-expert path: its positions stay reserved, but it gets
     // an empty record and its routes no transformed inputs and no outputs
-    const bool fat = valid && (perm ? pcnt : same) > a.cap;
+    const bool fat = valid && same > a.cap;
     // in-kernel routing: the records of the experts below the route's expert and of all, by one reduction over the first
     // wave (records of REC_ROUTES routes: lane l takes experts 16 l .. 16 l + 15)
     int below = 0, present = 0;
@@ -252,14 +268,15 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     {
         if (blockIdx.x == 0)
         {
-            a.counts[0] = perm ? a.nactive_in[0] : present;
+            a.counts[0] = !perm ? present : SPLIT ? nv : nact_perm;
             a.counts[1] = perm ? nvalid_perm : nv;
         }
         if (writer)
         {
             // the route's record: an expert's come after those of the experts below it, one per REC_ROUTES routes or one in
-            // all; with a permutation it has one, at its place in the active list (-1 if absent there)
-            const int ai = !valid ? -1 : (perm ? s_ai : below + (SPLIT ? rank / REC_ROUTES : 0));
+            // all; with a permutation an expert that is not in the active list has none
+            const int first_ai = !perm ? below : s_ai < 0 ? -1 : SPLIT ? less : s_ai;
+            const int ai = !valid || first_ai < 0 ? -1 : first_ai + (SPLIT ? rank / REC_ROUTES : 0);
             a.pos_of[s] = valid && !fat ? pos : -1;
             a.ai_of[s] = valid && !fat ? ai : -1;
             if (valid)
@@ -268,10 +285,10 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
                 a.e_at[pos] = fat ? -1 : e;
                 a.ai_at[pos] = fat ? -1 : ai;
                 // the record's first route writes it
-                const bool first_route = perm ? pos == a.offsets[e] : (SPLIT ? rank % REC_ROUTES : rank) == 0;
+                const bool first_route = (SPLIT ? rank % REC_ROUTES : rank) == 0;
                 if (first_route && ai >= 0)
                 {
-                    const int cnt = perm ? a.offsets[e + 1] - pos : SPLIT ? min(same - rank, REC_ROUTES) : same;
+                    const int cnt = SPLIT ? min(same - rank, REC_ROUTES) : same;
                     ExpertRec r{ e, fat ? 0 : cnt, pos, 0, { wt0, wt1, wt2 }, 0 };
                     a.rec[ai] = r;
                 }
@@ -294,7 +311,7 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     for (int b = blk;; ++b)
     {
         const int hb = b * PREP_ROWS + wave * 128;
-        const bool more = SPLIT && b + 1 < a.nb;
+        const bool more = walk && b + 1 < a.nb;
         float na = 0.f, nb = 0.f, pa = 0.f, pb = 0.f;
         if (more)
         {
@@ -838,12 +855,9 @@ int prep_blocks(int H) { return (H + PREP_ROWS - 1) / PREP_ROWS; }
 template <int XD>
 static void launch_route_prep_t(const PrepArgs& p, hipStream_t s)
 {
-    // more than REC_ROUTES tokens, routed in-kernel: records of REC_ROUTES routes, and one workgroup per route and matrix
-    // instead of one per 512 rows, each of which found the routing again (100 tokens, top-8: 39 us of a 790 us call; with
-    // this the call 962 -> 689 us where it went 925 -> 699 before; 24 tokens 1.21 x where it was 1.18). Fewer tokens have too
-    // few rows to fill the GPU with.
-    if (!p.offsets && p.n > REC_ROUTES * p.topk)
-        hipLaunchKernelGGL((k_route_prep<XD, true>), dim3(2 * p.npos), dim3(256), 0, s, p);
+    // more than REC_ROUTES tokens: records of REC_ROUTES routes, the same ones from a permutation as from the ids
+    if (p.n > REC_ROUTES * p.topk)
+        hipLaunchKernelGGL((k_route_prep<XD, true>), dim3(2 * p.npos * (p.walk ? 1 : p.nb)), dim3(256), 0, s, p);
     else
         hipLaunchKernelGGL((k_route_prep<XD, false>), dim3(2 * p.npos * p.nb), dim3(256), 0, s, p);
 }
@@ -966,9 +980,13 @@ static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_d
                         const int32_t* active, const int32_t* nactive, int cap, hipStream_t s)
 {
     const int nb = prep_blocks(L->H);
+    // With records of REC_ROUTES routes and routing in-kernel, one workgroup per route and matrix walks the row: one per 512
+    // rows found the routing again each (100 tokens, top-8: 39 us of a 790 us call). With a permutation it pays from three
+    // workgroups per CU on (a layer of 24 tokens, H 5120, 335 us walking and 331 not, 200 tokens 1,144 and 1,161).
+    const bool walk = n > REC_ROUTES * topk && (!offsets || n >= PREP_WALK_MIN);
     PrepArgs p{ x, ids, offsets, order, active, nactive, L->gate_ptr, L->up_ptr, L->down_ptr, L->suh13,
                 w.rec, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, w.xa, w.xsum, n, topk, L->E, L->H, nb,
-                x_dtype, rescale, cap, npos };
+                x_dtype, rescale, cap, walk ? 1 : 0, npos };
     launch_route_prep(p, s);
 }
 

@@ -397,3 +397,42 @@ def test_decode_layer_with_experts_of_many_routes(dev, exact):
     ref = OracleLayer(st, seed).forward(x16.astype(np.float32), ids, w)
     ok, m = within_tolerance(out.cpu().numpy(), ref)
     assert ok, m
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("T,max_rows", [(16, None), (17, None), (40, None), (40, 16), (300, 70)])
+def test_permutation_and_in_kernel_routing_agree_bitwise(dev, T, max_rows, exact):
+    """Up to 16 tokens (one record per expert) and above (one per 16 routes), with and without a cap on an expert's
+    routes, tokens that pick an expert twice and masked routes: the layer with its routes found in-kernel, taken from a
+    permutation, and run as one call is the same bit for bit (a route's products are summed over the same pieces); with
+    fp16-rounded weights, which the oracle has too, it matches the oracle."""
+    import torch
+    from mi355moe import moe
+    H, I, E, k, seed = 512, 256, 24, 3, 5150
+    shared = T < 300                                    # 300 tokens: 900 routes without it (1,024 at most in-kernel)
+    st = make_store(E + shared, H, I, seed, device=dev, exact=exact)
+    rng = np.random.default_rng(T)
+    p = 1.0 / np.arange(1, E + 1)
+    ids = rng.choice(E, (T, k), p=p / p.sum()).astype(np.int64)
+    ids[::7, 1] = -1
+    w = rng.uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    R = moe.DecodeRunner(E, H, I, T, k, device=dev, max_rows=max_rows, shared=shared)
+    R.set_routes(_t(ids, dev), _t(w, dev))
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    R.x16.copy_(_t(x16, dev))
+    print(f"permutation against in-kernel routing T={T} max_rows={max_rows} exact={exact}", flush=True)
+    a = R.run(st).clone()
+    b = R.run(st, use_permutation=True).clone()
+    c = R.layer(st).clone()
+    torch.cuda.synchronize()
+    assert torch.equal(a, b) and torch.equal(a, c)
+    flat = R.ids.cpu().numpy()
+    counts = np.bincount(flat[flat >= 0], minlength=st.E)
+    kept = (flat >= 0) & (counts[np.maximum(flat, 0)] <= R.max_rows)
+    if max_rows:
+        assert kept.any() and not kept[flat >= 0].all()
+    if not exact:
+        return
+    ref = OracleLayer(st, seed).forward(x16.astype(np.float32), np.where(kept, flat, -1), R.w.cpu().numpy())
+    ok, m = within_tolerance(a.cpu().numpy(), ref)
+    assert ok, m
