@@ -111,7 +111,8 @@ struct PrepArgs
     float* xsum;              // [n][2][nb] sums of xa over each workgroup's rows
     int n, topk, E, H, nb, x_dtype, rescale;
     int cap;                  // experts with more than cap routes are left out (no record work, no outputs)
-    int walk;                 // records of 16 routes: one workgroup per route and matrix
+    int split;                // records of 16 routes instead of one per expert
+    int walk;                 // with split: one workgroup per route and matrix takes all its input rows
     int npos;                 // sorted positions visited (n with in-kernel routing; the permutation's valid
                               // positions must lie below it)
 };

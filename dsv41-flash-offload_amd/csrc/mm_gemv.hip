@@ -26,6 +26,8 @@
 // per-weight rounding is spent. With MM_LAYER_EXACT every weight is rounded to fp16 first (v_pk_fma_f16), the
 // reference's EXACT expert (ft_core.h:977-1011). fp16 activations, fp32 accumulation, fp16 rounding at the
 // reference's points in both.
+#include <algorithm>
+
 #include "mm_decode.h"
 
 namespace mm {
@@ -855,8 +857,7 @@ int prep_blocks(int H) { return (H + PREP_ROWS - 1) / PREP_ROWS; }
 template <int XD>
 static void launch_route_prep_t(const PrepArgs& p, hipStream_t s)
 {
-    // more than REC_ROUTES tokens: records of REC_ROUTES routes, the same ones from a permutation as from the ids
-    if (p.n > REC_ROUTES * p.topk)
+    if (p.split)
         hipLaunchKernelGGL((k_route_prep<XD, true>), dim3(2 * p.npos * (p.walk ? 1 : p.nb)), dim3(256), 0, s, p);
     else
         hipLaunchKernelGGL((k_route_prep<XD, false>), dim3(2 * p.npos * p.nb), dim3(256), 0, s, p);
@@ -879,8 +880,16 @@ static int piece_cap(int n)
     return c > 32 ? 32 : (c < 4 ? 4 : c);
 }
 
-// Most records of n routes over E experts.
-static int max_records(int n, int E) { return (n < E ? n : E) + n / REC_ROUTES; }
+// Most records of n routes over E experts: a route each, or one per expert and one per further REC_ROUTES routes.
+static int max_records(int n, int E) { return std::min(n, std::min(n, E) + n / REC_ROUTES); }
+// tile rows of a partial launch (records x 2 matrices x column blocks x tile rows) count in int
+static bool rows_fit(const mm_layer_t* L, int records) { return (size_t)records * L->H / 1024 * L->I < ((size_t)1 << 31); }
+// Records of REC_ROUTES routes (the same ones from a permutation as from the ids) above REC_ROUTES tokens, one per expert
+// below and where more would leave int.
+static bool split_records(const mm_layer_t* L, int n, int topk)
+{
+    return n > REC_ROUTES * topk && rows_fit(L, max_records(n, L->E));
+}
 
 // Workspace of n routes whose sorted positions lie below npos (npos = n unless a caller bounds the positions).
 static Ws carve(void* base, int n, int npos, int E, int H, int I)
@@ -964,8 +973,7 @@ static int check_common(const mm_layer_t* L, const void* x, int x_dtype, int T, 
                  "%s: x_dtype must be MM_DTYPE_F16, MM_DTYPE_BF16 or MM_DTYPE_F32", who);
     MM_CHECK_ARG(T > 0 && n > 0 && topk > 0 && n <= T * topk, "%s: bad T/n/topk", who);
     MM_CHECK_ARG((size_t)n * 2 * (L->H > L->I ? L->H : L->I) * 2 < ((size_t)1 << 31), "%s: too many routes", who);
-    // tile rows of a partial launch (active experts x 2 matrices x column blocks x tile rows) count in int
-    MM_CHECK_ARG((size_t)max_records(n, L->E) * L->H / 1024 * L->I < ((size_t)1 << 31), "%s: too many routes", who);
+    MM_CHECK_ARG(rows_fit(L, std::min(n, L->E)), "%s: too many routes", who);
     MM_CHECK_ARG(max_rows > 0, "%s: max_rows must be at least 1", who);
     const bool perm = offsets != nullptr;
     MM_CHECK_ARG(perm ? (order && active && nactive) : n <= GV_ROUTE_MAX,
@@ -983,10 +991,10 @@ static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_d
     // With records of REC_ROUTES routes and routing in-kernel, one workgroup per route and matrix walks the row: one per 512
     // rows found the routing again each (100 tokens, top-8: 39 us of a 790 us call). With a permutation it pays from three
     // workgroups per CU on (a layer of 24 tokens, H 5120, 335 us walking and 331 not, 200 tokens 1,144 and 1,161).
-    const bool walk = n > REC_ROUTES * topk && (!offsets || n >= PREP_WALK_MIN);
+    const bool split = split_records(L, n, topk), walk = split && (!offsets || n >= PREP_WALK_MIN);
     PrepArgs p{ x, ids, offsets, order, active, nactive, L->gate_ptr, L->up_ptr, L->down_ptr, L->suh13,
                 w.rec, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, w.xa, w.xsum, n, topk, L->E, L->H, nb,
-                x_dtype, rescale, cap, walk ? 1 : 0, npos };
+                x_dtype, rescale, cap, split ? 1 : 0, walk ? 1 : 0, npos };
     launch_route_prep(p, s);
 }
 

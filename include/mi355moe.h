@@ -162,8 +162,8 @@ int mm_moe_decode(const mm_layer_t* layer, const void* x, int x_dtype, int resca
                   mm_stream_t stream);
 
 /* Bytes of the library's device scratch array behind mm_moe_decode_noalloc (one array per device, held from the
- * library's load until the process ends). */
-#define MM_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
+ * library's load until the process ends): 64 MiB, and 48 bytes for each 16 of 1,024 routes (their records). */
+#define MM_NOALLOC_SCRATCH_BYTES (((size_t)64 << 20) + 3072)
 
 /* mm_moe_decode without a workspace argument. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).

@@ -53,6 +53,36 @@ def test_argument_errors_without_device_work():
     assert L.mm_gemv_workspace(0, 385, 4096, 2048) == 0
 
 
+@pytest.mark.parametrize("H,I", [(1024, 512), (4096, 2048), (5120, 2304)])
+def test_scratch_holds_every_call_of_64_mib_with_one_record_per_expert(H, I):
+    """mm_moe_decode_noalloc takes every call (up to 1,024 routes) whose decode arrays, with one 48-byte record per active
+    expert, fill at most 64 MiB: the records of 16 routes of larger calls come on top of that."""
+    from mi355moe import _lib
+    L = _lib.load()
+    scratch = eval(re.search(r"#define MM_NOALLOC_SCRATCH_BYTES (.*)", open(HDR).read()).group(1).replace("(size_t)", ""))
+    al = lambda v: (v + 255) & ~255
+    for E in (8, 128, 384, 1024):
+        for n in range(1, 1025):
+            cap, nb = min(32, max(4, 8192 // n)), (H + 511) // 512
+            one = (al(min(n, E) * 48) + al(8) + 5 * al(n * 4) + al(n * 2 * H * 2) + al(n * 2 * nb * 4)
+                   + al(cap * n * 2 * I * 4) + al(n * I * 2) + al(n * (I // 128) * 4) + al(cap * n * H * 4))
+            need = L.mm_gemv_workspace(n, E, H, I)
+            assert one <= need <= one + al(n // 16 * 48), (E, n)
+            if one <= 64 << 20:
+                assert need <= scratch, (E, n)
+
+
+def test_route_limit_counts_one_record_per_expert():
+    """The limit on a partial launch's tile rows holds for one record per expert: 8,000 routes over 16 experts of 65,536 x
+    65,536 pass it (records of 16 routes would not) and fail on the workspace, argument checks only."""
+    import ctypes
+    from mi355moe import _lib
+    L = _lib.load()
+    lay = _lib.MMLayer(*([256] * 7), 16, 65536, 65536, 10.0, 0)
+    rc = L.mm_expert_gemv(ctypes.byref(lay), 256, 0, 0, 4000, 8000, 2, 256, 256, 256, 256, 256, 8000, 256, None, 0, 31, None)
+    assert rc == -1 and b"workspace too small" in L.mm_last_error(), L.mm_last_error()
+
+
 def test_expert_seed_matches_oracle():
     import oracle as O
     from mi355moe import _lib
