@@ -96,6 +96,7 @@ struct PrepArgs
     const int32_t* order;
     const int32_t* active;
     const int32_t* nactive_in;
+    const int32_t* nvalid_in; // routed positions of the permutation: offsets + E, or where fewer are to be computed
     const int64_t* wtab0;     // gate, up, down pointer tables
     const int64_t* wtab1;
     const int64_t* wtab2;
@@ -113,6 +114,7 @@ struct PrepArgs
     int cap;                  // experts with more than cap routes are left out (no record work, no outputs)
     int split;                // records of 16 routes instead of one per expert
     int walk;                 // with split: one workgroup per route and matrix takes all its input rows
+    int gated;                // no routed position: only counts are written (0, 0)
     int npos;                 // sorted positions visited (n with in-kernel routing; the permutation's valid
                               // positions must lie below it)
 };
@@ -133,9 +135,18 @@ __device__ __forceinline__ int wave_sum_int(int v)
 int prep_blocks(int H);
 void launch_route_prep(const PrepArgs& p, hipStream_t s);
 
-// The launches of mm_moe_decode on a given workspace (argument checks included); `who` names the caller in errors.
+constexpr int GV_ROUTE_MAX = 1024;    // in-kernel routing limit of the decode path (routes per call)
+
+// Whether the decode path can address n routes over E experts.
+bool decode_fits(int n, int E, int H, int I);
+
+// The launches of mm_moe_decode on a given workspace (argument checks included); `who` names the caller in errors. Calls of
+// more than GV_ROUTE_MAX routes pass mm_permute's offsets, order and active of them, nactive and nvalid (as offsets + E): with
+// 0 on the device in both nothing is computed and out is left as it is.
 int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int rescale, int T, int topk, const int64_t* ids,
                       const float* w, int max_rows, float* out, void* workspace, size_t workspace_bytes,
-                      mm_stream_t stream, const char* who);
+                      mm_stream_t stream, const char* who, const int32_t* offsets = nullptr, const int32_t* order = nullptr,
+                      const int32_t* active = nullptr, const int32_t* nactive = nullptr,
+                      const int32_t* nvalid = nullptr);
 
 }  // namespace mm

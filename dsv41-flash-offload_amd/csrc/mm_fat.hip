@@ -289,11 +289,15 @@ __device__ __forceinline__ int fat_big_tiles(int c) { return c / FT_BIG + (c % F
 // expert a's tiles and groups, the lists are then filled by all threads, each entry finding its expert by a binary search
 // over the sums in LDS. totals = 256-route tiles, FT_MID-route tiles, row groups. The FT_MID-route list holds the tiles of
 // three row groups first, then those of two, then those of one: the longest start first.
+// CHOICE (a fused call that either path may take, cap 0): the active experts and routed positions that the decode path is to
+// compute go to choice[0], [1]: all of them and no tile here, or none (see fused_path).
+template <bool CHOICE>
 __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts, const int32_t* offsets,
                                                          const int32_t* active, const int32_t* nactive,
                                                          const int64_t* gate, const int64_t* up, const int64_t* down,
                                                          ExpertRec* rec, FatTile* big, FatTile* mid, int2* groups,
-                                                         int32_t* totals, int max_active, int cap, BigRule rule)
+                                                         int32_t* totals, int max_active, int cap, BigRule rule,
+                                                         int32_t* choice, int E, int n)
 {
     // lists: 256-route tiles; tiles of three, two and one row groups; row groups
     constexpr int NL = 5;
@@ -325,6 +329,18 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
         if (a == 0) s_off[i][FT_PLAN_MAX] = total;
         return total;
     };
+    if constexpr (CHOICE)
+    {
+        const int64_t records = scan(1, (c + 15) / 16), tiles = scan(2, (c + FT_MID - 1) / FT_MID);
+        __syncthreads();
+        const bool decode = 800 * records + 8 * (int64_t)n <= 900 * tiles + 10400;
+        if (a == 0)
+        {
+            choice[0] = decode ? nact : 0;
+            choice[1] = decode ? offsets[E] : 0;
+        }
+        if (decode) c = 0;
+    }
     int nbig = c >= rule.min_rows ? fat_big_tiles(c) : 0;
     int tbig = scan(0, nbig);
     if (tbig < rule.min_tiles)                                    // uniform: too few to fill the GPU
@@ -1219,14 +1235,16 @@ __global__ __launch_bounds__(256, 2) void k_mid(FatArgs a)
         mid_tile<MODE, 1, EXACT, YH>(a, smem, rows, pos0, e, grp, nu, rp);
 }
 
+// (skip: where not 0, the decode path has computed the call)
 // Weighted combine of the fat routes: out[t] = (accumulate ? out[t] : 0) + sum_j w_j y_j over the routes j of
 // token t whose expert has more than cap routes, fp32 fma in ascending j (with cap 0 this is mm_combine). The
 // per-route rows y_j are fp16 (the down GEMM writes them so: its output transform rounds every value to fp16).
 __global__ __launch_bounds__(256) void k_fat_combine(float* __restrict__ out, const uint16_t* __restrict__ Y,
                                                      const int64_t* __restrict__ ids, const float* __restrict__ w,
                                                      const int32_t* __restrict__ counts, int T, int k, int H, int E,
-                                                     int cap, int accumulate)
+                                                     int cap, int accumulate, const int32_t* skip)
 {
+    if (skip && skip[0] != 0) return;
     const int t = blockIdx.y;
     const int h = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (t >= T || h >= H) return;
@@ -1419,6 +1437,7 @@ struct FatWs
     float* xds;           // [max_groups][I / 128][GRP_ROWS] down-input sums
     int nxs;
     float* Y;             // [n][H]
+    size_t plan_bytes;    // up to xa: permutation, records and lists
     size_t bytes;
 };
 
@@ -1454,6 +1473,8 @@ static FatWs fat_carve(void* base, int n, int E, int H, int I)
     w.big = (FatTile*)at[7]; w.mid = (FatTile*)at[8]; w.groups = (int2*)at[9]; w.totals = (int32_t*)at[10];
     w.xa = (uint16_t*)at[11]; w.xd = (uint16_t*)at[12]; w.Y = (float*)at[13];
     w.xs = (float*)at[14]; w.xds = (float*)at[15];
+    w.plan_bytes = 0;
+    for (int i = 0; i < 11; ++i) w.plan_bytes += sizes[i];
     w.bytes = off;
     return w;
 }
@@ -1477,21 +1498,41 @@ static int fat_check(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     return MM_OK;
 }
 
-// Plan, input transform and both GEMMs over the sorted positions in ws (counts, offsets, order, active, nactive filled):
-// Y rows of every position of an active expert with more than cap routes. token_sorted: the positions' tokens, or null
-// (order[pos] / topk).
-static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* token_sorted, int n,
-                     int cap, const FatWs& ws, hipStream_t s, bool yh, bool fused)
+// How a call's experts are taken: the fused call by the layer's codebook evaluation, the others with fp16-rounded weights.
+struct FatMode
 {
-    // the fused call takes the layer's codebook evaluation; the others round the weights to fp16
-    const bool exact = !fused || (L->flags & MM_LAYER_EXACT) != 0;
-    const BigRule rule = fused ? BigRule{ (FT_BIG_WORK + L->I / 128 - 1) / (L->I / 128), 0 } : BigRule{ 0, FT_BIG_ROWS };
+    bool exact;
+    BigRule rule;
+};
+static FatMode fat_mode(const mm_layer_t* L, bool fused)
+{
+    if (!fused) return { true, BigRule{ 0, FT_BIG_ROWS } };
+    return { (L->flags & MM_LAYER_EXACT) != 0, BigRule{ (FT_BIG_WORK + L->I / 128 - 1) / (L->I / 128), 0 } };
+}
+
+// Expert records, row groups and tile lists of the sorted positions in ws (counts, offsets, active, nactive filled).
+static void fat_plan(const mm_layer_t* L, int n, int cap, const FatWs& ws, hipStream_t s, const FatMode& mode, int32_t* choice)
+{
     const int E = L->E, na = n < E ? n : E;
-    hipLaunchKernelGGL(k_fat_plan, dim3(1), dim3(FT_PLAN_MAX), 0, s, ws.counts, ws.offsets, ws.active, ws.nactive,
-                       L->gate_ptr, L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.mid, ws.groups, ws.totals, na, cap, rule);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(FT_PLAN_MAX), 0, s, ws.counts, ws.offsets, ws.active, ws.nactive, L->gate_ptr,
+                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.mid, ws.groups, ws.totals, na, cap, mode.rule, choice, E, n);
+    };
+    if (choice) launch(k_fat_plan<true>);
+    else launch(k_fat_plan<false>);
+}
+
+// Input transform and both GEMMs of a plan: Y rows of every position of an active expert with more than cap routes.
+// token_sorted: the positions' tokens, or null (order[pos] / topk).
+static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* token_sorted, int n,
+                     const FatWs& ws, hipStream_t s, bool yh, const FatMode& mode)
+{
+    const bool exact = mode.exact;
     hipLaunchKernelGGL(k_fat_prep, dim3((unsigned)ws.max_groups, (unsigned)ws.nxs),
                        dim3(512), 0, s, x, x_dtype, ws.order, token_sorted, ws.rec, ws.groups, ws.totals + 2, L->suh13,
                        ws.xa, ws.xs, topk, T, L->H);
+    // 256-route tiles a call of n routes can have
+    const int max_big = ws.max_big >= mode.rule.min_tiles && n >= mode.rule.min_rows ? ws.max_big : 0;
     auto grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles * units + 7) & ~(size_t)7)); };    // >= 8 per_xcd
     auto mid_grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles + 7) / 8 * 8 * units)); };
     FatArgs g{ ws.rec, ws.big, ws.totals, ws.xa, L->svh13, L->suh2, L->svh2, ws.order, ws.xd, ws.Y,
@@ -1507,27 +1548,27 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     dm.ntiles = ws.totals + 1;
     // gate/up: 256-route tiles on the 8-wave kernel, down on the 16-wave kernel (same bits; measured on the 16k layer:
     // gate/up equal, down 2.76-2.85 against 2.92-2.94 ms)
-    if (ws.max_big > 0) hipLaunchKernelGGL((k_fat<0, FT_BIG / 32>), grid(ws.max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
+    if (max_big > 0) hipLaunchKernelGGL((k_fat<0, FT_BIG / 32>), grid(max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
     if (exact) hipLaunchKernelGGL((k_mid<0, true>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
     else hipLaunchKernelGGL((k_mid<0, false>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
     if (yh)
     {
-        if (ws.max_big > 0)
-            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64, true>), grid(ws.max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
+        if (max_big > 0)
+            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64, true>), grid(max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
         if (exact) hipLaunchKernelGGL((k_mid<1, true, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
         else hipLaunchKernelGGL((k_mid<1, false, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
     }
     else
     {
-        if (ws.max_big > 0)
-            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64>), grid(ws.max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
+        if (max_big > 0)
+            hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64>), grid(max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
         if (exact) hipLaunchKernelGGL((k_mid<1, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
         else hipLaunchKernelGGL((k_mid<1, false>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
     }
     return check_launch("fat path");
 }
 
-// Permutation, input transform, plan and both GEMMs: Y rows of every route whose expert has more than cap routes.
+// Permutation, plan, input transform and both GEMMs: Y rows of every route whose expert has more than cap routes.
 static int fat_run(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, int cap,
                    const FatWs& ws, hipStream_t s, bool yh, bool fused)
 {
@@ -1535,7 +1576,18 @@ static int fat_run(const mm_layer_t* L, const void* x, int x_dtype, int T, int t
     int rc = permute_launch(ids, nullptr, n, topk, E, ws.counts, ws.offsets, ws.order, nullptr, nullptr, nullptr,
                             ws.active, ws.nactive, nullptr, ws.pws, ws.pws_bytes, s);
     if (rc) return rc;
-    return fat_gemms(L, x, x_dtype, T, topk, nullptr, n, cap, ws, s, yh, fused);
+    const FatMode mode = fat_mode(L, fused);
+    fat_plan(L, n, cap, ws, s, mode, nullptr);
+    return fat_gemms(L, x, x_dtype, T, topk, nullptr, n, ws, s, yh, mode);
+}
+
+static int fat_combine(const mm_layer_t* L, int T, int topk, const int64_t* ids, const float* w, int cap, int accumulate,
+                       float* out, const FatWs& ws, hipStream_t s, const int32_t* skip)
+{
+    const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
+    hipLaunchKernelGGL(k_fat_combine, grid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.Y), ids, w,
+                       ws.counts, T, topk, L->H, L->E, cap, accumulate, skip);
+    return check_launch("fat layer");
 }
 
 // fat_run and the weighted combine of its rows.
@@ -1543,11 +1595,7 @@ static int fat_layer(const mm_layer_t* L, const void* x, int x_dtype, int T, int
                      int cap, int accumulate, float* out, const FatWs& ws, hipStream_t s, bool fused)
 {
     const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true, fused);
-    if (r) return r;
-    const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
-    hipLaunchKernelGGL(k_fat_combine, grid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.Y), ids, w,
-                       ws.counts, T, topk, L->H, L->E, cap, accumulate);
-    return check_launch("fat layer");
+    return r ? r : fat_combine(L, T, topk, ids, w, cap, accumulate, out, ws, s, nullptr);
 }
 
 // Workspace of the sorted-route form: the fat sections for n positions, then the token lists.
@@ -1576,14 +1624,54 @@ static FatbWs fatb_carve(void* base, int n, int T, int E, int H, int I)
 
 // ------------------------------------------------------------------------------------ the fused-MoE call
 
-// A call runs as a whole on one path. Up to FUSED_DECODE_MAX routes it is the decode path, whose launches cut the experts'
-// rows into equal runs over the whole GPU; an expert with many routes costs it a pass per 16, which few experts of such a
-// call need. Above, it is the grouped GEMM: k_mid decodes a tile as fast for one route as for 32 (34 against 33 ns per 16 x 16
-// tile and SIMD), and the decode path's combine over all tokens grows with the call (at 4,096 tokens 0.64 ms). Whole calls on
-// the decode path / on the grouped GEMM, H 4096, top-8 of 384: 100 tokens 741 / 796 us (Zipf routing) and 856 / 970 (64 hot
-// experts), 128 tokens 854 / 897 and 957 / 1,068; beyond 1,024 routes the decode path needs the permutation. Against the
-// experts divided by cap over both paths: 884 and 879 us at 100 tokens.
-constexpr int FUSED_DECODE_MAX = 1024;
+// A call runs as a whole on one path. The decode path cuts the experts' rows into equal runs over the whole GPU, but decodes
+// an expert once per 16 of its routes (a record); k_mid decodes a tile as fast for one route as for 32 and takes up to 96, but
+// is slower per tile and needs many to fill the GPU, and its call has more launches. Whole calls, us on the decode path / on the
+// grouped GEMM, H 4096, I 2048, n routes over E experts, routing uniform (u), Zipf (z) or on 8 experts (8):
+//   E 8:   n 256 104 / 133 u, 113 / 155 z; 512 175 / 163, 168 / 169; 1,024 281 / 172, 289 / 174
+//   E 16:  n 256 116 / 119 u, 123 / 138 z; 400 152 / 135, 146 / 164; 1,024 287 / 175, 288 / 187
+//   E 64:  n 600 276 / 304 u, 316 / 313 z; 768 290 / 308, 345 / 326; 1,020 376 / 309, 408 / 361
+//   E 128: n 800 470 / 535 u, 488 / 518 z; 1,024 488 / 532, 539 / 531; 1,600 586 / 552, 679 / 574
+//   E 256: n 1,024 861 / 957 u, 731 / 763 z; 2,048 932 / 993, 1,043 / 946; 3,200 1,104 / 1,002, 1,341 / 1,054
+//   E 384: n 1,024 1,141 / 1,326 u, 879 / 907 z, 249 / 174 8; 2,048 1,295 / 1,414, 1,252 / 1,146, 475 / 225
+// So up to GV_ROUTE_MAX routes the decode path (routed in-kernel) takes 384 routes or 10 per expert; what the host cannot see
+// is left there: tokens that agree on a few of many experts. Above, the permutation is needed in any case, and while experts
+// get few routes (7 each on average; 9 to 1,280 routes) the plan kernel chooses on the device by records and tiles: decode path
+// 40 + 3.05 records + n / 33 us, grouped GEMM 80 + 3.45 tiles us, within 5 % of the above. The launches of the path not taken
+// find no work (25-30 us in all), so calls of small layers, in the end faster than that, are not given the choice (E H I below
+// 2^30: 512 experts, H 2048, I 512, 2,500 routes take 290 us on the grouped GEMM and 330 chosen). With more routes the experts
+// are busy enough for the grouped GEMM.
+enum class FusedPath { DECODE, CHOICE, GEMM };
+static FusedPath fused_path(int n, int E, int H, int I)
+{
+    if (n <= GV_ROUTE_MAX) return n <= std::max(384, 10 * E) ? FusedPath::DECODE : FusedPath::GEMM;
+    const bool few = n <= std::min(9 * E, std::max(7 * E, 1280)), large = (int64_t)E * H * I >= (int64_t)1 << 30;
+    return few && large && decode_fits(n, E, H, I) ? FusedPath::CHOICE : FusedPath::GEMM;
+}
+
+// Workspace of a call that either path may take: the grouped GEMM's, with the decode workspace over its inputs and rows (one of
+// the two is used, and the decode path's launches come first), then the choice.
+struct FusedWs
+{
+    FatWs f;
+    void* dws;
+    size_t dws_bytes;
+    int32_t* choice;      // [2]
+    size_t bytes;
+};
+
+static FusedWs fused_carve(void* base, int n, int E, int H, int I)
+{
+    FusedWs w;
+    w.f = fat_carve(base, n, E, H, I);
+    w.dws_bytes = mm_gemv_workspace(n, E, H, I);
+    const size_t most = std::max(w.f.bytes, w.f.plan_bytes + w.dws_bytes);      // multiples of 256
+    char* p = static_cast<char*>(base);
+    w.dws = p ? p + w.f.plan_bytes : nullptr;
+    w.choice = p ? (int32_t*)(p + most) : nullptr;
+    w.bytes = most + 256;
+    return w;
+}
 
 }  // namespace mm
 
@@ -1595,7 +1683,12 @@ size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap)
 {
     if (T <= 0 || topk <= 0 || E <= 0 || H <= 0 || I <= 0 || cap < 0) return 0;
     const int n = T * topk;
-    return n <= FUSED_DECODE_MAX ? mm_gemv_workspace(n, E, H, I) : fat_carve(nullptr, n, E, H, I).bytes;
+    switch (fused_path(n, E, H, I))
+    {
+    case FusedPath::DECODE: return mm_gemv_workspace(n, E, H, I);
+    case FusedPath::CHOICE: return fused_carve(nullptr, n, E, H, I).bytes;
+    default: return fat_carve(nullptr, n, E, H, I).bytes;
+    }
 }
 
 int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1607,17 +1700,31 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
     MM_CHECK_ARG(topk <= 16, "mm_fused_moe: topk must be at most 16");
     const int n = T * topk, E = L->E;
     // a limit of the interface: n, or E x cap for larger n, transformed inputs within 32-bit byte offsets
-    const size_t npos = n <= FUSED_DECODE_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
+    const size_t npos = n <= GV_ROUTE_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
     MM_CHECK_ARG(npos * 2 * std::max(L->H, L->I) * 2 < ((size_t)1 << 31),
                  "mm_fused_moe: too many decode-path positions (%zu)", npos);
     const size_t need = mm_fused_moe_workspace(T, topk, E, L->H, L->I, cap);
     MM_CHECK_ARG(workspace && workspace_bytes >= need, "mm_fused_moe: workspace too small (%zu < %zu)", workspace_bytes,
                  need);
-    if (n <= FUSED_DECODE_MAX)
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const FusedPath path = fused_path(n, E, L->H, L->I);
+    if (path == FusedPath::DECODE)
         return moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, workspace, workspace_bytes, stream,
                                  "mm_fused_moe");
-    return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I),
-                     reinterpret_cast<hipStream_t>(stream), true);
+    if (path == FusedPath::GEMM)
+        return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I), s, true);
+    const FusedWs ws = fused_carve(workspace, n, E, L->H, L->I);
+    int r = permute_launch(ids, nullptr, n, topk, E, ws.f.counts, ws.f.offsets, ws.f.order, nullptr, nullptr, nullptr,
+                           ws.f.active, ws.f.nactive, nullptr, ws.f.pws, ws.f.pws_bytes, s);
+    if (r) return r;
+    const FatMode mode = fat_mode(L, true);
+    fat_plan(L, n, 0, ws.f, s, mode, ws.choice);
+    // the decode path's launches first: the grouped GEMM's inputs lie over their workspace
+    r = moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, ws.dws, ws.dws_bytes, stream, "mm_fused_moe",
+                          ws.f.offsets, ws.f.order, ws.f.active, ws.choice, ws.choice + 1);
+    if (r) return r;
+    r = fat_gemms(L, x, x_dtype, T, topk, nullptr, n, ws.f, s, true, mode);
+    return r ? r : fat_combine(L, T, topk, ids, w, 0, 0, out, ws.f, s, ws.choice + 1);
 }
 
 size_t mm_prefill_workspace(int n, int E, int H, int I)
@@ -1683,7 +1790,9 @@ int mm_fat_batched(const mm_layer_t* L, const void* x, int x_dtype, int T, int n
     hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)std::min((T + 255) / 256, 1024)), dim3(256), 0, s, ws.tcount, T, 0);
     hipLaunchKernelGGL(k_fatb_tokens<1>, dim3(pg), dim3(256), 0, s, token_sorted, ws.f.counts, ws.f.offsets, ws.f.order,
                        ws.tcount, ws.toff, ws.tpos, T, E, n);
-    int r = fat_gemms(L, x, x_dtype, T, 1, token_sorted, n, cap, ws.f, s, true, false);
+    const FatMode mode = fat_mode(L, false);
+    fat_plan(L, n, cap, ws.f, s, mode, nullptr);
+    int r = fat_gemms(L, x, x_dtype, T, 1, token_sorted, n, ws.f, s, true, mode);
     if (r) return r;
     const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);
     hipLaunchKernelGGL(k_fatb_combine, grid, dim3(256), 0, s, out, reinterpret_cast<const uint16_t*>(ws.f.Y),

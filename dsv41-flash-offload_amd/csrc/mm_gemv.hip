@@ -35,7 +35,6 @@ namespace mm {
 constexpr int GV_WAVES = 4;
 constexpr int GV_THREADS = 64 * GV_WAVES;
 constexpr int GV_COLS = 128;          // output columns per segment (8 tiles)
-constexpr int GV_ROUTE_MAX = 1024;    // in-kernel routing limit (routes per call)
 // Routes per record (one pass of a partial-sum wave) in calls of more than this many tokens. A segment costs
 // its waves one pass over its rows, whatever its routes, so equal runs of rows are equal work: with one record per expert
 // the waves of an expert with more than 16 routes took twice as long as the others and the launch waited for them (24
@@ -120,8 +119,13 @@ __global__ __launch_bounds__(256) void k_route_prep(PrepArgs a)
     const int nbk = walk ? 1 : a.nb;
     const int blk = blockIdx.x % nbk, m = (blockIdx.x / nbk) & 1, idx = blockIdx.x / (2 * nbk);
     const bool writer = m == 0 && blk == 0;      // the one workgroup of a route that writes its routing data
+    if (a.gated && a.nvalid_in[0] == 0)          // the whole call is left to another path
+    {
+        if (blockIdx.x == 0 && tid == 0) a.counts[0] = a.counts[1] = 0;
+        return;
+    }
     // routing from the permutation: the workgroups of index idx own sorted position idx
-    const int nvalid_perm = perm ? a.offsets[a.E] : 0;
+    const int nvalid_perm = perm ? a.nvalid_in[0] : 0;
     const int s = perm ? a.order[idx] : idx;
     const int64_t e64 = a.ids[s];
     const int t = s / a.topk;
@@ -737,6 +741,7 @@ struct DEpiArgs
     float* Y;                 // [n][H] (per-route rows)
     float* out;               // [T][H] (combine)
     int npos, H, I, topk, nwaves, cap, affine;
+    int gated;                // combine: out is left untouched where no route is computed
 };
 
 // Down output of one (sorted position, 128-column block of H): pieces added in order (then the AFFINE
@@ -800,6 +805,7 @@ __global__ __launch_bounds__(1024) void k_down_combine(DEpiArgs a)
     const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;
     const int ncb = a.H / GV_COLS;
     const int t = blockIdx.x / ncb, c = (blockIdx.x % ncb) * GV_COLS;
+    if (a.gated && a.counts[1] == 0) return;
     if (j < a.topk)
     {
         // round trip 1: the route's position, expert, active index and weight and the active-expert count. A pick
@@ -883,12 +889,15 @@ static int piece_cap(int n)
 // Most records of n routes over E experts: a route each, or one per expert and one per further REC_ROUTES routes.
 static int max_records(int n, int E) { return std::min(n, std::min(n, E) + n / REC_ROUTES); }
 // tile rows of a partial launch (records x 2 matrices x column blocks x tile rows) count in int
-static bool rows_fit(const mm_layer_t* L, int records) { return (size_t)records * L->H / 1024 * L->I < ((size_t)1 << 31); }
+static bool rows_fit(int H, int I, int records) { return (size_t)records * H / 1024 * I < ((size_t)1 << 31); }
+// the inputs of n routes are addressed with 32-bit buffer offsets
+static bool inputs_fit(int n, int H, int I) { return (size_t)n * 2 * std::max(H, I) * 2 < ((size_t)1 << 31); }
+bool decode_fits(int n, int E, int H, int I) { return inputs_fit(n, H, I) && rows_fit(H, I, std::min(n, E)); }
 // Records of REC_ROUTES routes (the same ones from a permutation as from the ids) above REC_ROUTES tokens, one per expert
 // below and where more would leave int.
 static bool split_records(const mm_layer_t* L, int n, int topk)
 {
-    return n > REC_ROUTES * topk && rows_fit(L, max_records(n, L->E));
+    return n > REC_ROUTES * topk && rows_fit(L->H, L->I, max_records(n, L->E));
 }
 
 // Workspace of n routes whose sorted positions lie below npos (npos = n unless a caller bounds the positions).
@@ -972,8 +981,7 @@ static int check_common(const mm_layer_t* L, const void* x, int x_dtype, int T, 
     MM_CHECK_ARG(x_dtype == MM_DTYPE_F16 || x_dtype == MM_DTYPE_BF16 || x_dtype == MM_DTYPE_F32,
                  "%s: x_dtype must be MM_DTYPE_F16, MM_DTYPE_BF16 or MM_DTYPE_F32", who);
     MM_CHECK_ARG(T > 0 && n > 0 && topk > 0 && n <= T * topk, "%s: bad T/n/topk", who);
-    MM_CHECK_ARG((size_t)n * 2 * (L->H > L->I ? L->H : L->I) * 2 < ((size_t)1 << 31), "%s: too many routes", who);
-    MM_CHECK_ARG(rows_fit(L, std::min(n, L->E)), "%s: too many routes", who);
+    MM_CHECK_ARG(decode_fits(n, L->E, L->H, L->I), "%s: too many routes", who);
     MM_CHECK_ARG(max_rows > 0, "%s: max_rows must be at least 1", who);
     const bool perm = offsets != nullptr;
     MM_CHECK_ARG(perm ? (order && active && nactive) : n <= GV_ROUTE_MAX,
@@ -985,16 +993,17 @@ static int check_common(const mm_layer_t* L, const void* x, int x_dtype, int T, 
 
 static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_dtype, int rescale, int n, int npos,
                         int topk, const int64_t* ids, const int32_t* offsets, const int32_t* order,
-                        const int32_t* active, const int32_t* nactive, int cap, hipStream_t s)
+                        const int32_t* active, const int32_t* nactive, const int32_t* nvalid, bool gated, int cap,
+                        hipStream_t s)
 {
     const int nb = prep_blocks(L->H);
     // With records of REC_ROUTES routes and routing in-kernel, one workgroup per route and matrix walks the row: one per 512
     // rows found the routing again each (100 tokens, top-8: 39 us of a 790 us call). With a permutation it pays from three
     // workgroups per CU on (a layer of 24 tokens, H 5120, 335 us walking and 331 not, 200 tokens 1,144 and 1,161).
     const bool split = split_records(L, n, topk), walk = split && (!offsets || n >= PREP_WALK_MIN);
-    PrepArgs p{ x, ids, offsets, order, active, nactive, L->gate_ptr, L->up_ptr, L->down_ptr, L->suh13,
+    PrepArgs p{ x, ids, offsets, order, active, nactive, nvalid, L->gate_ptr, L->up_ptr, L->down_ptr, L->suh13,
                 w.rec, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, w.xa, w.xsum, n, topk, L->E, L->H, nb,
-                x_dtype, rescale, cap, split ? 1 : 0, walk ? 1 : 0, npos };
+                x_dtype, rescale, cap, split ? 1 : 0, walk ? 1 : 0, gated ? 1 : 0, npos };
     launch_route_prep(p, s);
 }
 
@@ -1019,32 +1028,32 @@ static void launch_gu_epilogue(const mm_layer_t* L, const Ws& w, int npos, hipSt
 }
 
 static DEpiArgs down_args(const mm_layer_t* L, const Ws& w, int npos, int topk, const int64_t* ids, const float* wt,
-                          float* Y, float* out)
+                          float* Y, float* out, bool gated = false)
 {
     return DEpiArgs{ w.part_d, w.xdsum, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, ids, wt, L->svh2, Y, out, npos, L->H,
-                     L->I, topk, partial_waves(seg_max(L, npos, 1)), piece_cap(npos), (L->flags & MM_LAYER_EXACT) ? 0 : 1 };
+                     L->I, topk, partial_waves(seg_max(L, npos, 1)), piece_cap(npos), (L->flags & MM_LAYER_EXACT) ? 0 : 1, gated ? 1 : 0 };
 }
 
-// One decode layer (mm_moe_decode) on a caller-provided workspace; `who` names the entry point in errors.
 int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int rescale, int T, int topk, const int64_t* ids,
                       const float* w, int max_rows, float* out, void* workspace, size_t workspace_bytes,
-                      mm_stream_t stream, const char* who)
+                      mm_stream_t stream, const char* who, const int32_t* offsets, const int32_t* order,
+                      const int32_t* active, const int32_t* nactive, const int32_t* nvalid)
 {
     MM_CHECK_ARG(topk > 0 && topk <= MAX_TOPK, "%s: topk must be in [1, %d]", who, MAX_TOPK);
     const int n = T * topk;
-    const int rc = check_common(L, x, x_dtype, T, n, topk, ids, nullptr, nullptr, nullptr, nullptr, max_rows, workspace,
+    const int rc = check_common(L, x, x_dtype, T, n, topk, ids, offsets, order, active, nactive, max_rows, workspace,
                                 workspace_bytes, who);
     if (rc) return rc;
     MM_CHECK_ARG(w && out, "%s: null pointer", who);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const Ws ws = carve(workspace, n, n, L->E, L->H, L->I);
-    launch_prep(L, ws, x, x_dtype, rescale, n, n, topk, ids, nullptr, nullptr, nullptr, nullptr, max_rows, s);
+    launch_prep(L, ws, x, x_dtype, rescale, n, n, topk, ids, offsets, order, active, nactive, nvalid, nvalid != nullptr, max_rows, s);
     launch_partial<0>(L, ws, n, s);
     launch_gu_epilogue(L, ws, n, s);
     launch_partial<1>(L, ws, n, s);
     const int threads = 64 * (topk < 2 ? 2 : topk);
     hipLaunchKernelGGL(k_down_combine, dim3(T * (L->H / GV_COLS)), dim3(threads), 0, s,
-                       down_args(L, ws, n, topk, ids, w, nullptr, out));
+                       down_args(L, ws, n, topk, ids, w, nullptr, out, nvalid != nullptr));
     return check_launch(who);
 }
 
@@ -1072,7 +1081,9 @@ int mm_expert_gemv(const mm_layer_t* L, const void* x, int x_dtype, int rescale,
     MM_CHECK_ARG(Y || !(phases & 16), "mm_expert_gemv: null Y");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const Ws w = carve(workspace, n, n, L->E, L->H, L->I);
-    if (phases & 1) launch_prep(L, w, x, x_dtype, rescale, n, n, topk, ids, offsets, order, active, nactive, max_rows, s);
+    if (phases & 1)
+        launch_prep(L, w, x, x_dtype, rescale, n, n, topk, ids, offsets, order, active, nactive,
+                    offsets ? offsets + L->E : nullptr, false, max_rows, s);
     if (phases & 2) launch_partial<0>(L, w, n, s);
     if (phases & 4) launch_gu_epilogue(L, w, n, s);
     if (phases & 8) launch_partial<1>(L, w, n, s);

@@ -299,7 +299,7 @@ def apply_exl3_fused_moe(x2d, ids, weights, layer, inners=None, expert_map=None,
             and T >= _DMA_MIN_TOKENS and inners is None and not torch.cuda.is_current_stream_capturing()):
         return _dma_prefill(x2d, ids, w16, layer, limit, dev)
     # at most FAT_EXPERT_THRESHOLD tokens: every route on the decode path (the reference's fat_possible test); above it
-    # the call's number of routes decides. No call synchronises the host, so every call can be captured in a graph.
+    # the call's routes and the layer's experts decide. No call synchronises the host, so every call can be captured in a graph.
     return moe.moe_forward(L, x2d, ids, w16, fat_threshold=FAT_EXPERT_THRESHOLD)
 
 

@@ -6,8 +6,8 @@ import torch
 
 from . import _lib
 
-# Default fat-expert threshold of moe_forward: experts with more routes than this in a call go to the fat-expert
-# grouped GEMM (the reference image's VLLM_EXL3_FAT_THRESHOLD, docker/entrypoint.sh:69).
+# Default fat-expert threshold of moe_forward (the reference image's VLLM_EXL3_FAT_THRESHOLD, docker/entrypoint.sh:69): calls
+# of at most this many tokens run on the decode path, larger ones go to mm_fused_moe.
 FAT_THRESHOLD = 32
 # Routes per call the decode path routes in-kernel (more go through the permutation).
 GEMV_ROUTE_MAX = 1024
@@ -117,8 +117,8 @@ def moe_forward(store, x, ids, w, shared_expert=None, fat_threshold=FAT_THRESHOL
 
     Routes with ids outside [0, E) contribute nothing. As the reference's fused-MoE call does
     (patches/vllm-exl3-host-dma.patch:241-290), a call of at most `fat_threshold` tokens runs every route on the
-    decode path. A larger call goes to mm_fused_moe, which takes the decode path or the grouped GEMM by its number of
-    routes. No call synchronises the host, so every call can be captured in a HIP graph."""
+    decode path. A larger call goes to mm_fused_moe, which takes the decode path or the grouped GEMM by its routes and
+    experts. No call synchronises the host, so every call can be captured in a HIP graph."""
     T = x.shape[0]
     ids, w = _with_shared(ids, w, T, shared_expert)
     k = ids.shape[1]
@@ -132,8 +132,8 @@ def moe_forward(store, x, ids, w, shared_expert=None, fat_threshold=FAT_THRESHOL
 
 
 def fused_moe(store, x, ids, w, cap, stream=None):
-    """mm_fused_moe: out fp32 [T, H] over ids [T, k] / w [T, k], on the decode path (up to 1,024 routes) or the grouped
-    GEMM; `cap` is the reference's threshold between the two and only bounds the call's size."""
+    """mm_fused_moe: out fp32 [T, H] over ids [T, k] / w [T, k], on the decode path (few routes, or few per expert) or the
+    grouped GEMM; `cap` is the reference's threshold between the two and only bounds the call's size."""
     T, k = ids.shape
     x = x.contiguous()
     ids = ids.contiguous().long()

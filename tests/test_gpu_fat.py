@@ -276,3 +276,78 @@ def test_full_tiles_of_a_large_call(dev):
     ref = OracleLayer(st, seed).forward(x16[rows].astype(np.float32), ids[rows], w[rows])
     ok, m = within_tolerance(out.cpu().numpy()[rows], ref)
     assert ok, m
+
+
+@pytest.mark.parametrize("E,H,I,T,k,hot,path", [
+    (8, 256, 128, 192, 2, 8, "decode"), (8, 256, 128, 193, 2, 8, "gemm"), (64, 256, 128, 80, 8, 64, "decode"),
+    (64, 256, 128, 81, 8, 64, "gemm"), (160, 256, 128, 1024, 1, 160, "decode"), (160, 256, 128, 1025, 1, 160, "gemm"),
+    (1024, 1024, 1024, 1025, 1, 90, "decode"), (1024, 1024, 1024, 1025, 1, 12, "gemm"),
+    (1024, 1024, 1024, 540, 2, 110, "decode"), (1024, 1024, 1024, 540, 2, 8, "gemm"), (1024, 1024, 1024, 1195, 6, 12, "gemm")])
+def test_fused_call_on_either_side_of_its_path_rule(dev, E, H, I, T, k, hot, path):
+    """Fused calls at the last routes of the decode path and the first of the grouped GEMM (384 routes, or 10 per expert),
+    and above 1,024 routes of large layers on either side of the choice made on the device (up to 7 routes per expert; by
+    records of 16 and tiles of 96 routes): nothing is written past the workspace asked for, stale workspace is not read, the
+    decode path's calls equal it bit for bit whatever the threshold, and every call matches the oracle."""
+    import torch
+    from mi355moe import _lib, moe
+    seed = 9300 + E
+    st = make_store(E, H, I, seed, device=dev, exact=True)
+    rng = np.random.default_rng(T)
+    ids = np.stack([rng.choice(hot, k, replace=False) for _ in range(T)]).astype(np.int64)
+    ids[::13, k - 1] = -1
+    w = rng.uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    n = T * k
+    counts = np.bincount(ids[ids >= 0], minlength=E)
+    if n <= 1024:
+        decode = n <= max(384, 10 * E)
+    else:
+        chosen = n <= min(9 * E, max(7 * E, 1280)) and E * H * I >= 1 << 30
+        decode = chosen and 800 * np.sum(-(-counts // 16)) + 8 * n <= 900 * np.sum(-(-counts // 96)) + 10400
+    assert decode == (path == "decode")
+    print(f"fused call E={E} T={T} k={k} hot={hot} ({path})", flush=True)
+    xd, idd, wd = _t(x16, dev), _t(ids, dev), _t(w, dev)
+    wsb = _lib.load().mm_fused_moe_workspace(T, k, E, H, I, 32)
+    ws = torch.full((wsb + 4096,), 0xff, dtype=torch.uint8, device=dev)     # NaNs before, guard bytes behind
+    out = torch.empty((T, H), dtype=torch.float32, device=dev)
+    _lib.call("mm_fused_moe", st.mm_layer(), xd.data_ptr(), _lib.DTYPE_F16, T, k, idd.data_ptr(), wd.data_ptr(), 32,
+              out.data_ptr(), ws.data_ptr(), wsb, _lib.stream_ptr())
+    again = moe.fused_moe(st, xd, idd, wd, 1)
+    routed = moe.decode_routes(st, xd, idd, wd, n)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again) and (ws[wsb:] == 0xff).all().item()
+    assert torch.equal(out, routed) == (path == "decode")
+    rows = np.arange(0, T, max(1, T // 200))
+    ref = OracleLayer(st, seed).forward(x16[rows].astype(np.float32), ids[rows], w[rows])
+    ok, m = within_tolerance(out.cpu().numpy()[rows], ref)
+    assert ok, m
+
+
+def test_fused_call_chosen_on_the_device_in_a_graph(dev):
+    """A captured call of more than 1,024 routes in the range where the device chooses the path: replays with routes that
+    take the decode path, the grouped GEMM, nothing (every id masked: zeros) and the decode path again equal the eager calls
+    bit for bit."""
+    import torch
+    from mi355moe import moe
+    H, I, E, T = 1024, 1024, 1024, 1100
+    st = make_store(E, H, I, 9400, device=dev)
+    rng = np.random.default_rng(3)
+    x = _t(rng.normal(0, 1, (T, H)).astype(np.float16), dev)
+    w = _t(rng.uniform(0.1, 1.0, (T, 1)).astype(np.float32), dev)
+    wide, few, none = (_t(v.astype(np.int64), dev) for v in (rng.integers(0, E, (T, 1)), rng.integers(0, 6, (T, 1)),
+                                                             np.full((T, 1), -1)))
+    print("fused call chosen in a graph", flush=True)
+    eager = [moe.fused_moe(st, x, i, w, 32) for i in (wide, few, none)]
+    torch.cuda.synchronize()
+    assert torch.equal(eager[0], moe.decode_routes(st, x, wide, w, T))
+    assert not torch.equal(eager[1], moe.decode_routes(st, x, few, w, T)) and torch.count_nonzero(eager[2]).item() == 0
+    ids = wide.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = moe.fused_moe(st, x, ids, w, 32)
+    for step, (i, want) in enumerate(zip((wide, few, none, wide), (eager[0], eager[1], eager[2], eager[0]))):
+        ids.copy_(i)
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), f"replay {step}"
