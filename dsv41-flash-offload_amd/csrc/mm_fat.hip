@@ -32,23 +32,41 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int FT_BIG = 256;         // routes per tile (8 row blocks per row-wave)
 constexpr int FT_MID = 96;          // routes per tile of k_mid
-constexpr int FT_BIG_MIN = 193;     // smallest remainder of c / 256 that takes a 256-route tile (two FT_MID tiles hold 192)
+constexpr int FT_SMALL = 128;       // routes per tile of k_fat16<*, 2>
 
-// Where 256-route tiles are used. The kernels of the two tile sizes add an expert's products in different orders.
-//   a fused call: where it has workgroups of 256-route tiles for at least three rounds of the GPU (one fits a CU). Fewer
-//     leave CUs idle that FT_MID-route tiles fill: 3 tiles (48 workgroups) of a 512-token call took 214 us of its 1,540
-//     where FT_MID-route tiles took 60; at 64 tiles (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at
-//     297 (16,384 tokens) 8.25 and 8.65.
-//   the other entry points, whose rows must have the same bits whichever other experts a call computes (a layer in one call
-//     or in staging batches): by the expert's own routes, from three such tiles on. Staging batches hold few experts: 12
-//     tiles of a batch of 16 experts took 189 us of its 470, as FT_MID-route tiles 50.
-struct BigRule
+// Which tiles an expert's routes take. Tiles of 256 routes (and of 128, where the weights are rounded) cost the least per route
+// once there are several rounds of workgroups of them (one fits a CU), FT_MID-route tiles leave fewer CUs idle before that and
+// fewer rows empty. The kernels of the tile sizes add an expert's products in different orders, except those of 256 and 128.
+//   a fused call (FatCall::FUSED): 256-route tiles where it has at least three rounds (FT_BIG_WORK workgroups) of them, the
+//     rest in FT_MID-route tiles. 3 tiles (48 workgroups) of a 512-token call took 214 us of its 1,540 where FT_MID-route tiles
+//     took 60; at 64 tiles (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at 297 (16,384 tokens) 8.25 and 8.65.
+//   a whole call with rounded weights (WHOLE): the same, but from a remainder of 129 routes on, and the remainders of 97 to 128
+//     routes in 128-route tiles from six rounds of them on; then the shorter ones too, if they are under one and a half rounds
+//     (a launch of a few k_mid workgroups takes 99 + 50 us). k_mid costs more with rounded weights (55 against 34 ns per 16 x 16
+//     tile and SIMD). mm_moe_prefill, FT_MID-route tiles for experts below 768 routes / this, ms: H 5120, 16,384 tokens 10.91 /
+//     10.47 (64 hot experts), 10.94 / 10.05 (even routing); 8,192 6.51 / 6.10 (even); H 4096, 16,384 10.50 / 9.60 (even), 8,192 5.49 /
+//     5.33 (even); 4,096 tokens on 170 experts 2.85 / 2.58, on 64 2.60 / 2.26. A 256-route tile of fewer than FT_FULL routes counts
+//     half: 64 of 154 routes (2,048 tokens) take 2.29 ms a call, as FT_MID-route tiles 2.22.
+//   some experts of a layer (EXPERTS; mm_fat_batched), whose rows must have the same bits whichever others the call computes (a
+//     layer in one call or in staging batches): by the expert's own routes and the size of the layer's call. From 768 routes on 256-route
+//     tiles: a staging batch of 16 experts holds few (12 took 189 us of its 470, as FT_MID-route tiles 50). In layers of more than
+//     FT_LARGE routes and 200 per expert every expert takes 256- and 128-route tiles, as many staged experts then do (16 of a
+//     16,384-token call, H 4096: 840 us without, 775 with; the whole call at H 5120 10.9 and 10.4 ms).
+struct TileRule
 {
-    int min_tiles;      // of the call
-    int min_rows;       // of the expert
+    int min_tiles;      // 256-route tiles of the call
+    int min_rows;       // routes of an expert that takes them
+    int min_rest;       // remainder of c / 256 that takes one more
+    int min_small;      // 128-route tiles of the call
+    int fold;           // FT_MID-route tiles of up to 128 routes that go with them
 };
 constexpr int FT_BIG_WORK = 3 * 256;
 constexpr int FT_BIG_ROWS = 3 * FT_BIG;
+constexpr int FT_REST = 193;        // two FT_MID tiles hold 192
+constexpr int FT_REST_EXACT = 129;
+constexpr int FT_FULL = 177;
+constexpr int FT_LARGE = 80000;
+constexpr int FT_NEVER = 0x3fffffff;
 constexpr int GRP_ROWS = 32;        // rows of a row group
 constexpr int GRP_HALVES = 1024;    // one matrix's 32-element step of a row group
 // 128-blocks per input transform workgroup (16,384 tokens, H 4096, 2.3 GB written: 783 us with 2, 844 with 4, 946 with 8;
@@ -164,7 +182,7 @@ __device__ __forceinline__ int lane8_k(int lane, int i)
 
 // One 16-lane group transforms row `rl` of a row group: blocks b0 .. b1 - 1 of the token's row, both matrices (the
 // input is read once), two blocks per pass, all loaded before any is used.
-template <int XD>
+template <int XD, bool SUMS>
 __device__ __forceinline__ void fat_prep_row(const void* x, size_t row, const uint16_t* su0, uint16_t* dst, int H,
                                              int b0, int b1, float (&sum)[2])
 {
@@ -232,8 +250,9 @@ __device__ __forceinline__ void fat_prep_row(const void* x, size_t row, const ui
                     v[i + 1] = xv[i + 1] * h2f((uint16_t)(sr[it][m][th] >> 16));
                 }
                 fwht128_lane8(v, sg);
+                if constexpr (SUMS)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) sum[m] += r16(v[i] * HAD);
+                    for (int i = 0; i < 8; ++i) sum[m] += r16(v[i] * HAD);
                 uint4 o;
                 o.x = (uint32_t)f2h(v[0] * HAD) | ((uint32_t)f2h(v[1] * HAD) << 16);
                 o.y = (uint32_t)f2h(v[2] * HAD) | ((uint32_t)f2h(v[3] * HAD) << 16);
@@ -248,6 +267,7 @@ __device__ __forceinline__ void fat_prep_row(const void* x, size_t row, const ui
 // One workgroup per (row group, PREP_BLOCKS 128-blocks of the input row): wave w transforms rows 4 w .. 4 w + 3, so the
 // workgroup's waves together write whole 512-byte runs of the row group. The token of a position is token_sorted's
 // (a position of a token outside [0, T) is left unwritten), or order[pos] / topk.
+template <bool SUMS>
 __global__ __launch_bounds__(512) void k_fat_prep(const void* x, int x_dtype, const int32_t* order,
                                                   const int64_t* token_sorted, const ExpertRec* rec, const int2* groups,
                                                   const int32_t* ngroups, const uint16_t* suh13, uint16_t* xa, float* xs,
@@ -266,11 +286,12 @@ __global__ __launch_bounds__(512) void k_fat_prep(const void* x, int x_dtype, co
     uint16_t* dst = xa + (size_t)G * 64 * H + rl * 8;          // a row group: 32 rows x 2 matrices x H
     float sum[2] = { 0.0f, 0.0f };
     if (x_dtype == MM_DTYPE_F16)
-        fat_prep_row<MM_DTYPE_F16>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+        fat_prep_row<MM_DTYPE_F16, SUMS>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
     else if (x_dtype == MM_DTYPE_BF16)
-        fat_prep_row<MM_DTYPE_BF16>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+        fat_prep_row<MM_DTYPE_BF16, SUMS>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
     else
-        fat_prep_row<MM_DTYPE_F32>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+        fat_prep_row<MM_DTYPE_F32, SUMS>(x, (size_t)t * H, su0, dst, H, b0, b1, sum);
+    if constexpr (!SUMS) return;
 #pragma unroll
     for (int m = 0; m < 2; ++m)
     {
@@ -282,12 +303,12 @@ __global__ __launch_bounds__(512) void k_fat_prep(const void* x, int x_dtype, co
     }
 }
 
-// 256-route tiles of an expert with c routes; the rest (at most FT_BIG_MIN - 1 routes) goes to FT_MID-route tiles.
-__device__ __forceinline__ int fat_big_tiles(int c) { return c / FT_BIG + (c % FT_BIG >= FT_BIG_MIN ? 1 : 0); }
+// 256-route tiles of an expert with c routes; the rest (fewer than min_rest routes) goes to the other tiles.
+__device__ __forceinline__ int fat_big_tiles(int c, int min_rest) { return c / FT_BIG + (c % FT_BIG >= min_rest ? 1 : 0); }
 
 // Expert records, row groups and the tile lists of the experts with more than cap routes, one workgroup: thread a counts
 // expert a's tiles and groups, the lists are then filled by all threads, each entry finding its expert by a binary search
-// over the sums in LDS. totals = 256-route tiles, FT_MID-route tiles, row groups. The FT_MID-route list holds the tiles of
+// over the sums in LDS. totals = 256-route tiles, FT_MID-route tiles, row groups, 128-route tiles. The FT_MID-route list holds the tiles of
 // three row groups first, then those of two, then those of one: the longest start first.
 // CHOICE (a fused call that either path may take, cap 0): the active experts and routed positions that the decode path is to
 // compute go to choice[0], [1]: all of them and no tile here, or none (see fused_path).
@@ -295,12 +316,12 @@ template <bool CHOICE>
 __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts, const int32_t* offsets,
                                                          const int32_t* active, const int32_t* nactive,
                                                          const int64_t* gate, const int64_t* up, const int64_t* down,
-                                                         ExpertRec* rec, FatTile* big, FatTile* mid, int2* groups,
-                                                         int32_t* totals, int max_active, int cap, BigRule rule,
+                                                         ExpertRec* rec, FatTile* big, FatTile* small, FatTile* mid,
+                                                         int2* groups, int32_t* totals, int max_active, int cap, TileRule rule,
                                                          int32_t* choice, int E, int n)
 {
-    // lists: 256-route tiles; tiles of three, two and one row groups; row groups
-    constexpr int NL = 5;
+    // lists: 256-route tiles; tiles of three, two and one row groups; row groups; 128-route tiles
+    constexpr int NL = 6;
     __shared__ int s_w[NL][FT_PLAN_MAX / 64];
     __shared__ int s_off[NL][FT_PLAN_MAX + 1];             // exclusive sums
     const int a = threadIdx.x, lane = a & 63, wave = a >> 6;
@@ -341,15 +362,28 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
         }
         if (decode) c = 0;
     }
-    int nbig = c >= rule.min_rows ? fat_big_tiles(c) : 0;
-    int tbig = scan(0, nbig);
-    if (tbig < rule.min_tiles)                                    // uniform: too few to fill the GPU
+    int nbig = c >= rule.min_rows ? fat_big_tiles(c, rule.min_rest) : 0;
+    // (a tile of fewer than FT_FULL routes counts half)
+    if (scan(0, 2 * nbig - (nbig && c % FT_BIG >= rule.min_rest && c % FT_BIG < FT_FULL ? 1 : 0)) < 2 * rule.min_tiles)
+        nbig = 0;                                                 // uniform: too few to fill the GPU
+    __syncthreads();
+    const int tbig = scan(0, nbig);
+    int rest = max(c - nbig * FT_BIG, 0);
+    int nsmall = rest > FT_MID && rest <= FT_SMALL ? 1 : 0, tsmall = scan(5, nsmall);
+    __syncthreads();
+    if (tsmall < rule.min_small)
     {
-        __syncthreads();
-        nbig = 0;
-        tbig = scan(0, 0);
+        nsmall = 0;
+        tsmall = scan(5, 0);
     }
-    const int rest = max(c - nbig * FT_BIG, 0), full = rest / FT_MID, r = rest % FT_MID;
+    else if (scan(1, nsmall ? 0 : (rest + FT_MID - 1) / FT_MID) <= rule.fold)
+    {
+        nsmall = rest > 0 && rest <= FT_SMALL ? 1 : 0;
+        tsmall = scan(5, nsmall);
+    }
+    if (nsmall) rest = 0;
+    const int full = rest / FT_MID, r = rest % FT_MID;
+    __syncthreads();
     const int t3 = scan(1, full + (r > 2 * GRP_ROWS ? 1 : 0));
     const int t2 = scan(2, r > GRP_ROWS && r <= 2 * GRP_ROWS ? 1 : 0);
     const int t1 = scan(3, r > 0 && r <= GRP_ROWS ? 1 : 0);
@@ -359,6 +393,7 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
         totals[0] = tbig;
         totals[1] = t3 + t2 + t1;
         totals[2] = tg;
+        totals[3] = tsmall;
     }
     __syncthreads();
     // entry j of list i belongs to the last expert whose sum is at most j (later experts without entries share it)
@@ -375,6 +410,11 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
     {
         const int o = owner(0, j), row0 = (j - s_off[0][o]) * FT_BIG;
         big[j] = FatTile{ o, row0, s_off[4][o] + row0 / GRP_ROWS, 0 };
+    }
+    for (int j = a; j < tsmall; j += FT_PLAN_MAX)
+    {
+        const int o = owner(5, j), row0 = (s_off[0][o + 1] - s_off[0][o]) * FT_BIG;
+        small[j] = FatTile{ o, row0, s_off[4][o] + row0 / GRP_ROWS, 0 };
     }
     for (int j = a; j < t3 + t2 + t1; j += FT_PLAN_MAX)
     {
@@ -1427,10 +1467,11 @@ struct FatWs
     size_t pws_bytes;
     ExpertRec* rec;       // [min(n, E)]
     FatTile* big;         // 256-route tiles
+    FatTile* small;       // 128-route tiles
     FatTile* mid;         // FT_MID-route tiles
     int2* groups;         // row groups: record, first row
-    int32_t* totals;      // [3] entries of the three lists
-    int max_big, max_mid, max_groups;
+    int32_t* totals;      // [4] entries of the lists
+    int max_big, max_small, max_mid, max_groups;
     uint16_t* xa;         // [max_groups][H / 32][2][GRP_HALVES]
     uint16_t* xd;         // [max_groups][I / 32][GRP_HALVES]
     float* xs;            // [max_groups][prep slices][2][GRP_ROWS] input sums
@@ -1446,18 +1487,20 @@ static FatWs fat_carve(void* base, int n, int E, int H, int I)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t na = (size_t)(n < E ? n : E);
     const size_t pwsb = mm_permute_workspace(n, E);
-    // an expert of c routes has at most c / FT_BIG_MIN 256-route tiles, c / FT_MID + 1 others and c / GRP_ROWS + 1 row
-    // groups
+    // an expert of c routes has at most c / min_rest 256-route tiles, one 128-route tile of more than FT_MID routes, c / FT_MID
+    // + 1 others and c / GRP_ROWS + 1 row groups
     FatWs w;
-    w.max_big = n / FT_BIG_MIN;
+    w.max_big = n / FT_REST_EXACT;
+    w.max_small = (int)na;
     w.max_mid = n / FT_MID + (int)na;
     w.max_groups = n / GRP_ROWS + (int)na;
     const size_t ng = (size_t)w.max_groups;
     w.nxs = (H / 128 + PREP_BLOCKS - 1) / PREP_BLOCKS;
-    constexpr int NS = 16;
+    constexpr int NS = 17;
     const size_t sizes[NS] = { al((size_t)(E + 1) * 4), al((size_t)(E + 2) * 4), al((size_t)n * 4), al((size_t)E * 4),
                                al(4), al(pwsb), al(na * sizeof(ExpertRec)), al(w.max_big * sizeof(FatTile)),
-                               al(w.max_mid * sizeof(FatTile)), al(ng * sizeof(int2)), al(12),
+                               al(w.max_small * sizeof(FatTile)),
+                               al(w.max_mid * sizeof(FatTile)), al(ng * sizeof(int2)), al(16),
                                al(ng * GRP_ROWS * 2 * H * 2), al(ng * GRP_ROWS * I * 2), al((size_t)n * H * 4),
                                al(ng * w.nxs * 2 * GRP_ROWS * 4), al(ng * (I / 128) * GRP_ROWS * 4) };
     char* p = static_cast<char*>(base);
@@ -1470,11 +1513,11 @@ static FatWs fat_carve(void* base, int n, int E, int H, int I)
     }
     w.counts = (int32_t*)at[0]; w.offsets = (int32_t*)at[1]; w.order = (int32_t*)at[2]; w.active = (int32_t*)at[3];
     w.nactive = (int32_t*)at[4]; w.pws = at[5]; w.pws_bytes = pwsb; w.rec = (ExpertRec*)at[6];
-    w.big = (FatTile*)at[7]; w.mid = (FatTile*)at[8]; w.groups = (int2*)at[9]; w.totals = (int32_t*)at[10];
-    w.xa = (uint16_t*)at[11]; w.xd = (uint16_t*)at[12]; w.Y = (float*)at[13];
-    w.xs = (float*)at[14]; w.xds = (float*)at[15];
+    w.big = (FatTile*)at[7]; w.small = (FatTile*)at[8]; w.mid = (FatTile*)at[9]; w.groups = (int2*)at[10];
+    w.totals = (int32_t*)at[11]; w.xa = (uint16_t*)at[12]; w.xd = (uint16_t*)at[13]; w.Y = (float*)at[14];
+    w.xs = (float*)at[15]; w.xds = (float*)at[16];
     w.plan_bytes = 0;
-    for (int i = 0; i < 11; ++i) w.plan_bytes += sizes[i];
+    for (int i = 0; i < 12; ++i) w.plan_bytes += sizes[i];
     w.bytes = off;
     return w;
 }
@@ -1498,16 +1541,25 @@ static int fat_check(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     return MM_OK;
 }
 
-// How a call's experts are taken: the fused call by the layer's codebook evaluation, the others with fp16-rounded weights.
+// How a call's experts are taken: the fused call by the layer's codebook evaluation, the others with fp16-rounded weights; the
+// whole calls may choose their tiles together, those of some experts of a layer by the expert alone.
+enum class FatCall { FUSED, WHOLE, EXPERTS };
 struct FatMode
 {
     bool exact;
-    BigRule rule;
+    TileRule rule;
 };
-static FatMode fat_mode(const mm_layer_t* L, bool fused)
+static FatMode fat_mode(const mm_layer_t* L, int n, FatCall call)
 {
-    if (!fused) return { true, BigRule{ 0, FT_BIG_ROWS } };
-    return { (L->flags & MM_LAYER_EXACT) != 0, BigRule{ (FT_BIG_WORK + L->I / 128 - 1) / (L->I / 128), 0 } };
+    const int units = L->I / 128, tiles = (FT_BIG_WORK + units - 1) / units;
+    switch (call)
+    {
+    case FatCall::FUSED: return { (L->flags & MM_LAYER_EXACT) != 0, TileRule{ tiles, 0, FT_REST, FT_NEVER, 0 } };
+    case FatCall::WHOLE: return { true, TileRule{ tiles, 0, FT_REST_EXACT, 2 * tiles, tiles / 2 } };
+    default:
+        if (n >= FT_LARGE && n / 200 >= L->E) return { true, TileRule{ 0, 0, FT_REST_EXACT, 0, FT_NEVER } };
+        return { true, TileRule{ 0, FT_BIG_ROWS, FT_REST, FT_NEVER, 0 } };
+    }
 }
 
 // Expert records, row groups and tile lists of the sorted positions in ws (counts, offsets, active, nactive filled).
@@ -1516,7 +1568,7 @@ static void fat_plan(const mm_layer_t* L, int n, int cap, const FatWs& ws, hipSt
     const int E = L->E, na = n < E ? n : E;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(1), dim3(FT_PLAN_MAX), 0, s, ws.counts, ws.offsets, ws.active, ws.nactive, L->gate_ptr,
-                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.mid, ws.groups, ws.totals, na, cap, mode.rule, choice, E, n);
+                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.small, ws.mid, ws.groups, ws.totals, na, cap, mode.rule, choice, E, n);
     };
     if (choice) launch(k_fat_plan<true>);
     else launch(k_fat_plan<false>);
@@ -1528,10 +1580,14 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
                      const FatWs& ws, hipStream_t s, bool yh, const FatMode& mode)
 {
     const bool exact = mode.exact;
-    hipLaunchKernelGGL(k_fat_prep, dim3((unsigned)ws.max_groups, (unsigned)ws.nxs),
-                       dim3(512), 0, s, x, x_dtype, ws.order, token_sorted, ws.rec, ws.groups, ws.totals + 2, L->suh13,
-                       ws.xa, ws.xs, topk, T, L->H);
-    // 256-route tiles a call of n routes can have
+    auto prep = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ws.max_groups, (unsigned)ws.nxs), dim3(512), 0, s, x, x_dtype, ws.order,
+                           token_sorted, ws.rec, ws.groups, ws.totals + 2, L->suh13, ws.xa, ws.xs, topk, T, L->H);
+    };
+    if (exact) prep(k_fat_prep<false>);
+    else prep(k_fat_prep<true>);
+    // 256-route and 128-route tiles a call of n routes can have
+    const int max_small = std::min(n / (FT_MID + 1), ws.max_small) >= mode.rule.min_small ? ws.max_small : 0;
     const int max_big = ws.max_big >= mode.rule.min_tiles && n >= mode.rule.min_rows ? ws.max_big : 0;
     auto grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles * units + 7) & ~(size_t)7)); };    // >= 8 per_xcd
     auto mid_grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles + 7) / 8 * 8 * units)); };
@@ -1540,21 +1596,30 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     FatArgs gm = g;
     gm.tiles = ws.mid;
     gm.ntiles = ws.totals + 1;
+    FatArgs gs = g;
+    gs.tiles = ws.small;
+    gs.ntiles = ws.totals + 3;
     FatArgs d = g;
     d.xa = ws.xd; d.K = L->I; d.N = L->H; d.nunits = L->H / 256;
     d.xs = ws.xds; d.nxs = g.nxds;
     FatArgs dm = d;
     dm.tiles = ws.mid;
     dm.ntiles = ws.totals + 1;
+    FatArgs ds = d;
+    ds.tiles = ws.small;
+    ds.ntiles = ws.totals + 3;
     // gate/up: 256-route tiles on the 8-wave kernel, down on the 16-wave kernel (same bits; measured on the 16k layer:
     // gate/up equal, down 2.76-2.85 against 2.92-2.94 ms)
     if (max_big > 0) hipLaunchKernelGGL((k_fat<0, FT_BIG / 32>), grid(max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
+    if (max_small > 0) hipLaunchKernelGGL((k_fat16<0, FT_SMALL / 64>), grid(max_small, g.nunits), dim3(FT16_THREADS), 0, s, gs);
     if (exact) hipLaunchKernelGGL((k_mid<0, true>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
     else hipLaunchKernelGGL((k_mid<0, false>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
     if (yh)
     {
         if (max_big > 0)
             hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64, true>), grid(max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
+        if (max_small > 0)
+            hipLaunchKernelGGL((k_fat16<1, FT_SMALL / 64, true>), grid(max_small, d.nunits), dim3(FT16_THREADS), 0, s, ds);
         if (exact) hipLaunchKernelGGL((k_mid<1, true, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
         else hipLaunchKernelGGL((k_mid<1, false, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
     }
@@ -1562,6 +1627,8 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     {
         if (max_big > 0)
             hipLaunchKernelGGL((k_fat16<1, FT_BIG / 64>), grid(max_big, d.nunits), dim3(FT16_THREADS), 0, s, d);
+        if (max_small > 0)
+            hipLaunchKernelGGL((k_fat16<1, FT_SMALL / 64>), grid(max_small, d.nunits), dim3(FT16_THREADS), 0, s, ds);
         if (exact) hipLaunchKernelGGL((k_mid<1, true>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
         else hipLaunchKernelGGL((k_mid<1, false>), mid_grid(ws.max_mid, d.nunits), dim3(256), 0, s, dm);
     }
@@ -1570,13 +1637,13 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
 
 // Permutation, plan, input transform and both GEMMs: Y rows of every route whose expert has more than cap routes.
 static int fat_run(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, int cap,
-                   const FatWs& ws, hipStream_t s, bool yh, bool fused)
+                   const FatWs& ws, hipStream_t s, bool yh, FatCall call)
 {
     const int n = T * topk, E = L->E;
     int rc = permute_launch(ids, nullptr, n, topk, E, ws.counts, ws.offsets, ws.order, nullptr, nullptr, nullptr,
                             ws.active, ws.nactive, nullptr, ws.pws, ws.pws_bytes, s);
     if (rc) return rc;
-    const FatMode mode = fat_mode(L, fused);
+    const FatMode mode = fat_mode(L, n, call);
     fat_plan(L, n, cap, ws, s, mode, nullptr);
     return fat_gemms(L, x, x_dtype, T, topk, nullptr, n, ws, s, yh, mode);
 }
@@ -1592,9 +1659,9 @@ static int fat_combine(const mm_layer_t* L, int T, int topk, const int64_t* ids,
 
 // fat_run and the weighted combine of its rows.
 static int fat_layer(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
-                     int cap, int accumulate, float* out, const FatWs& ws, hipStream_t s, bool fused)
+                     int cap, int accumulate, float* out, const FatWs& ws, hipStream_t s, FatCall call)
 {
-    const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true, fused);
+    const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true, call);
     return r ? r : fat_combine(L, T, topk, ids, w, cap, accumulate, out, ws, s, nullptr);
 }
 
@@ -1712,12 +1779,13 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
         return moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, workspace, workspace_bytes, stream,
                                  "mm_fused_moe");
     if (path == FusedPath::GEMM)
-        return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I), s, true);
+        return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I), s,
+                         FatCall::FUSED);
     const FusedWs ws = fused_carve(workspace, n, E, L->H, L->I);
     int r = permute_launch(ids, nullptr, n, topk, E, ws.f.counts, ws.f.offsets, ws.f.order, nullptr, nullptr, nullptr,
                            ws.f.active, ws.f.nactive, nullptr, ws.f.pws, ws.f.pws_bytes, s);
     if (r) return r;
-    const FatMode mode = fat_mode(L, true);
+    const FatMode mode = fat_mode(L, n, FatCall::FUSED);
     fat_plan(L, n, 0, ws.f, s, mode, ws.choice);
     // the decode path's launches first: the grouped GEMM's inputs lie over their workspace
     r = moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, ws.dws, ws.dws_bytes, stream, "mm_fused_moe",
@@ -1742,7 +1810,7 @@ int mm_grouped_gemm(const mm_layer_t* L, const void* x, int x_dtype, int T, int 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     FatWs ws = fat_carve(workspace, T * topk, L->E, L->H, L->I);
     ws.Y = Y;
-    return fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, false, false);
+    return fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, false, FatCall::WHOLE);
 }
 
 int mm_moe_prefill(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1752,7 +1820,7 @@ int mm_moe_prefill(const mm_layer_t* L, const void* x, int x_dtype, int T, int t
     if (rc) return rc;
     MM_CHECK_ARG(w && out && cap >= 0, "mm_moe_prefill: null pointer or negative cap");
     return fat_layer(L, x, x_dtype, T, topk, ids, w, cap, accumulate, out, fat_carve(workspace, T * topk, L->E, L->H, L->I),
-                     reinterpret_cast<hipStream_t>(stream), false);
+                     reinterpret_cast<hipStream_t>(stream), FatCall::WHOLE);
 }
 
 size_t mm_fat_batched_workspace(int n, int T, int E, int H, int I)
@@ -1790,7 +1858,7 @@ int mm_fat_batched(const mm_layer_t* L, const void* x, int x_dtype, int T, int n
     hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)std::min((T + 255) / 256, 1024)), dim3(256), 0, s, ws.tcount, T, 0);
     hipLaunchKernelGGL(k_fatb_tokens<1>, dim3(pg), dim3(256), 0, s, token_sorted, ws.f.counts, ws.f.offsets, ws.f.order,
                        ws.tcount, ws.toff, ws.tpos, T, E, n);
-    const FatMode mode = fat_mode(L, false);
+    const FatMode mode = fat_mode(L, n, FatCall::EXPERTS);
     fat_plan(L, n, cap, ws.f, s, mode, nullptr);
     int r = fat_gemms(L, x, x_dtype, T, 1, token_sorted, n, ws.f, s, true, mode);
     if (r) return r;

@@ -254,22 +254,24 @@ def test_row_group_tiles_at_their_edges(dev, exact):
             assert ok, (name, counts[e], m)
 
 
-def test_full_tiles_of_a_large_call(dev):
+@pytest.mark.parametrize("exact", [True, False])
+def test_full_tiles_of_a_large_call(dev, exact):
     """Enough 256-route tiles to take their own kernels (at least three rounds of 256 workgroups of them), with remainders
-    of one route, of one and of two row groups, and partial tiles of 193 and 255 routes: sampled rows of every expert."""
+    of one route, of one and of two row groups, and partial tiles of 193 and 255 routes: sampled rows of every expert. In a
+    layer without MM_LAYER_EXACT the 256-route tiles round the weights and write no input sums, the others need them."""
     import torch
     from mi355moe import moe
     H, I, seed = 256, 2048, 8282
     counts = [193, 255, 256, 257, 290, 330] * 9
     E = len(counts)
     assert sum(c // 256 + (c % 256 >= 193) for c in counts) * (I // 128) >= 3 * 256
-    st = make_store(E, H, I, seed, device=dev, exact=True)
+    st = make_store(E, H, I, seed, device=dev, exact=exact)
     rng = np.random.default_rng(14)
     ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
     T = ids.shape[0]
     w = np.ones((T, 1), np.float32)
     x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
-    print(f"full tiles T={T}", flush=True)
+    print(f"full tiles T={T} exact={exact}", flush=True)
     out = moe.fused_moe(st, _t(x16, dev), _t(ids, dev), _t(w, dev), 32)
     torch.cuda.synchronize()
     rows = np.concatenate([np.flatnonzero(ids[:, 0] == e)[[0, 100, 192, -1]] for e in range(E)])
@@ -351,3 +353,131 @@ def test_fused_call_chosen_on_the_device_in_a_graph(dev):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), f"replay {step}"
+
+
+@pytest.mark.parametrize("more", [[], [1, 17, 32, 33, 64, 95, 96] * 2], ids=["folded", "all_sizes"])
+def test_tiles_of_a_whole_rounding_call(dev, more):
+    """Tiles of mm_grouped_gemm and mm_moe_prefill calls with many busy experts: remainders of 97 to 128 routes in 128-route
+    tiles, from 129 routes on in 256-route tiles (129, 176, 177, 255 and full ones, with remainders of 1, 96, 97 and 128
+    after them), and the shorter ones in 128-route tiles too where they are few, else in tiles of their own. Sampled rows of
+    every expert of both entries, whose rows are the same bits."""
+    import torch
+    from mi355moe import moe
+    H, I, seed = 256, 4096, 8383
+    tiles = -(-768 // (I // 128))                                   # three rounds of 256 workgroups
+    counts = [97, 112, 113, 128] * (tiles // 2) + [129, 176, 177, 255, 256, 257, 352, 353, 384] * 4 + [31, 32, 96] + more
+    rest = [c % 256 for c in counts]
+    assert sum(96 < r <= 128 for r in rest) >= 2 * tiles
+    assert sum(2 * (c // 256) + (r >= 129) + (r >= 177) for c, r in zip(counts, rest)) >= 2 * tiles
+    assert (sum(0 < r <= 96 for r in rest) <= tiles // 2) == (not more)
+    E = len(counts)
+    st = make_store(E, H, I, seed, device=dev, exact=True)
+    rng = np.random.default_rng(16)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
+    T = ids.shape[0]
+    w = np.ones((T, 1), np.float32)
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    print(f"whole call tiles T={T} experts={E}", flush=True)
+    Y = moe.grouped_gemm(st, _t(x16, dev), _t(ids, dev), cap=0)
+    out = moe.moe_prefill(st, _t(x16, dev), _t(ids, dev), _t(w, dev))
+    torch.cuda.synchronize()
+    assert torch.equal(Y.half(), out.half())                        # the layer's rows pass through fp16
+    at = [np.flatnonzero(ids[:, 0] == e) for e in range(E)]
+    rows = np.concatenate([r[np.unique([0, len(r) // 2, min(96, len(r) - 1), min(128, len(r) - 1), len(r) - 1])] for r in at])
+    ref = OracleLayer(st, seed).forward(x16[rows].astype(np.float32), ids[rows], w[rows])
+    ok, m = within_tolerance(Y.cpu().numpy()[rows], ref)
+    assert ok, m
+
+
+def test_tiles_of_sorted_experts(dev):
+    """apply_exl3_batched_fat takes 256-route tiles by the expert's own routes, from 768 on: 767 to 1,025 routes, every row
+    against the oracle, and an expert computed alone has the bits it has among the others."""
+    import torch
+    from mi355moe import exl3, moe
+    H, I, seed = 512, 256, 8484
+    counts = [767, 768, 769, 960, 961, 1025]
+    E = len(counts)
+    st = make_store(E, H, I, seed, device=dev, exact=True)
+    rng = np.random.default_rng(17)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
+    T = ids.shape[0]
+    w = np.ones((T, 1), np.float32)
+    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
+    xd = _t(x16, dev)
+    r = moe.permute(_t(ids, dev), _t(w, dev), 1, E)
+    tok, wts = r["token_sorted"].long(), r["weight_sorted"].half()
+    print(f"sorted experts T={T}", flush=True)
+
+    def run(skip):
+        o = torch.zeros((T, H), dtype=torch.float32, device=dev)
+        return exl3.apply_exl3_batched_fat(xd, tok, wts, counts, None, 10.0, 0, o, skip=skip, layer=st)
+
+    out = run(None)
+    alone = sum(run(set(range(E)) - {e}) for e in range(E))
+    torch.cuda.synchronize()
+    assert torch.equal(out, alone)
+    ref = OracleLayer(st, seed).forward(x16.astype(np.float32), ids, w)
+    for e in range(E):
+        rows = ids[:, 0] == e
+        ok, m = within_tolerance(out.cpu().numpy()[rows], ref[rows])
+        assert ok, (counts[e], m)
+
+
+def test_tiles_of_sorted_experts_of_a_large_layer(dev):
+    """apply_exl3_batched_fat of a layer with at least 80,000 routes and 200 per expert: every remainder in 256- or 128-route
+    tiles (1, 96, 97, 128, 129 and 255 routes among them); sampled rows of every expert against the oracle, and experts
+    computed alone have the bits they have among the others."""
+    import torch
+    from mi355moe import exl3, moe
+    H, I, seed = 256, 128, 8585
+    counts = [1, 96, 97, 128, 129, 255, 256 + 1, 256 + 128, 512 + 129]
+    counts.append(80000 - sum(counts))
+    E = len(counts)
+    st = make_store(E, H, I, seed, device=dev, exact=True)
+    rng = np.random.default_rng(18)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
+    T = ids.shape[0]
+    xd = torch.randn((T, H), generator=torch.Generator(device=dev).manual_seed(18), device=dev).half()
+    w = torch.ones((T, 1), device=dev)
+    r = moe.permute(_t(ids, dev), w, 1, E)
+    tok, wts = r["token_sorted"].long(), r["weight_sorted"].half()
+    print(f"sorted experts of a large layer T={T}", flush=True)
+
+    def run(skip):
+        o = torch.zeros((T, H), dtype=torch.float32, device=dev)
+        return exl3.apply_exl3_batched_fat(xd, tok, wts, counts, None, 10.0, 0, o, skip=skip, layer=st)
+
+    out = run(None)
+    parts = sum(run(set(range(E)) - set(b)) for b in ([0, 3], [1, 9], [2], [4, 5, 6], [7, 8]))
+    torch.cuda.synchronize()
+    assert torch.equal(out, parts)
+    rows = np.concatenate([np.flatnonzero(ids[:, 0] == e)[np.unique([0, c // 2, c - 1])] for e, c in enumerate(counts)])
+    ref = OracleLayer(st, seed).forward(xd[_t(rows, dev)].float().cpu().numpy(), ids[rows], np.ones((len(rows), 1), np.float32))
+    ok, m = within_tolerance(out.cpu().numpy()[rows], ref)
+    assert ok, m
+
+
+def test_full_tiles_match_reference_golden(dev):
+    """The compiled reference's golden experts with 800 routes each (three 256-route tiles and a row group) through
+    apply_exl3_batched_fat: every route's row equals the reference's output."""
+    import torch
+    from mi355moe import exl3
+    g = np.load(os.path.join(GOLD, "expert_4096x2048.npz"), allow_pickle=False)
+    H, I, R = int(g["H"]), int(g["I"]), 800
+    st = make_store(256, H, I, int(g["layer_seed"]), device=dev, exact=True)
+    es = [int(g["e0"]), int(g["e1"])]
+    for j, e in enumerate(es):
+        st.w13_suh[e, 0].copy_(_t(g[f"suh_g{j}"], dev)); st.w13_svh[e, 0].copy_(_t(g[f"svh_g{j}"], dev))
+        st.w13_suh[e, 1].copy_(_t(g[f"suh_u{j}"], dev)); st.w13_svh[e, 1].copy_(_t(g[f"svh_u{j}"], dev))
+        st.w2_suh[e].copy_(_t(g[f"suh_d{j}"], dev)); st.w2_svh[e].copy_(_t(g[f"svh_d{j}"], dev))
+    x = _t(np.stack([g["x0"], g["x1"]]).repeat(R, 0).astype(np.float16), dev)
+    order = sorted((0, 1), key=lambda j: es[j])
+    tok = torch.cat([torch.arange(j * R, (j + 1) * R, device=dev) for j in order])
+    counts = [R if e in es else 0 for e in range(256)]
+    out = torch.zeros((2 * R, H), dtype=torch.float32, device=dev)
+    print("golden experts in full tiles", flush=True)
+    exl3.apply_exl3_batched_fat(x, tok, torch.ones(2 * R, device=dev).half(), counts, None, 10.0, 0, out, layer=st)
+    torch.cuda.synchronize()
+    for j in (0, 1):
+        ok, m = within_tolerance(out.cpu().numpy()[j * R:(j + 1) * R], np.repeat(g[f"y{j}_lim10"][None, :], R, 0))
+        assert ok, (j, m)
