@@ -137,6 +137,9 @@ void launch_route_prep(const PrepArgs& p, hipStream_t s);
 
 constexpr int GV_ROUTE_MAX = 1024;    // in-kernel routing limit of the decode path (routes per call)
 
+// Bytes that hold the decode workspace of every call of up to n routes.
+size_t decode_workspace_upto(int n, int E, int H, int I);
+
 // Whether the decode path can address n routes over E experts.
 bool decode_fits(int n, int E, int H, int I);
 

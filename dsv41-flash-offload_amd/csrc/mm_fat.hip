@@ -1709,11 +1709,15 @@ static FatbWs fatb_carve(void* base, int n, int T, int E, int H, int I)
 // 2^30: 512 experts, H 2048, I 512, 2,500 routes take 290 us on the grouped GEMM and 330 chosen). With more routes the experts
 // are busy enough for the grouped GEMM.
 enum class FusedPath { DECODE, CHOICE, GEMM };
+static int fused_most_decode(int E) { return std::min(GV_ROUTE_MAX, std::max(384, 10 * E)); }
+static int fused_most_choice(int E, int H, int I)
+{
+    return (int64_t)E * H * I >= (int64_t)1 << 30 ? std::min(9 * E, std::max(7 * E, 1280)) : 0;
+}
 static FusedPath fused_path(int n, int E, int H, int I)
 {
-    if (n <= GV_ROUTE_MAX) return n <= std::max(384, 10 * E) ? FusedPath::DECODE : FusedPath::GEMM;
-    const bool few = n <= std::min(9 * E, std::max(7 * E, 1280)), large = (int64_t)E * H * I >= (int64_t)1 << 30;
-    return few && large && decode_fits(n, E, H, I) ? FusedPath::CHOICE : FusedPath::GEMM;
+    if (n <= GV_ROUTE_MAX) return n <= fused_most_decode(E) ? FusedPath::DECODE : FusedPath::GEMM;
+    return n <= fused_most_choice(E, H, I) && decode_fits(n, E, H, I) ? FusedPath::CHOICE : FusedPath::GEMM;
 }
 
 // Workspace of a call that either path may take: the grouped GEMM's, with the decode workspace over its inputs and rows (one of
@@ -1727,17 +1731,28 @@ struct FusedWs
     size_t bytes;
 };
 
-static FusedWs fused_carve(void* base, int n, int E, int H, int I)
+static FusedWs fused_carve(void* base, int n, int E, int H, int I, size_t decode_bytes)
 {
     FusedWs w;
     w.f = fat_carve(base, n, E, H, I);
-    w.dws_bytes = mm_gemv_workspace(n, E, H, I);
+    w.dws_bytes = decode_bytes;
     const size_t most = std::max(w.f.bytes, w.f.plan_bytes + w.dws_bytes);      // multiples of 256
     char* p = static_cast<char*>(base);
     w.dws = p ? p + w.f.plan_bytes : nullptr;
     w.choice = p ? (int32_t*)(p + most) : nullptr;
     w.bytes = most + 256;
     return w;
+}
+
+// Bytes a call of n routes needs.
+static size_t fused_bytes(int n, int E, int H, int I)
+{
+    switch (fused_path(n, E, H, I))
+    {
+    case FusedPath::DECODE: return mm_gemv_workspace(n, E, H, I);
+    case FusedPath::CHOICE: return fused_carve(nullptr, n, E, H, I, mm_gemv_workspace(n, E, H, I)).bytes;
+    default: return fat_carve(nullptr, n, E, H, I).bytes;
+    }
 }
 
 }  // namespace mm
@@ -1750,12 +1765,12 @@ size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap)
 {
     if (T <= 0 || topk <= 0 || E <= 0 || H <= 0 || I <= 0 || cap < 0) return 0;
     const int n = T * topk;
-    switch (fused_path(n, E, H, I))
-    {
-    case FusedPath::DECODE: return mm_gemv_workspace(n, E, H, I);
-    case FusedPath::CHOICE: return fused_carve(nullptr, n, E, H, I).bytes;
-    default: return fat_carve(nullptr, n, E, H, I).bytes;
-    }
+    // enough for every smaller call too, whichever path it takes
+    size_t bytes = decode_workspace_upto(std::min(n, fused_most_decode(E)), E, H, I);
+    const int choice = std::min(n, fused_most_choice(E, H, I));
+    if (choice > GV_ROUTE_MAX)
+        bytes = std::max(bytes, fused_carve(nullptr, choice, E, H, I, decode_workspace_upto(choice, E, H, I)).bytes);
+    return n > fused_most_decode(E) ? std::max(bytes, fat_carve(nullptr, n, E, H, I).bytes) : bytes;
 }
 
 int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1770,7 +1785,7 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
     const size_t npos = n <= GV_ROUTE_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
     MM_CHECK_ARG(npos * 2 * std::max(L->H, L->I) * 2 < ((size_t)1 << 31),
                  "mm_fused_moe: too many decode-path positions (%zu)", npos);
-    const size_t need = mm_fused_moe_workspace(T, topk, E, L->H, L->I, cap);
+    const size_t need = fused_bytes(n, E, L->H, L->I);
     MM_CHECK_ARG(workspace && workspace_bytes >= need, "mm_fused_moe: workspace too small (%zu < %zu)", workspace_bytes,
                  need);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -1781,7 +1796,7 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
     if (path == FusedPath::GEMM)
         return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I), s,
                          FatCall::FUSED);
-    const FusedWs ws = fused_carve(workspace, n, E, L->H, L->I);
+    const FusedWs ws = fused_carve(workspace, n, E, L->H, L->I, mm_gemv_workspace(n, E, L->H, L->I));
     int r = permute_launch(ids, nullptr, n, topk, E, ws.f.counts, ws.f.offsets, ws.f.order, nullptr, nullptr, nullptr,
                            ws.f.active, ws.f.nactive, nullptr, ws.f.pws, ws.f.pws_bytes, s);
     if (r) return r;

@@ -900,18 +900,19 @@ static bool split_records(const mm_layer_t* L, int n, int topk)
     return n > REC_ROUTES * topk && rows_fit(L->H, L->I, max_records(n, L->E));
 }
 
-// Workspace of n routes whose sorted positions lie below npos (npos = n unless a caller bounds the positions).
-static Ws carve(void* base, int n, int npos, int E, int H, int I)
+// Workspace of n routes whose sorted positions lie below npos (npos = n unless a caller bounds the positions), with room for
+// `pieces` x 1 route of partial sums.
+static Ws carve(void* base, int n, int npos, int E, int H, int I, size_t pieces)
 {
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t m = (size_t)npos;
-    const size_t na = (size_t)max_records(npos, E), cap = (size_t)piece_cap(npos);
+    const size_t na = (size_t)max_records(npos, E);
     // the small routing arrays first and together (records, counts, pos_of, route_at, e_at, ai_at, ai_of), so the
     // epilogues' first loads fall in the same few pages
     const size_t sizes[13] = { al(na * sizeof(ExpertRec)), al(2 * 4), al((size_t)n * 4), al(m * 4),
                                al(m * 4), al(m * 4), al((size_t)n * 4), al(m * 2 * H * 2),
-                               al(m * 2 * prep_blocks(H) * 4), al(cap * m * 2 * I * 4), al(m * I * 2),
-                               al(m * (I / GV_COLS) * 4), al(cap * m * H * 4) };
+                               al(m * 2 * prep_blocks(H) * 4), al(pieces * 2 * I * 4), al(m * I * 2),
+                               al(m * (I / GV_COLS) * 4), al(pieces * H * 4) };
     char* p = static_cast<char*>(base);
     char* at[13];
     size_t off = 0;
@@ -936,6 +937,16 @@ static Ws carve(void* base, int n, int npos, int E, int H, int I)
     w.part_d = reinterpret_cast<float*>(at[12]);
     w.bytes = off;
     return w;
+}
+static Ws carve(void* base, int n, int npos, int E, int H, int I)
+{
+    return carve(base, n, npos, E, H, I, (size_t)piece_cap(npos) * npos);
+}
+
+// Bytes that hold the decode workspace of every call of up to n routes (piece_cap(m) m is at most 32 m, 8192 or 4 m).
+size_t decode_workspace_upto(int n, int E, int H, int I)
+{
+    return carve(nullptr, n, n, E, H, I, n <= 256 ? (size_t)32 * n : (size_t)std::max(8192, 4 * n)).bytes;
 }
 
 // Waves of one partial launch: the whole GPU once (WAVES_PER_CU per CU, a multiple of 8 workgroups), or half of

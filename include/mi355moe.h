@@ -210,7 +210,8 @@ int mm_moe_prefill(const mm_layer_t* layer, const void* x, int x_dtype, int T, i
  * bounds the call's size as before: n, or E x cap of more than 1,024, transformed inputs below 2 GiB. Weights follow the
  * layer's codebook evaluation (MM_LAYER_EXACT or not), except in tiles of 256 routes, which round them to fp16 as the
  * reference's reconstruct does. No host synchronisation: the call can be captured. ids int64 [T*topk], w fp32 [T*topk],
- * topk <= 16, cap >= 1; x as for mm_moe_prefill. Workspace: mm_fused_moe_workspace(T, topk, E, H, I, cap) bytes. */
+ * topk <= 16, cap >= 1; x as for mm_moe_prefill. Workspace: mm_fused_moe_workspace(T, topk, E, H, I, cap)
+ * bytes, which also hold every call of fewer tokens. */
 size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap);
 int mm_fused_moe(const mm_layer_t* layer, const void* x, int x_dtype, int T, int topk, const int64_t* ids,
                  const float* w, int cap, float* out, void* workspace, size_t workspace_bytes, mm_stream_t stream);

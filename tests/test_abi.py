@@ -83,6 +83,25 @@ def test_route_limit_counts_one_record_per_expert():
     assert rc == -1 and b"workspace too small" in L.mm_last_error(), L.mm_last_error()
 
 
+@pytest.mark.parametrize("E,H,I,k", [(384, 4096, 2048, 8), (384, 5120, 2304, 6), (8, 4096, 2048, 2), (64, 4096, 2048, 6),
+                                     (32, 1024, 512, 4), (4, 256, 128, 1), (1024, 1024, 1024, 1)])
+def test_fused_workspace_holds_every_smaller_call(E, H, I, k):
+    """mm_fused_moe_workspace grows with the tokens, and is at least what a call asks for (read from the argument error of a
+    call without any), on both sides of every change of path."""
+    import ctypes
+    from mi355moe import _lib
+    L = _lib.load()
+    lay = _lib.MMLayer(*([256] * 7), E, H, I, 10.0, 0)
+    had = 0
+    for T in sorted(set(range(1, 3000, 7)) | {384 // k, 384 // k + 1, 1024 // k, 1024 // k + 1}):
+        rc = L.mm_fused_moe(ctypes.byref(lay), 256, 0, T, k, 256, 256, 32, 256, 256, 0, None)
+        m = re.search(rb"workspace too small \(0 < (\d+)\)", L.mm_last_error())
+        assert rc == -1 and m, L.mm_last_error()
+        ws = L.mm_fused_moe_workspace(T, k, E, H, I, 32)
+        assert ws >= int(m.group(1)) and ws >= had, T
+        had = ws
+
+
 def test_expert_seed_matches_oracle():
     import oracle as O
     from mi355moe import _lib
