@@ -101,13 +101,13 @@ struct PrepArgs
     const int64_t* wtab1;
     const int64_t* wtab2;
     const uint16_t* suh13;    // [E][2][H]
-    ExpertRec* rec;           // [max_active]
-    int32_t* counts;          // [2]: active experts, routed (valid) routes
+    ExpertRec* rec;           // experts' records
+    int32_t* counts;          // [2]: records, routed (valid) routes
     int32_t* pos_of;          // [n] sorted position of each route, -1 if its id is outside [0, E)
     int32_t* route_at;        // [n] route at each sorted position
     int32_t* e_at;            // [n] expert at each sorted position
-    int32_t* ai_at;           // [n] active index (record) of the expert at each sorted position
-    int32_t* ai_of;           // [n] active index of each route's expert
+    int32_t* ai_at;           // [n] record of each sorted position
+    int32_t* ai_of;           // [n] record of each route
     uint16_t* xa;             // [n][2][H] fp16 in operand order
     float* xsum;              // [n][2][nb] sums of xa over each workgroup's rows
     int n, topk, E, H, nb, x_dtype, rescale;
@@ -115,8 +115,6 @@ struct PrepArgs
     int split;                // records of 16 routes instead of one per expert
     int walk;                 // with split: one workgroup per route and matrix takes all its input rows
     int gated;                // no routed position: only counts are written (0, 0)
-    int npos;                 // sorted positions visited (n with in-kernel routing; the permutation's valid
-                              // positions must lie below it)
 };
 
 __device__ __forceinline__ int wave_sum_int(int v)

@@ -4,14 +4,15 @@
 // 128x128 GEMM).
 //
 // Launches: mm_permute (sorted positions) -> k_fat_plan (expert records, row groups, tile lists) -> k_fat_prep
-// (transformed inputs per row group) -> k_fat<0, 8>, k_mid<0> (gate/up) -> k_fat16<1, 4>, k_mid<1> (down) -> k_fat_combine.
+// (transformed inputs per row group) -> k_fat, k_fat16<0, 2>, k_mid<0> (gate/up) -> k_fat16<1, 4>, k_fat16<1, 2>, k_mid<1>
+// (down) -> k_fat_combine; a tile size that the call cannot have is not launched.
 //
 // An expert's routes (sorted positions) are taken in row groups of 32, whose inputs are stored in MFMA operand order: per
 // matrix and 32-element step one contiguous 2 KB, chunk g (8 elements: tile rows 0 and 1 of decode window g) of row r at
 // 16 (32 g + r). A wave's operand load is then one contiguous KB, whichever kernel reads it.
 //
 // k_mid takes tiles of at most 96 routes (below). k_fat (8 waves, two per SIMD) and k_fat16 (16 waves) own a tile of 256
-// routes of one expert x 256 output columns, for calls with many of them:
+// (k_fat16 also 128) routes of one expert x 256 output columns, for calls with many of them:
 //   gate/up (MODE 0): gate columns 128 c .. 128 c + 127 and the same up columns, so the epilogue holds both and
 //                     applies the output transforms, SwiGLU and the down-input transform of that 128-block (the
 //                     transforms act within 128-blocks);
@@ -37,36 +38,30 @@ constexpr int FT_SMALL = 128;       // routes per tile of k_fat16<*, 2>
 // Which tiles an expert's routes take. Tiles of 256 routes (and of 128, where the weights are rounded) cost the least per route
 // once there are several rounds of workgroups of them (one fits a CU), FT_MID-route tiles leave fewer CUs idle before that and
 // fewer rows empty. The kernels of the tile sizes add an expert's products in different orders, except those of 256 and 128.
-//   a fused call (FatCall::FUSED): 256-route tiles where it has at least three rounds (FT_BIG_WORK workgroups) of them, the
-//     rest in FT_MID-route tiles. 3 tiles (48 workgroups) of a 512-token call took 214 us of its 1,540 where FT_MID-route tiles
-//     took 60; at 64 tiles (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at 297 (16,384 tokens) 8.25 and 8.65.
-//   a whole call with rounded weights (WHOLE): the same, but from a remainder of 129 routes on, and the remainders of 97 to 128
-//     routes in 128-route tiles from six rounds of them on; then the shorter ones too, if they are under one and a half rounds
-//     (a launch of a few k_mid workgroups takes 99 + 50 us). k_mid costs more with rounded weights (55 against 34 ns per 16 x 16
-//     tile and SIMD). mm_moe_prefill, FT_MID-route tiles for experts below 768 routes / this, ms: H 5120, 16,384 tokens 10.91 /
-//     10.47 (64 hot experts), 10.94 / 10.05 (even routing); 8,192 6.51 / 6.10 (even); H 4096, 16,384 10.50 / 9.60 (even), 8,192 5.49 /
-//     5.33 (even); 4,096 tokens on 170 experts 2.85 / 2.58, on 64 2.60 / 2.26. A 256-route tile of fewer than FT_FULL routes counts
-//     half: 64 of 154 routes (2,048 tokens) take 2.29 ms a call, as FT_MID-route tiles 2.22.
-//   some experts of a layer (EXPERTS; mm_fat_batched), whose rows must have the same bits whichever others the call computes (a
-//     layer in one call or in staging batches): by the expert's own routes and the size of the layer's call. From 768 routes on 256-route
-//     tiles: a staging batch of 16 experts holds few (12 took 189 us of its 470, as FT_MID-route tiles 50). In layers of more than
-//     FT_LARGE routes and 200 per expert every expert takes 256- and 128-route tiles, as many staged experts then do (16 of a
-//     16,384-token call, H 4096: 840 us without, 775 with; the whole call at H 5120 10.9 and 10.4 ms).
+//   a fused call: 256-route tiles where it has at least three rounds (FT_BIG_WORK workgroups) of them, the rest in FT_MID-route
+//     tiles. 3 tiles (48 workgroups) of a 512-token call took 214 us of its 1,540 where FT_MID-route tiles took 60; at 64 tiles
+//     (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at 297 (16,384 tokens) 8.25 and 8.65.
+//   the other entry points, whose rows must have the same bits whichever experts of a layer a call computes (a layer in one call
+//     or in staging batches): by the expert's routes and the layer's. From 768 routes on 256-route tiles: a staging batch of 16 experts
+//     holds few (12 took 189 us of its 470, as FT_MID-route tiles 50). In layers of more than FT_LARGE routes and 200 per
+//     expert, from a remainder of 129 routes on, and remainders of 97 to 128 routes in 128-route tiles (k_mid costs more with
+//     rounded weights, 55 against 34 ns per 16 x 16 tile and SIMD); the shorter ones too where the layer has under one and a
+//     half rounds of them (a launch of a few k_mid workgroups takes 99 + 50 us). mm_moe_prefill of 16,384 tokens by the first / by this
+//     rule, ms: H 5120 10.91 / 10.35 (64 hot experts), 10.94 / 10.05 (even routing), H 4096 10.50 / 9.60 (even); 16 staged experts
+//     0.84 / 0.73. At 8,192 tokens staged experts take 0.48 ms by the first rule and 0.55 by this, the whole layer 5.5 and 5.3.
 struct TileRule
 {
     int min_tiles;      // 256-route tiles of the call
     int min_rows;       // routes of an expert that takes them
     int min_rest;       // remainder of c / 256 that takes one more
-    int min_small;      // 128-route tiles of the call
-    int fold;           // FT_MID-route tiles of up to 128 routes that go with them
+    int min_small;      // smallest remainder in a 128-route tile
+    int fold;           // the shorter remainders of the layer that go with them
 };
 constexpr int FT_BIG_WORK = 3 * 256;
 constexpr int FT_BIG_ROWS = 3 * FT_BIG;
 constexpr int FT_REST = 193;        // two FT_MID tiles hold 192
-constexpr int FT_REST_EXACT = 129;
-constexpr int FT_FULL = 177;
+constexpr int FT_REST_LARGE = 129;
 constexpr int FT_LARGE = 80000;
-constexpr int FT_NEVER = 0x3fffffff;
 constexpr int GRP_ROWS = 32;        // rows of a row group
 constexpr int GRP_HALVES = 1024;    // one matrix's 32-element step of a row group
 // 128-blocks per input transform workgroup (16,384 tokens, H 4096, 2.3 GB written: 783 us with 2, 844 with 4, 946 with 8;
@@ -105,15 +100,12 @@ struct FatArgs
     float limit;
 };
 
-// Transformed inputs of every fat route, one workgroup per sorted position: r16(FWHT(x16 * suh_m) * HAD) per
-// 128-block (ft_core.h:96-102), where x16 is fp16 input as is, or bf16 / fp32 input rounded through bf16. Row pos
-// of xa holds, per 32-element step, the gate step then the up step in operand order (128 bytes: one cache line
-// per step, which the gate/up kernel loads whole).
+// Transformed inputs of every fat route (k_fat_prep): r16(FWHT(x16 * suh_m) * HAD) per 128-block (ft_core.h:96-102),
+// where x16 is fp16 input as is, or bf16 / fp32 input rounded through bf16, in the row groups described above.
 //
-// Wave w transforms matrix w >> 1, blocks (w & 1) * nb / 2 .. , four blocks at a time, 16 lanes per block and
-// 8 elements per lane: lane 4 q + g of a block holds the elements k = 32 q + 2 g + j + 8 h + 16 t (j, h, t in
-// {0, 1}) as v[4 t + 2 h + j], exactly the 8 operand-order positions 8 g .. 8 g + 7 of step q, so it stores them
-// with one 16-byte write. The butterflies keep the reference's order and arithmetic (strides 1, 2, 4, ..., 64,
+// 16 lanes hold a block, 8 elements per lane: lane 4 q + g of a block holds the elements k = 32 q + 2 g + j + 8 h + 16 t
+// (j, h, t in {0, 1}) as v[4 t + 2 h + j], exactly chunk g of step q, so it stores them with one 16-byte write. The
+// butterflies keep the reference's order and arithmetic (strides 1, 2, 4, ..., 64,
 // (a, b) -> (a + b, a - b), ft_core.h:89-94): strides 1, 8, 16 pair elements within a lane; strides 2 and 4 pair
 // lanes 4 q + g and 4 q + (g ^ 1 or 2), strides 32 and 64 lanes q ^ 1 and q ^ 2 of the block (DPP moves, all
 // within the block's 16 lanes). The lane holding the upper element of a cross-lane pair forms partner - self as
@@ -180,8 +172,8 @@ __device__ __forceinline__ int lane8_k(int lane, int i)
     return 32 * ((lane >> 2) & 3) + 2 * (lane & 3) + (i & 1) + 8 * ((i >> 1) & 1) + 16 * (i >> 2);
 }
 
-// One 16-lane group transforms row `rl` of a row group: blocks b0 .. b1 - 1 of the token's row, both matrices (the
-// input is read once), two blocks per pass, all loaded before any is used.
+// One 16-lane group transforms one row of a row group: blocks b0 .. b1 - 1 of the token's row, both matrices (the
+// input is read once), two blocks per pass, all loaded before any is used. SUMS: sum[m] += the values of matrix m.
 template <int XD, bool SUMS>
 __device__ __forceinline__ void fat_prep_row(const void* x, size_t row, const uint16_t* su0, uint16_t* dst, int H,
                                              int b0, int b1, float (&sum)[2])
@@ -318,7 +310,7 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
                                                          const int64_t* gate, const int64_t* up, const int64_t* down,
                                                          ExpertRec* rec, FatTile* big, FatTile* small, FatTile* mid,
                                                          int2* groups, int32_t* totals, int max_active, int cap, TileRule rule,
-                                                         int32_t* choice, int E, int n)
+                                                         const int32_t* layer_counts, int32_t* choice, int E, int n)
 {
     // lists: 256-route tiles; tiles of three, two and one row groups; row groups; 128-route tiles
     constexpr int NL = 6;
@@ -363,24 +355,20 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
         if (decode) c = 0;
     }
     int nbig = c >= rule.min_rows ? fat_big_tiles(c, rule.min_rest) : 0;
-    // (a tile of fewer than FT_FULL routes counts half)
-    if (scan(0, 2 * nbig - (nbig && c % FT_BIG >= rule.min_rest && c % FT_BIG < FT_FULL ? 1 : 0)) < 2 * rule.min_tiles)
-        nbig = 0;                                                 // uniform: too few to fill the GPU
+    if (scan(0, nbig) < rule.min_tiles) nbig = 0;                 // uniform: too few to fill the GPU
     __syncthreads();
     const int tbig = scan(0, nbig);
+    // the shorter remainders of the whole layer, computed here or not
+    int shorter = 0;
+    if (a < E)
+    {
+        const int lc = max(layer_counts[a], 0), lr = lc - (lc >= rule.min_rows ? fat_big_tiles(lc, rule.min_rest) : 0) * FT_BIG;
+        shorter = lr > 0 && lr < rule.min_small ? 1 : 0;
+    }
+    const bool fold = scan(1, shorter) <= rule.fold;
     int rest = max(c - nbig * FT_BIG, 0);
-    int nsmall = rest > FT_MID && rest <= FT_SMALL ? 1 : 0, tsmall = scan(5, nsmall);
-    __syncthreads();
-    if (tsmall < rule.min_small)
-    {
-        nsmall = 0;
-        tsmall = scan(5, 0);
-    }
-    else if (scan(1, nsmall ? 0 : (rest + FT_MID - 1) / FT_MID) <= rule.fold)
-    {
-        nsmall = rest > 0 && rest <= FT_SMALL ? 1 : 0;
-        tsmall = scan(5, nsmall);
-    }
+    const int nsmall = rest > 0 && rest <= FT_SMALL && (fold || rest >= rule.min_small) ? 1 : 0;
+    const int tsmall = scan(5, nsmall);
     if (nsmall) rest = 0;
     const int full = rest / FT_MID, r = rest % FT_MID;
     __syncthreads();
@@ -615,19 +603,18 @@ __device__ __forceinline__ void fat_scales(const FatArgs& a, int e, int nu, cons
     }
 }
 
-// MB = 16-row blocks per row-wave: tiles of BM = 32 MB routes (256 or 128). 8 waves: wave (wm, wn) = (w >> 2,
+// Gate/up tiles of FT_BIG routes, MB = 8 row blocks of 16 per row-wave. 8 waves: wave (wm, wn) = (w >> 2,
 // w & 3) multiplies row blocks wm, wm + 2, wm + 4, ... (rows 16 (2 i + wm) .. + 15) by column tiles 4 wn .. 4 wn + 3
 // of 16, so in a tile with fewer routes the two waves of a SIMD keep about the same number of row blocks
 // (0.7 % off the 16k layer against contiguous halves); every wave loads an
-// eighth of the inputs and waves 0 .. 3 also the trellis (chunk w: tile row w >> 1 of matrix / block w & 1),
+// eighth of the inputs and waves 0 .. 3 also the trellis (chunk w: tile row w >> 1 of matrix w & 1),
 // which runs further ahead; wave w decodes column tiles 2 (w & 3), 2 (w & 3) + 1 of sub-block w >> 2 in both tile
 // rows (chunks w >> 2 and 2 + (w >> 2)). Rows past the tile's routes multiply what their row group holds (zeros past the
 // last group) and are not stored.
-template <int MODE, int MB, bool YH = false>
 __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
 {
-    constexpr int BM = 32 * MB;
-    constexpr int NA = MODE == 0 ? 2 : 1;                        // input matrices (gate, up share the tile)
+    constexpr int MB = 8, BM = FT_BIG;
+    constexpr int NA = 2;                                        // input matrices (gate, up share the tile)
     constexpr int SEG = NA * 64;                                 // bytes of one route's step (gate, up)
     constexpr int A_STAGE = BM * SEG;                            // one step's inputs
     constexpr int LA = A_STAGE / 1024 / FT_WAVES;                // input loads (1 KB each) per wave and step
@@ -639,7 +626,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
     constexpr int SMEM = MAIN > FT_BN * CS * 2 ? MAIN : FT_BN * CS * 2;
     static_assert(SMEM <= 160 * 1024, "LDS");
     static_assert(((CS / 2) & 1) == 1, "odd dword stride: conflict-free column reads");
-    static_assert(MB % 2 == 0, "one decoded tile per two row blocks");
+    static_assert(BM == 32 * MB, "two row-waves");
     __shared__ __align__(16) uint8_t smem[SMEM];
     uint8_t* Aring = smem;
     uint8_t* Tring = smem + A_BYTES;
@@ -658,15 +645,15 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
     const int S = a.K / 32;
 
     const bool tloader = wave < 4;
-    // trellis loader (waves 0 .. 3): chunk q = wave of step s is tile row 2 s + (q >> 1) of matrix q & 1 (gate/up)
-    // or of column block 2 nu + (q & 1) (down), 8 tiles = 768 bytes, 12 bytes per lane stored 16 bytes apart.
+    // trellis loader (waves 0 .. 3): chunk q = wave of step s is tile row 2 s + (q >> 1) of matrix q & 1, 8 tiles =
+    // 768 bytes, 12 bytes per lane stored 16 bytes apart.
     // Steps past the end reload the last row into the free slot, so every step issues one load.
     const int tq = wave & 3;
     const uint32_t row_bytes = (uint32_t)(a.N / 16) * 96, wbytes = (uint32_t)(a.K / 16) * row_bytes;
-    const void* wbase = (const void*)(uintptr_t)(MODE == 0 ? ((tq & 1) ? rp->w[1] : rp->w[0]) : rp->w[2]);
+    const void* wbase = (const void*)(uintptr_t)((tq & 1) ? rp->w[1] : rp->w[0]);
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(wbase), (short)0, (int)wbytes,
                                                                           0x00020000);
-    const uint32_t wcol = MODE == 0 ? (uint32_t)nu * 768 : (uint32_t)(2 * nu + (tq & 1)) * 768;
+    const uint32_t wcol = (uint32_t)nu * 768;
     auto load_trellis = [&](int s) {
         const uint32_t tr = (uint32_t)(2 * min(s, S - 1) + (tq >> 1));
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, Tring + (size_t)(s % FT_TS) * T_SLOT + (size_t)tq * 1024, 12,
@@ -700,7 +687,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
     const int db = wave >> 2, dc = 2 * (wave & 3);
     const uint32_t* tword = reinterpret_cast<const uint32_t*>(Tring + (size_t)db * 1024 + (size_t)dc * 128);
     uint8_t* bdst = Bdec + ((size_t)(db * 8 + dc) * 64 + lane) * 16;
-    // ---- MFMA: rows 16 (2 i + wm) + col of input matrix wn >> 1 (gate/up), B tiles 4 wn .. + 3
+    // ---- MFMA: rows 16 (2 i + wm) + col of input matrix wn >> 1, B tiles 4 wn .. + 3
     const int wm = wave >> 2, wn = wave & 3;
     const uint8_t* bsrc = Bdec + ((size_t)(wn * 4) * 64 + lane) * 16;
     int aoff[MB];
@@ -708,7 +695,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
     for (int i = 0; i < MB; ++i)
     {
         const int r = 16 * (2 * i + wm) + col;
-        aoff[i] = ((r >> 5) * NA + (MODE == 0 ? (wn >> 1) : 0)) * 2048 + (g * 32 + (r & 31)) * 16;
+        aoff[i] = ((r >> 5) * NA + (wn >> 1)) * 2048 + (g * 32 + (r & 31)) * 16;
     }
     float4_t acc[MB][4];
 #pragma unroll
@@ -760,7 +747,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
             const uint8_t* thp = reinterpret_cast<const uint8_t*>(tword + lhi) + toff;
             const uint8_t* tlp = reinterpret_cast<const uint8_t*>(tword + llo) + toff;
             uint32_t th[4], tl[4];
-    #pragma unroll
+#pragma unroll
             for (int u = 0; u < 4; ++u)
             {
                 th[u] = *reinterpret_cast<const uint32_t*>(thp + (u & 1) * 2048 + (u >> 1) * 128);
@@ -773,9 +760,9 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
             // compiler keeps LDS accesses that may alias in program order, so reads placed after a write would each
             // wait a full LDS round trip
             half8_t B[4], A[MB];
-    #pragma unroll
+#pragma unroll
             for (int j = 0; j < 4; ++j) B[j] = *reinterpret_cast<const half8_t*>(bs + j * 1024);
-    #pragma unroll
+#pragma unroll
             for (int i = 0; i < MB; ++i)
                 if (!PART || i < nvb) A[i] = *reinterpret_cast<const half8_t*>(as + aoff[i]);
             // tile 0 is decoded before the first MFMA: the decode runs while the workgroup's operand reads of the
@@ -783,11 +770,11 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
             // blocks 0 .. MB / 4 - 1); tiles 1 .. 3 follow row blocks MB / 4 - 1, MB / 2 - 1, 3 MB / 4 - 1, and
             // each column tile is stored once both of its tile rows are decoded
             half4_t d0 = decode4<true>(th[0], tl[0], sh);
-    #pragma unroll
+#pragma unroll
             for (int i = 0; i < MB; ++i)
             {
                 if (!PART || i < nvb)
-    #pragma unroll
+#pragma unroll
                     for (int j = 0; j < 4; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[i], B[j], acc[i][j], 0, 0, 0);
                 if (i % (MB / LA) == 0) load_input(s + FT_PA - 1, i / (MB / LA));
@@ -809,7 +796,7 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
             {
                 __builtin_amdgcn_sched_group_barrier(0x0100, 4 + MB + 8, 0);
                 __builtin_amdgcn_sched_group_barrier(0x0002, 16, 0);
-    #pragma unroll
+#pragma unroll
                 for (int k = 0; k < 4 * MB; ++k)
                 {
                     __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
@@ -840,12 +827,12 @@ __global__ __launch_bounds__(FT_THREADS, 1) void k_fat(FatArgs a)
         }
     __syncthreads();
     const uint16_t* sc[3];
-    fat_scales<MODE>(a, e, nu, sc);
-    fat_tile_epilogue<MODE, CS, YH>(a, C, rows, nu, grp, wave, lane, sc, a.route_at + pos0);
+    fat_scales<0>(a, e, nu, sc);
+    fat_tile_epilogue<0, CS, false>(a, C, rows, nu, grp, wave, lane, sc, a.route_at + pos0);
 }
 
-// Sixteen-wave form of the tile (four waves per SIMD, 64 accumulators per lane): MBW = row blocks per wave, BM =
-// 64 MBW routes (256 or 128). Wave (wm, wn) = (w >> 2, w & 3) multiplies row blocks wm, wm + 4, ... (rows
+// Sixteen-wave form of the tile (four waves per SIMD, at most 64 accumulators per lane): MBW = row blocks per wave, BM =
+// 64 MBW routes (4: 256, down only; 2: 128). Wave (wm, wn) = (w >> 2, w & 3) multiplies row blocks wm, wm + 4, ... (rows
 // 16 (4 i + wm) .. + 15) by column tiles 4 wn .. 4 wn + 3, so each SIMD (waves w, w + 4, w + 8, w + 12) holds
 // one column group over every row block of the tile. Inputs: buffer-to-LDS, two steps ahead in a three-stage ring,
 // input load li of a step (1 KB) issued by wave li % 16; trellis as k_fat (waves 0 .. 3); wave w decodes column
@@ -1490,7 +1477,7 @@ static FatWs fat_carve(void* base, int n, int E, int H, int I)
     // an expert of c routes has at most c / min_rest 256-route tiles, one 128-route tile of more than FT_MID routes, c / FT_MID
     // + 1 others and c / GRP_ROWS + 1 row groups
     FatWs w;
-    w.max_big = n / FT_REST_EXACT;
+    w.max_big = n / FT_REST_LARGE;
     w.max_small = (int)na;
     w.max_mid = n / FT_MID + (int)na;
     w.max_groups = n / GRP_ROWS + (int)na;
@@ -1541,34 +1528,30 @@ static int fat_check(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     return MM_OK;
 }
 
-// How a call's experts are taken: the fused call by the layer's codebook evaluation, the others with fp16-rounded weights; the
-// whole calls may choose their tiles together, those of some experts of a layer by the expert alone.
-enum class FatCall { FUSED, WHOLE, EXPERTS };
+// How a call's experts are taken: the fused call by the layer's codebook evaluation, the others with fp16-rounded weights.
 struct FatMode
 {
     bool exact;
     TileRule rule;
 };
-static FatMode fat_mode(const mm_layer_t* L, int n, FatCall call)
+static FatMode fat_mode(const mm_layer_t* L, int n, bool fused)
 {
-    const int units = L->I / 128, tiles = (FT_BIG_WORK + units - 1) / units;
-    switch (call)
-    {
-    case FatCall::FUSED: return { (L->flags & MM_LAYER_EXACT) != 0, TileRule{ tiles, 0, FT_REST, FT_NEVER, 0 } };
-    case FatCall::WHOLE: return { true, TileRule{ tiles, 0, FT_REST_EXACT, 2 * tiles, tiles / 2 } };
-    default:
-        if (n >= FT_LARGE && n / 200 >= L->E) return { true, TileRule{ 0, 0, FT_REST_EXACT, 0, FT_NEVER } };
-        return { true, TileRule{ 0, FT_BIG_ROWS, FT_REST, FT_NEVER, 0 } };
-    }
+    const int units = L->I / 128, tiles = (FT_BIG_WORK + units - 1) / units, none = FT_SMALL + 1;
+    if (fused) return { (L->flags & MM_LAYER_EXACT) != 0, TileRule{ tiles, 0, FT_REST, none, -1 } };
+    if (n >= FT_LARGE && n / 200 >= L->E) return { true, TileRule{ 0, 0, FT_REST_LARGE, FT_MID + 1, tiles / 2 } };
+    return { true, TileRule{ 0, FT_BIG_ROWS, FT_REST, none, -1 } };
 }
 
 // Expert records, row groups and tile lists of the sorted positions in ws (counts, offsets, active, nactive filled).
-static void fat_plan(const mm_layer_t* L, int n, int cap, const FatWs& ws, hipStream_t s, const FatMode& mode, int32_t* choice)
+// layer_counts: the routes of every expert of the layer, whether the call computes it or not.
+static void fat_plan(const mm_layer_t* L, int n, int cap, const FatWs& ws, hipStream_t s, const FatMode& mode,
+                     const int32_t* layer_counts, int32_t* choice)
 {
     const int E = L->E, na = n < E ? n : E;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(1), dim3(FT_PLAN_MAX), 0, s, ws.counts, ws.offsets, ws.active, ws.nactive, L->gate_ptr,
-                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.small, ws.mid, ws.groups, ws.totals, na, cap, mode.rule, choice, E, n);
+                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.small, ws.mid, ws.groups, ws.totals, na, cap, mode.rule, layer_counts,
+                           choice, E, n);
     };
     if (choice) launch(k_fat_plan<true>);
     else launch(k_fat_plan<false>);
@@ -1586,8 +1569,8 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     };
     if (exact) prep(k_fat_prep<false>);
     else prep(k_fat_prep<true>);
-    // 256-route and 128-route tiles a call of n routes can have
-    const int max_small = std::min(n / (FT_MID + 1), ws.max_small) >= mode.rule.min_small ? ws.max_small : 0;
+    // tiles of 128 and of 256 routes the call can have
+    const int max_small = mode.rule.min_small <= FT_SMALL ? ws.max_small : 0;
     const int max_big = ws.max_big >= mode.rule.min_tiles && n >= mode.rule.min_rows ? ws.max_big : 0;
     auto grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles * units + 7) & ~(size_t)7)); };    // >= 8 per_xcd
     auto mid_grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles + 7) / 8 * 8 * units)); };
@@ -1610,7 +1593,7 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     ds.ntiles = ws.totals + 3;
     // gate/up: 256-route tiles on the 8-wave kernel, down on the 16-wave kernel (same bits; measured on the 16k layer:
     // gate/up equal, down 2.76-2.85 against 2.92-2.94 ms)
-    if (max_big > 0) hipLaunchKernelGGL((k_fat<0, FT_BIG / 32>), grid(max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
+    if (max_big > 0) hipLaunchKernelGGL(k_fat, grid(max_big, g.nunits), dim3(FT_THREADS), 0, s, g);
     if (max_small > 0) hipLaunchKernelGGL((k_fat16<0, FT_SMALL / 64>), grid(max_small, g.nunits), dim3(FT16_THREADS), 0, s, gs);
     if (exact) hipLaunchKernelGGL((k_mid<0, true>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
     else hipLaunchKernelGGL((k_mid<0, false>), mid_grid(ws.max_mid, g.nunits), dim3(256), 0, s, gm);
@@ -1637,14 +1620,14 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
 
 // Permutation, plan, input transform and both GEMMs: Y rows of every route whose expert has more than cap routes.
 static int fat_run(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, int cap,
-                   const FatWs& ws, hipStream_t s, bool yh, FatCall call)
+                   const FatWs& ws, hipStream_t s, bool yh, bool fused)
 {
     const int n = T * topk, E = L->E;
     int rc = permute_launch(ids, nullptr, n, topk, E, ws.counts, ws.offsets, ws.order, nullptr, nullptr, nullptr,
-                            ws.active, ws.nactive, nullptr, ws.pws, ws.pws_bytes, s);
+                            ws.active, ws.nactive, ws.pws, ws.pws_bytes, s);
     if (rc) return rc;
-    const FatMode mode = fat_mode(L, n, call);
-    fat_plan(L, n, cap, ws, s, mode, nullptr);
+    const FatMode mode = fat_mode(L, n, fused);
+    fat_plan(L, n, cap, ws, s, mode, ws.counts, nullptr);
     return fat_gemms(L, x, x_dtype, T, topk, nullptr, n, ws, s, yh, mode);
 }
 
@@ -1659,9 +1642,9 @@ static int fat_combine(const mm_layer_t* L, int T, int topk, const int64_t* ids,
 
 // fat_run and the weighted combine of its rows.
 static int fat_layer(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
-                     int cap, int accumulate, float* out, const FatWs& ws, hipStream_t s, FatCall call)
+                     int cap, int accumulate, float* out, const FatWs& ws, hipStream_t s, bool fused)
 {
-    const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true, call);
+    const int r = fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, true, fused);
     return r ? r : fat_combine(L, T, topk, ids, w, cap, accumulate, out, ws, s, nullptr);
 }
 
@@ -1794,14 +1777,13 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
         return moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, workspace, workspace_bytes, stream,
                                  "mm_fused_moe");
     if (path == FusedPath::GEMM)
-        return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I), s,
-                         FatCall::FUSED);
+        return fat_layer(L, x, x_dtype, T, topk, ids, w, 0, 0, out, fat_carve(workspace, n, E, L->H, L->I), s, true);
     const FusedWs ws = fused_carve(workspace, n, E, L->H, L->I, mm_gemv_workspace(n, E, L->H, L->I));
     int r = permute_launch(ids, nullptr, n, topk, E, ws.f.counts, ws.f.offsets, ws.f.order, nullptr, nullptr, nullptr,
-                           ws.f.active, ws.f.nactive, nullptr, ws.f.pws, ws.f.pws_bytes, s);
+                           ws.f.active, ws.f.nactive, ws.f.pws, ws.f.pws_bytes, s);
     if (r) return r;
-    const FatMode mode = fat_mode(L, n, FatCall::FUSED);
-    fat_plan(L, n, 0, ws.f, s, mode, ws.choice);
+    const FatMode mode = fat_mode(L, n, true);
+    fat_plan(L, n, 0, ws.f, s, mode, ws.f.counts, ws.choice);
     // the decode path's launches first: the grouped GEMM's inputs lie over their workspace
     r = moe_decode_launch(L, x, x_dtype, 0, T, topk, ids, w, n, out, ws.dws, ws.dws_bytes, stream, "mm_fused_moe",
                           ws.f.offsets, ws.f.order, ws.f.active, ws.choice, ws.choice + 1);
@@ -1825,7 +1807,7 @@ int mm_grouped_gemm(const mm_layer_t* L, const void* x, int x_dtype, int T, int 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     FatWs ws = fat_carve(workspace, T * topk, L->E, L->H, L->I);
     ws.Y = Y;
-    return fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, false, FatCall::WHOLE);
+    return fat_run(L, x, x_dtype, T, topk, ids, cap, ws, s, false, false);
 }
 
 int mm_moe_prefill(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,
@@ -1835,7 +1817,7 @@ int mm_moe_prefill(const mm_layer_t* L, const void* x, int x_dtype, int T, int t
     if (rc) return rc;
     MM_CHECK_ARG(w && out && cap >= 0, "mm_moe_prefill: null pointer or negative cap");
     return fat_layer(L, x, x_dtype, T, topk, ids, w, cap, accumulate, out, fat_carve(workspace, T * topk, L->E, L->H, L->I),
-                     reinterpret_cast<hipStream_t>(stream), FatCall::WHOLE);
+                     reinterpret_cast<hipStream_t>(stream), false);
 }
 
 size_t mm_fat_batched_workspace(int n, int T, int E, int H, int I)
@@ -1873,8 +1855,8 @@ int mm_fat_batched(const mm_layer_t* L, const void* x, int x_dtype, int T, int n
     hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)std::min((T + 255) / 256, 1024)), dim3(256), 0, s, ws.tcount, T, 0);
     hipLaunchKernelGGL(k_fatb_tokens<1>, dim3(pg), dim3(256), 0, s, token_sorted, ws.f.counts, ws.f.offsets, ws.f.order,
                        ws.tcount, ws.toff, ws.tpos, T, E, n);
-    const FatMode mode = fat_mode(L, n, FatCall::EXPERTS);
-    fat_plan(L, n, cap, ws.f, s, mode, nullptr);
+    const FatMode mode = fat_mode(L, n, false);
+    fat_plan(L, n, cap, ws.f, s, mode, counts, nullptr);
     int r = fat_gemms(L, x, x_dtype, T, 1, token_sorted, n, ws.f, s, true, mode);
     if (r) return r;
     const dim3 grid((unsigned)((L->H / 4 + 255) / 256), (unsigned)T);

@@ -3,13 +3,13 @@
 //
 // A layer runs as five launches on the caller's stream. Stream order is the only synchronisation (no fences,
 // no atomics between workgroups), so every result is deterministic:
-//   1. k_route_prep    one workgroup per (route, gate|up, 512 input rows): the route's sorted position (stable
-//                      by expert, then route index), one record per active expert, and the route's transformed
-//                      input xt = r16(FWHT128(x * suh) * HAD) in MFMA operand order, with its sums (the input
+//   1. k_route_prep    one workgroup per (route, gate|up, 512 input rows), or per (route, gate|up) in larger calls: the
+//                      route's sorted position (stable by expert, then route index), the experts' records (one per active
+//                      expert, above 16 tokens one per 16 of its routes), and the route's transformed input xt = r16(FWHT128(x * suh) * HAD) in MFMA operand order, with its sums (the input
 //                      conversion and the optional unit-RMS rescale happen here too).
 //   2. k_partial<0>    gate/up partial sums, one launch that fills the GPU once: the work -- every
-//                      (active expert, matrix, 128 output columns) segment of 256 tile rows -- is cut into
-//                      equal runs of rows, one per wave, from the active-expert count on the device. A wave
+//                      (record, matrix, 128 output columns) segment of 256 tile rows -- is cut into
+//                      equal runs of rows, one per wave, from the record count on the device. A wave
 //                      streams its rows (8 tiles = 768 contiguous bytes each) from HBM into a 4-deep
 //                      wave-private LDS ring with buffer-to-LDS loads, decodes each tile in registers and
 //                      multiplies two tile rows at a time on v_mfma_f32_16x16x32_f16 against the inputs of up
@@ -51,7 +51,7 @@ constexpr int PREP_WALK_MIN = 384;    // routes from which a permutation's route
 constexpr int SS_LOADS = 16;          // route prep: row elements per thread loaded at once for the rescale
 constexpr int MAX_TOPK = 16;
 
-// Rows of a partial launch: nseg segments of KT tile rows each (KT a multiple of 8), in segment order, cut into
+// Rows of a partial launch: nseg (records x matrices x column blocks) segments of KT tile rows each (KT a multiple of 8), in segment order, cut into
 // nw runs of equal length (within 4 rows) that start and end on multiples of 4 rows, one per wave, so every wave
 // streams as many rows as every other. A run that reaches the end of a segment goes on in the next one; the wave
 // then computes one piece of each, and a segment's pieces are the runs that meet it, numbered from 0 in row
@@ -360,8 +360,8 @@ struct PartArgs
     const ExpertRec* rec;
     const int32_t* counts;
     const uint16_t* xa;       // mode 0: [n][2][K]; mode 1: [n][K] (operand order)
-    float* part;              // [pieces][npos][nmat][N]
-    int npos, K, N, ncb, cap; // npos: sorted positions the workspace holds
+    float* part;              // [pieces][n][nmat][N]
+    int n, K, N, ncb, cap;
 };
 
 // One pass of a partial-sum wave (k_partial): r0 of the run's rows [tr0, tr0 + nrow) of segment seg.
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(GV_THREADS, 6) void k_partial(PartArgs a)
     if (w >= split.nw) return;
     const uint32_t row_bytes = (uint32_t)NT * 96;
     const uint32_t wbytes = (uint32_t)KT * row_bytes;                   // one matrix
-    const uint32_t xbytes = (uint32_t)((size_t)a.npos * NMAT * a.K * 2);   // the input array
+    const uint32_t xbytes = (uint32_t)((size_t)a.n * NMAT * a.K * 2);   // the input array
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.xa), (short)0,
                                                                           (int)xbytes, 0x00020000);
     // lane constants of the decode
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(GV_THREADS, 6) void k_partial(PartArgs a)
             int l = lane;
             asm volatile("" : "+v"(l));
             const int sg = l >> 4;
-            float* dst = a.part + ((size_t)(cur.piece * a.npos + cur.first + cur.r0 + 4 * sg) * NMAT + cur.m) * a.N +
+            float* dst = a.part + ((size_t)(cur.piece * a.n + cur.first + cur.r0 + 4 * sg) * NMAT + cur.m) * a.N +
                          cur.cb * GV_COLS + (l & 15);
 #pragma unroll
             for (int v = 0; v < 4; ++v)
@@ -658,7 +658,7 @@ struct GuEpiArgs
     const uint16_t* suh2;     // [E][I]
     uint16_t* xd;             // [n][I] fp16 in operand order
     float* xdsum;             // [n][I / 128] sums of xd over each 128-column block
-    int npos, H, I, nb, nwaves, cap, affine;
+    int n, H, I, nb, nwaves, cap, affine;
     float limit;
 };
 
@@ -675,8 +675,8 @@ __global__ __launch_bounds__(256) void k_gu_epilogue(GuEpiArgs a)
     const int nvalid = a.counts[1], nact = a.counts[0];
     // (the wave's position is one, so e and ai are too: read as scalars, the piece counts and the branches on
     // them below stay scalar)
-    const int e = __builtin_amdgcn_readfirstlane(a.e_at[min(pos, a.npos - 1)]);
-    const int ai = __builtin_amdgcn_readfirstlane(a.ai_at[min(pos, a.npos - 1)]);
+    const int e = __builtin_amdgcn_readfirstlane(a.e_at[min(pos, a.n - 1)]);
+    const int ai = __builtin_amdgcn_readfirstlane(a.ai_at[min(pos, a.n - 1)]);
     asm volatile("" ::"s"(nact), "s"(e), "s"(ai));      // one round trip, not the count after the branch below
     if (pos >= nvalid || e < 0 || ai < 0) return;      // past the routes, or a route of an expert above the cap
     const int KT = a.H / 16;
@@ -699,7 +699,7 @@ __global__ __launch_bounds__(256) void k_gu_epilogue(GuEpiArgs a)
     }
     const float* const pgu[2] = { a.part + ((size_t)pos * 2 + 0) * a.I + c, a.part + ((size_t)pos * 2 + 1) * a.I + c };
     float s0[2] = { 0.f, 0.f }, s1[2] = { 0.f, 0.f };
-    sum_pieces<2>(pgu, (size_t)a.npos * 2 * a.I, np, lane, s0, s1);
+    sum_pieces<2>(pgu, (size_t)a.n * 2 * a.I, np, lane, s0, s1);
     float ga = s0[0], gb = s1[0], ua = s0[1], ub = s1[1];
     if (a.affine)
     {
@@ -740,13 +740,13 @@ struct DEpiArgs
     const uint16_t* svh2;     // [E][H]
     float* Y;                 // [n][H] (per-route rows)
     float* out;               // [T][H] (combine)
-    int npos, H, I, topk, nwaves, cap, affine;
+    int n, H, I, topk, nwaves, cap, affine;
     int gated;                // combine: out is left untouched where no route is computed
 };
 
 // Down output of one (sorted position, 128-column block of H): pieces added in order (then the AFFINE
 // fixup), output transform.
-// nact = active experts (counts[0]), read by the caller with its other first loads; the scales, input sums and
+// nact = records (counts[0]), read by the caller with its other first loads; the scales, input sums and
 // partial sums then share one round trip.
 __device__ __forceinline__ void down_block(const DEpiArgs& a, int nact, int ai, int pos, int c, int64_t e, int lane,
                                            float& ya, float& yb)
@@ -760,7 +760,7 @@ __device__ __forceinline__ void down_block(const DEpiArgs& a, int nact, int ai, 
     float sx = a.affine ? wave_sum_first(xs, a.I / GV_COLS, lane) : 0.f;
     const float* const pd[1] = { a.part + (size_t)pos * a.H + c };
     float s0[1] = { 0.f }, s1[1] = { 0.f };
-    sum_pieces<1>(pd, (size_t)a.npos * a.H, np, lane, s0, s1);
+    sum_pieces<1>(pd, (size_t)a.n * a.H, np, lane, s0, s1);
     ya = s0[0];
     yb = s1[0];
     if (a.affine)
@@ -781,7 +781,7 @@ __global__ __launch_bounds__(256) void k_down_y(DEpiArgs a)
     const int ncb = a.H / GV_COLS;
     const int pos = item / ncb, cb = item % ncb;
     const int nvalid = a.counts[1], nact = a.counts[0];
-    const int pc = min(pos, a.npos - 1);
+    const int pc = min(pos, a.n - 1);
     // one position per wave: read as scalars
     const int s = __builtin_amdgcn_readfirstlane(a.route_at[pc]), e = __builtin_amdgcn_readfirstlane(a.e_at[pc]);
     const int ai = __builtin_amdgcn_readfirstlane(a.ai_at[pc]);
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(1024) void k_down_combine(DEpiArgs a)
     if (a.gated && a.counts[1] == 0) return;
     if (j < a.topk)
     {
-        // round trip 1: the route's position, expert, active index and weight and the active-expert count. A pick
+        // round trip 1: the route's position, expert, record and weight and the record count. A pick
         // outside [0, E) (position -1) is computed on position 0 and expert 0 and left out of the sum, so no branch
         // keeps the expert's load from being issued with the others.
         const int s = t * a.topk + j;     // one route per wave: its fields are read as scalars
@@ -864,9 +864,9 @@ template <int XD>
 static void launch_route_prep_t(const PrepArgs& p, hipStream_t s)
 {
     if (p.split)
-        hipLaunchKernelGGL((k_route_prep<XD, true>), dim3(2 * p.npos * (p.walk ? 1 : p.nb)), dim3(256), 0, s, p);
+        hipLaunchKernelGGL((k_route_prep<XD, true>), dim3(2 * p.n * (p.walk ? 1 : p.nb)), dim3(256), 0, s, p);
     else
-        hipLaunchKernelGGL((k_route_prep<XD, false>), dim3(2 * p.npos * p.nb), dim3(256), 0, s, p);
+        hipLaunchKernelGGL((k_route_prep<XD, false>), dim3(2 * p.n * p.nb), dim3(256), 0, s, p);
 }
 
 void launch_route_prep(const PrepArgs& p, hipStream_t s)
@@ -900,17 +900,15 @@ static bool split_records(const mm_layer_t* L, int n, int topk)
     return n > REC_ROUTES * topk && rows_fit(L->H, L->I, max_records(n, L->E));
 }
 
-// Workspace of n routes whose sorted positions lie below npos (npos = n unless a caller bounds the positions), with room for
-// `pieces` x 1 route of partial sums.
-static Ws carve(void* base, int n, int npos, int E, int H, int I, size_t pieces)
+// Workspace of n routes; pieces: the partial sums it holds, each of one route.
+static Ws carve(void* base, int n, int E, int H, int I, size_t pieces)
 {
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t m = (size_t)npos;
-    const size_t na = (size_t)max_records(npos, E);
+    const size_t m = (size_t)n, na = (size_t)max_records(n, E);
     // the small routing arrays first and together (records, counts, pos_of, route_at, e_at, ai_at, ai_of), so the
     // epilogues' first loads fall in the same few pages
-    const size_t sizes[13] = { al(na * sizeof(ExpertRec)), al(2 * 4), al((size_t)n * 4), al(m * 4),
-                               al(m * 4), al(m * 4), al((size_t)n * 4), al(m * 2 * H * 2),
+    const size_t sizes[13] = { al(na * sizeof(ExpertRec)), al(2 * 4), al(m * 4), al(m * 4),
+                               al(m * 4), al(m * 4), al(m * 4), al(m * 2 * H * 2),
                                al(m * 2 * prep_blocks(H) * 4), al(pieces * 2 * I * 4), al(m * I * 2),
                                al(m * (I / GV_COLS) * 4), al(pieces * H * 4) };
     char* p = static_cast<char*>(base);
@@ -938,15 +936,12 @@ static Ws carve(void* base, int n, int npos, int E, int H, int I, size_t pieces)
     w.bytes = off;
     return w;
 }
-static Ws carve(void* base, int n, int npos, int E, int H, int I)
-{
-    return carve(base, n, npos, E, H, I, (size_t)piece_cap(npos) * npos);
-}
+static Ws carve(void* base, int n, int E, int H, int I) { return carve(base, n, E, H, I, (size_t)piece_cap(n) * n); }
 
 // Bytes that hold the decode workspace of every call of up to n routes (piece_cap(m) m is at most 32 m, 8192 or 4 m).
 size_t decode_workspace_upto(int n, int E, int H, int I)
 {
-    return carve(nullptr, n, n, E, H, I, n <= 256 ? (size_t)32 * n : (size_t)std::max(8192, 4 * n)).bytes;
+    return carve(nullptr, n, E, H, I, n <= 256 ? (size_t)32 * n : (size_t)std::max(8192, 4 * n)).bytes;
 }
 
 // Waves of one partial launch: the whole GPU once (WAVES_PER_CU per CU, a multiple of 8 workgroups), or half of
@@ -997,13 +992,13 @@ static int check_common(const mm_layer_t* L, const void* x, int x_dtype, int T, 
     const bool perm = offsets != nullptr;
     MM_CHECK_ARG(perm ? (order && active && nactive) : n <= GV_ROUTE_MAX,
                  "%s: more than %d routes need the permutation (offsets, order, active, nactive)", who, GV_ROUTE_MAX);
-    const size_t need = carve(nullptr, n, n, L->E, L->H, L->I).bytes;
+    const size_t need = carve(nullptr, n, L->E, L->H, L->I).bytes;
     MM_CHECK_ARG(ws && ws_bytes >= need, "%s: workspace too small (%zu < %zu)", who, ws_bytes, need);
     return MM_OK;
 }
 
-static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_dtype, int rescale, int n, int npos,
-                        int topk, const int64_t* ids, const int32_t* offsets, const int32_t* order,
+static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_dtype, int rescale, int n, int topk,
+                        const int64_t* ids, const int32_t* offsets, const int32_t* order,
                         const int32_t* active, const int32_t* nactive, const int32_t* nvalid, bool gated, int cap,
                         hipStream_t s)
 {
@@ -1014,35 +1009,35 @@ static void launch_prep(const mm_layer_t* L, const Ws& w, const void* x, int x_d
     const bool split = split_records(L, n, topk), walk = split && (!offsets || n >= PREP_WALK_MIN);
     PrepArgs p{ x, ids, offsets, order, active, nactive, nvalid, L->gate_ptr, L->up_ptr, L->down_ptr, L->suh13,
                 w.rec, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, w.xa, w.xsum, n, topk, L->E, L->H, nb,
-                x_dtype, rescale, cap, split ? 1 : 0, walk ? 1 : 0, gated ? 1 : 0, npos };
+                x_dtype, rescale, cap, split ? 1 : 0, walk ? 1 : 0, gated ? 1 : 0 };
     launch_route_prep(p, s);
 }
 
 template <int MODE>
-static void launch_partial(const mm_layer_t* L, const Ws& w, int npos, hipStream_t s)
+static void launch_partial(const mm_layer_t* L, const Ws& w, int n, hipStream_t s)
 {
     const int K = MODE == 0 ? L->H : L->I, N = MODE == 0 ? L->I : L->H;
-    PartArgs p{ w.rec, w.counts, MODE == 0 ? w.xa : w.xd, MODE == 0 ? w.part_gu : w.part_d, npos, K, N, N / GV_COLS,
-                piece_cap(npos) };
-    const dim3 grid(partial_waves(seg_max(L, npos, MODE)) / GV_WAVES), block(GV_THREADS);
+    PartArgs p{ w.rec, w.counts, MODE == 0 ? w.xa : w.xd, MODE == 0 ? w.part_gu : w.part_d, n, K, N, N / GV_COLS,
+                piece_cap(n) };
+    const dim3 grid(partial_waves(seg_max(L, n, MODE)) / GV_WAVES), block(GV_THREADS);
     if (L->flags & MM_LAYER_EXACT)
         hipLaunchKernelGGL((k_partial<MODE, true>), grid, block, 0, s, p);
     else
         hipLaunchKernelGGL((k_partial<MODE, false>), grid, block, 0, s, p);
 }
 
-static void launch_gu_epilogue(const mm_layer_t* L, const Ws& w, int npos, hipStream_t s)
+static void launch_gu_epilogue(const mm_layer_t* L, const Ws& w, int n, hipStream_t s)
 {
-    GuEpiArgs g{ w.part_gu, w.xsum, w.counts, w.e_at, w.ai_at, L->svh13, L->suh2, w.xd, w.xdsum, npos, L->H, L->I,
-                 prep_blocks(L->H), partial_waves(seg_max(L, npos, 0)), piece_cap(npos), (L->flags & MM_LAYER_EXACT) ? 0 : 1, L->limit };
-    hipLaunchKernelGGL(k_gu_epilogue, dim3((npos * (L->I / GV_COLS) + 3) / 4), dim3(256), 0, s, g);
+    GuEpiArgs g{ w.part_gu, w.xsum, w.counts, w.e_at, w.ai_at, L->svh13, L->suh2, w.xd, w.xdsum, n, L->H, L->I,
+                 prep_blocks(L->H), partial_waves(seg_max(L, n, 0)), piece_cap(n), (L->flags & MM_LAYER_EXACT) ? 0 : 1, L->limit };
+    hipLaunchKernelGGL(k_gu_epilogue, dim3((n * (L->I / GV_COLS) + 3) / 4), dim3(256), 0, s, g);
 }
 
-static DEpiArgs down_args(const mm_layer_t* L, const Ws& w, int npos, int topk, const int64_t* ids, const float* wt,
+static DEpiArgs down_args(const mm_layer_t* L, const Ws& w, int n, int topk, const int64_t* ids, const float* wt,
                           float* Y, float* out, bool gated = false)
 {
-    return DEpiArgs{ w.part_d, w.xdsum, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, ids, wt, L->svh2, Y, out, npos, L->H,
-                     L->I, topk, partial_waves(seg_max(L, npos, 1)), piece_cap(npos), (L->flags & MM_LAYER_EXACT) ? 0 : 1, gated ? 1 : 0 };
+    return DEpiArgs{ w.part_d, w.xdsum, w.counts, w.pos_of, w.route_at, w.e_at, w.ai_at, w.ai_of, ids, wt, L->svh2, Y, out, n, L->H,
+                     L->I, topk, partial_waves(seg_max(L, n, 1)), piece_cap(n), (L->flags & MM_LAYER_EXACT) ? 0 : 1, gated ? 1 : 0 };
 }
 
 int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int rescale, int T, int topk, const int64_t* ids,
@@ -1057,8 +1052,8 @@ int moe_decode_launch(const mm_layer_t* L, const void* x, int x_dtype, int resca
     if (rc) return rc;
     MM_CHECK_ARG(w && out, "%s: null pointer", who);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const Ws ws = carve(workspace, n, n, L->E, L->H, L->I);
-    launch_prep(L, ws, x, x_dtype, rescale, n, n, topk, ids, offsets, order, active, nactive, nvalid, nvalid != nullptr, max_rows, s);
+    const Ws ws = carve(workspace, n, L->E, L->H, L->I);
+    launch_prep(L, ws, x, x_dtype, rescale, n, topk, ids, offsets, order, active, nactive, nvalid, nvalid != nullptr, max_rows, s);
     launch_partial<0>(L, ws, n, s);
     launch_gu_epilogue(L, ws, n, s);
     launch_partial<1>(L, ws, n, s);
@@ -1077,7 +1072,7 @@ extern "C" {
 size_t mm_gemv_workspace(int n, int E, int H, int I)
 {
     if (n <= 0 || E <= 0 || H <= 0 || I <= 0) return 0;
-    return carve(nullptr, n, n, E, H, I).bytes;
+    return carve(nullptr, n, E, H, I).bytes;
 }
 
 int mm_expert_gemv(const mm_layer_t* L, const void* x, int x_dtype, int rescale, int T, int n, int topk,
@@ -1091,9 +1086,9 @@ int mm_expert_gemv(const mm_layer_t* L, const void* x, int x_dtype, int rescale,
     if (rc) return rc;
     MM_CHECK_ARG(Y || !(phases & 16), "mm_expert_gemv: null Y");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const Ws w = carve(workspace, n, n, L->E, L->H, L->I);
+    const Ws w = carve(workspace, n, L->E, L->H, L->I);
     if (phases & 1)
-        launch_prep(L, w, x, x_dtype, rescale, n, n, topk, ids, offsets, order, active, nactive,
+        launch_prep(L, w, x, x_dtype, rescale, n, topk, ids, offsets, order, active, nactive,
                     offsets ? offsets + L->E : nullptr, false, max_rows, s);
     if (phases & 2) launch_partial<0>(L, w, n, s);
     if (phases & 4) launch_gu_epilogue(L, w, n, s);

@@ -829,8 +829,7 @@ __device__ __forceinline__ int route_bin(const int64_t* ids, int s, int E)
 
 // Scatter routes [lo, hi) in order; fill[] (LDS) holds the next free sorted position of every bin.
 __device__ void scatter_chunk(const int64_t* ids, const float* w, int lo, int hi, int topk, int E, int* fill,
-                              int32_t* order, int32_t* token_sorted, float* weight_sorted, int32_t* inv_order,
-                              int32_t* e_sorted)
+                              int32_t* order, int32_t* token_sorted, float* weight_sorted, int32_t* inv_order)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     for (int base = lo; base < hi; base += blockDim.x)
@@ -859,7 +858,6 @@ __device__ void scatter_chunk(const int64_t* ids, const float* w, int lo, int hi
             if (token_sorted) token_sorted[pos] = s / topk;
             if (weight_sorted && w) weight_sorted[pos] = w[s];
             if (inv_order) inv_order[s] = pos;
-            if (e_sorted) e_sorted[pos] = e;
         }
         (void)lane;
     }
@@ -883,7 +881,7 @@ __device__ void write_active(const int* cnt, int E, int32_t* active, int32_t* na
 
 __global__ __launch_bounds__(PERM_THREADS) void k_permute_single(const int64_t* __restrict__ ids, const float* __restrict__ w,
     int n, int topk, int E, int32_t* counts, int32_t* offsets, int32_t* order, int32_t* token_sorted,
-    float* weight_sorted, int32_t* inv_order, int32_t* active, int32_t* nactive, int32_t* e_sorted)
+    float* weight_sorted, int32_t* inv_order, int32_t* active, int32_t* nactive)
 {
     __shared__ int cnt[1025 + 1];
     __shared__ int fill[1025 + 1];
@@ -911,7 +909,7 @@ __global__ __launch_bounds__(PERM_THREADS) void k_permute_single(const int64_t* 
     if (threadIdx.x == 0) offsets[nb] = run;
     write_active(cnt, E, active, nactive, scan_tmp);
     __syncthreads();
-    scatter_chunk(ids, w, 0, n, topk, E, fill, order, token_sorted, weight_sorted, inv_order, e_sorted);
+    scatter_chunk(ids, w, 0, n, topk, E, fill, order, token_sorted, weight_sorted, inv_order);
 }
 
 // Multi-block path: per-block bin histograms (bin-major), one-block scan, then per-block stable scatter.
@@ -963,14 +961,14 @@ __global__ __launch_bounds__(PERM_THREADS) void k_permute_scan(int32_t* hist, in
 
 __global__ __launch_bounds__(PERM_THREADS) void k_permute_scatter(const int64_t* __restrict__ ids, const float* __restrict__ w,
     int n, int topk, int E, int chunk, const int32_t* __restrict__ hist, int32_t* order, int32_t* token_sorted,
-    float* weight_sorted, int32_t* inv_order, int32_t* e_sorted)
+    float* weight_sorted, int32_t* inv_order)
 {
     __shared__ int fill[1025 + 1];
     const int nb = E + 1, B = gridDim.x, b = blockIdx.x;
     for (int e = threadIdx.x; e < nb; e += blockDim.x) fill[e] = hist[(size_t)e * B + b];
     __syncthreads();
     const int lo = b * chunk, hi = min(n, lo + chunk);
-    scatter_chunk(ids, w, lo, hi, topk, E, fill, order, token_sorted, weight_sorted, inv_order, e_sorted);
+    scatter_chunk(ids, w, lo, hi, topk, E, fill, order, token_sorted, weight_sorted, inv_order);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -1081,10 +1079,10 @@ __global__ __launch_bounds__(256) void k_synth_layer(const int64_t* __restrict__
     }
 }
 
-// mm_permute's launches; e_sorted (optional, [n]) receives the expert bin of each sorted position.
+// mm_permute's launches.
 int permute_launch(const int64_t* ids, const float* w, int n, int topk, int E, int32_t* counts, int32_t* offsets,
                    int32_t* order, int32_t* token_sorted, float* weight_sorted, int32_t* inv_order, int32_t* active,
-                   int32_t* nactive, int32_t* e_sorted, void* workspace, size_t workspace_bytes, mm_stream_t stream)
+                   int32_t* nactive, void* workspace, size_t workspace_bytes, mm_stream_t stream)
 {
     MM_CHECK_ARG(E > 0 && E <= 1024, "mm_permute: E must be in [1, 1024] (E=%d)", E);
     MM_CHECK_ARG(n >= 0 && topk > 0, "mm_permute: bad n/topk");
@@ -1096,7 +1094,7 @@ int permute_launch(const int64_t* ids, const float* w, int n, int topk, int E, i
     if (n <= PERM_SINGLE_MAX)
     {
         hipLaunchKernelGGL(k_permute_single, dim3(1), dim3(PERM_THREADS), 0, hs, ids, w, n, topk, E, counts, offsets,
-                           order, token_sorted, weight_sorted, inv_order, active, nactive, e_sorted);
+                           order, token_sorted, weight_sorted, inv_order, active, nactive);
     }
     else
     {
@@ -1106,7 +1104,7 @@ int permute_launch(const int64_t* ids, const float* w, int n, int topk, int E, i
         hipLaunchKernelGGL(k_permute_scan, dim3(1), dim3(PERM_THREADS), 0, hs, hist, B, n, E, counts, offsets, active,
                            nactive);
         hipLaunchKernelGGL(k_permute_scatter, dim3(B), dim3(PERM_THREADS), 0, hs, ids, w, n, topk, E, PERM_CHUNK, hist,
-                           order, token_sorted, weight_sorted, inv_order, e_sorted);
+                           order, token_sorted, weight_sorted, inv_order);
     }
     return check_launch("mm_permute");
 }
@@ -1222,7 +1220,7 @@ int mm_permute(const int64_t* ids, const float* w, int n, int topk, int E, int32
                int32_t* nactive, void* workspace, size_t workspace_bytes, mm_stream_t stream)
 {
     return mm::permute_launch(ids, w, n, topk, E, counts, offsets, order, token_sorted, weight_sorted, inv_order, active,
-                              nactive, nullptr, workspace, workspace_bytes, stream);
+                              nactive, workspace, workspace_bytes, stream);
 }
 
 int mm_combine(float* out, const float* Y, const int64_t* ids, const float* w, int T, int k, int H, int E, int accumulate,

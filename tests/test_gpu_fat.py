@@ -355,40 +355,6 @@ def test_fused_call_chosen_on_the_device_in_a_graph(dev):
         assert torch.equal(out, want), f"replay {step}"
 
 
-@pytest.mark.parametrize("more", [[], [1, 17, 32, 33, 64, 95, 96] * 2], ids=["folded", "all_sizes"])
-def test_tiles_of_a_whole_rounding_call(dev, more):
-    """Tiles of mm_grouped_gemm and mm_moe_prefill calls with many busy experts: remainders of 97 to 128 routes in 128-route
-    tiles, from 129 routes on in 256-route tiles (129, 176, 177, 255 and full ones, with remainders of 1, 96, 97 and 128
-    after them), and the shorter ones in 128-route tiles too where they are few, else in tiles of their own. Sampled rows of
-    every expert of both entries, whose rows are the same bits."""
-    import torch
-    from mi355moe import moe
-    H, I, seed = 256, 4096, 8383
-    tiles = -(-768 // (I // 128))                                   # three rounds of 256 workgroups
-    counts = [97, 112, 113, 128] * (tiles // 2) + [129, 176, 177, 255, 256, 257, 352, 353, 384] * 4 + [31, 32, 96] + more
-    rest = [c % 256 for c in counts]
-    assert sum(96 < r <= 128 for r in rest) >= 2 * tiles
-    assert sum(2 * (c // 256) + (r >= 129) + (r >= 177) for c, r in zip(counts, rest)) >= 2 * tiles
-    assert (sum(0 < r <= 96 for r in rest) <= tiles // 2) == (not more)
-    E = len(counts)
-    st = make_store(E, H, I, seed, device=dev, exact=True)
-    rng = np.random.default_rng(16)
-    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
-    T = ids.shape[0]
-    w = np.ones((T, 1), np.float32)
-    x16 = rng.normal(0, 1, (T, H)).astype(np.float16)
-    print(f"whole call tiles T={T} experts={E}", flush=True)
-    Y = moe.grouped_gemm(st, _t(x16, dev), _t(ids, dev), cap=0)
-    out = moe.moe_prefill(st, _t(x16, dev), _t(ids, dev), _t(w, dev))
-    torch.cuda.synchronize()
-    assert torch.equal(Y.half(), out.half())                        # the layer's rows pass through fp16
-    at = [np.flatnonzero(ids[:, 0] == e) for e in range(E)]
-    rows = np.concatenate([r[np.unique([0, len(r) // 2, min(96, len(r) - 1), min(128, len(r) - 1), len(r) - 1])] for r in at])
-    ref = OracleLayer(st, seed).forward(x16[rows].astype(np.float32), ids[rows], w[rows])
-    ok, m = within_tolerance(Y.cpu().numpy()[rows], ref)
-    assert ok, m
-
-
 def test_tiles_of_sorted_experts(dev):
     """apply_exl3_batched_fat takes 256-route tiles by the expert's own routes, from 768 on: 767 to 1,025 routes, every row
     against the oracle, and an expert computed alone has the bits it has among the others."""
@@ -423,37 +389,45 @@ def test_tiles_of_sorted_experts(dev):
         assert ok, (counts[e], m)
 
 
-def test_tiles_of_sorted_experts_of_a_large_layer(dev):
-    """apply_exl3_batched_fat of a layer with at least 80,000 routes and 200 per expert: every remainder in 256- or 128-route
-    tiles (1, 96, 97, 128, 129 and 255 routes among them); sampled rows of every expert against the oracle, and experts
-    computed alone have the bits they have among the others."""
+@pytest.mark.parametrize("more", [[], [1, 17, 32, 33, 64, 95, 96] * 2], ids=["folded", "all_sizes"])
+def test_tiles_of_a_large_rounding_layer(dev, more):
+    """Layers of at least 80,000 routes and 200 per expert: remainders of 97 to 128 routes in 128-route tiles, from 129 on in
+    256-route tiles (with remainders of 1, 96, 97 and 128 after full ones), and the shorter ones in 128-route tiles too where
+    the layer has few of them (an 18th of a round of workgroups here), else in tiles of their own. mm_grouped_gemm, mm_moe_prefill
+    and apply_exl3_batched_fat, the last in one call and in batches, give every row the same bits; sampled rows of every
+    expert against the oracle."""
     import torch
     from mi355moe import exl3, moe
-    H, I, seed = 256, 128, 8585
-    counts = [1, 96, 97, 128, 129, 255, 256 + 1, 256 + 128, 512 + 129]
-    counts.append(80000 - sum(counts))
+    H, I, seed = 256, 4096, 8585
+    counts = [97, 112, 113, 128, 129, 176, 255, 256, 257, 352, 353, 384, 31, 32, 96] + more
+    shorter = sum(0 < c % 256 <= 96 for c in counts)
+    counts.append(80256 - sum(counts) - (80256 - sum(counts)) % 256)
+    assert (shorter <= 12) == (not more) and 80000 <= sum(counts)   # half of 24 tiles = 768 workgroups of I / 128
     E = len(counts)
     st = make_store(E, H, I, seed, device=dev, exact=True)
     rng = np.random.default_rng(18)
     ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int64)[:, None]
     T = ids.shape[0]
     xd = torch.randn((T, H), generator=torch.Generator(device=dev).manual_seed(18), device=dev).half()
-    w = torch.ones((T, 1), device=dev)
-    r = moe.permute(_t(ids, dev), w, 1, E)
+    idd, w = _t(ids, dev), torch.ones((T, 1), device=dev)
+    r = moe.permute(idd, w, 1, E)
     tok, wts = r["token_sorted"].long(), r["weight_sorted"].half()
-    print(f"sorted experts of a large layer T={T}", flush=True)
+    print(f"large rounding layer T={T} experts={E}", flush=True)
 
     def run(skip):
         o = torch.zeros((T, H), dtype=torch.float32, device=dev)
         return exl3.apply_exl3_batched_fat(xd, tok, wts, counts, None, 10.0, 0, o, skip=skip, layer=st)
 
-    out = run(None)
-    parts = sum(run(set(range(E)) - set(b)) for b in ([0, 3], [1, 9], [2], [4, 5, 6], [7, 8]))
+    Y = moe.grouped_gemm(st, xd, idd, cap=0)
+    out = moe.moe_prefill(st, xd, idd, w)
+    whole = run(None)
+    parts = sum(run(set(range(E)) - set(range(b, E, 4))) for b in range(4))
     torch.cuda.synchronize()
-    assert torch.equal(out, parts)
-    rows = np.concatenate([np.flatnonzero(ids[:, 0] == e)[np.unique([0, c // 2, c - 1])] for e, c in enumerate(counts)])
+    assert torch.equal(Y.half().float(), out) and torch.equal(whole, out) and torch.equal(parts, out)
+    at = [np.flatnonzero(ids[:, 0] == e) for e in range(E)]
+    rows = np.concatenate([q[np.unique(np.minimum([0, len(q) // 2, 96, 128, len(q) - 1], len(q) - 1))] for q in at])
     ref = OracleLayer(st, seed).forward(xd[_t(rows, dev)].float().cpu().numpy(), ids[rows], np.ones((len(rows), 1), np.float32))
-    ok, m = within_tolerance(out.cpu().numpy()[rows], ref)
+    ok, m = within_tolerance(Y.cpu().numpy()[rows], ref)
     assert ok, m
 
 
