@@ -358,17 +358,21 @@ __global__ __launch_bounds__(FT_PLAN_MAX) void k_fat_plan(const int32_t* counts,
     if (scan(0, nbig) < rule.min_tiles) nbig = 0;                 // uniform: too few to fill the GPU
     __syncthreads();
     const int tbig = scan(0, nbig);
-    // the shorter remainders of the whole layer, computed here or not
-    int shorter = 0;
-    if (a < E)
+    int rest = max(c - nbig * FT_BIG, 0), nsmall = 0, tsmall = 0;
+    if (rule.min_small <= FT_SMALL)
     {
-        const int lc = max(layer_counts[a], 0), lr = lc - (lc >= rule.min_rows ? fat_big_tiles(lc, rule.min_rest) : 0) * FT_BIG;
-        shorter = lr > 0 && lr < rule.min_small ? 1 : 0;
+        // the shorter remainders of the whole layer, computed here or not
+        int shorter = 0;
+        if (a < E)
+        {
+            const int lc = max(layer_counts[a], 0);
+            const int lr = lc - (lc >= rule.min_rows ? fat_big_tiles(lc, rule.min_rest) : 0) * FT_BIG;
+            shorter = lr > 0 && lr < rule.min_small ? 1 : 0;
+        }
+        const bool fold = scan(1, shorter) <= rule.fold;
+        nsmall = rest > 0 && rest <= FT_SMALL && (fold || rest >= rule.min_small) ? 1 : 0;
+        tsmall = scan(5, nsmall);
     }
-    const bool fold = scan(1, shorter) <= rule.fold;
-    int rest = max(c - nbig * FT_BIG, 0);
-    const int nsmall = rest > 0 && rest <= FT_SMALL && (fold || rest >= rule.min_small) ? 1 : 0;
-    const int tsmall = scan(5, nsmall);
     if (nsmall) rest = 0;
     const int full = rest / FT_MID, r = rest % FT_MID;
     __syncthreads();
@@ -1537,9 +1541,9 @@ struct FatMode
 static FatMode fat_mode(const mm_layer_t* L, int n, bool fused)
 {
     const int units = L->I / 128, tiles = (FT_BIG_WORK + units - 1) / units, none = FT_SMALL + 1;
-    if (fused) return { (L->flags & MM_LAYER_EXACT) != 0, TileRule{ tiles, 0, FT_REST, none, -1 } };
+    if (fused) return { (L->flags & MM_LAYER_EXACT) != 0, TileRule{ tiles, 0, FT_REST, none, 0 } };
     if (n >= FT_LARGE && n / 200 >= L->E) return { true, TileRule{ 0, 0, FT_REST_LARGE, FT_MID + 1, tiles / 2 } };
-    return { true, TileRule{ 0, FT_BIG_ROWS, FT_REST, none, -1 } };
+    return { true, TileRule{ 0, FT_BIG_ROWS, FT_REST, none, 0 } };
 }
 
 // Expert records, row groups and tile lists of the sorted positions in ws (counts, offsets, active, nactive filled).
@@ -1571,7 +1575,8 @@ static int fat_gemms(const mm_layer_t* L, const void* x, int x_dtype, int T, int
     else prep(k_fat_prep<true>);
     // tiles of 128 and of 256 routes the call can have
     const int max_small = mode.rule.min_small <= FT_SMALL ? ws.max_small : 0;
-    const int max_big = ws.max_big >= mode.rule.min_tiles && n >= mode.rule.min_rows ? ws.max_big : 0;
+    const int most_big = n / mode.rule.min_rest;
+    const int max_big = most_big >= mode.rule.min_tiles && n >= mode.rule.min_rows ? most_big : 0;
     auto grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles * units + 7) & ~(size_t)7)); };    // >= 8 per_xcd
     auto mid_grid = [](int tiles, int units) { return dim3((unsigned)(((size_t)tiles + 7) / 8 * 8 * units)); };
     FatArgs g{ ws.rec, ws.big, ws.totals, ws.xa, L->svh13, L->suh2, L->svh2, ws.order, ws.xd, ws.Y,

@@ -345,8 +345,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_router_mfma(const uint16_t* __
 // workgroups still fit the GPU's CUs (RS_CUS) once, so every call of up to 512, 1,024 and, at two rounds, 4,096 tokens x 384
 // experts is one or two rounds deep. Router call, H 4096: 65 to 512 tokens 31 us (32 x 32 tiles), 700 and 1,024 tokens 40
 // (64 x 32; 55 with 32 x 32), 2,048 tokens 52 (64 x 48; 73 with 64 x 32), 4,096 tokens 96; the 128 x 192 tiles take 156 to
-// 162 us at all of these (12 to 64 workgroups) and 168 at 8,192 tokens, where 64 x 48 takes 181. Four steps in flight
-// instead of two: 34, 57 us.
+// 162 us at all of these (12 to 64 workgroups). The line of two rounds is on the safe side: three rounds of 64 x 48 (4,097 to
+// 6,144 tokens) take 127 to 144 us where the 128 x 192 tiles take 165 to 171, four 184 to 187 against 171 to 174, and so for 128
+// to 512 experts. Four steps in flight instead of two: 34, 57 us.
 constexpr size_t RS_CUS = 256;
 template <int MI, int NJ, int NW>
 __global__ __launch_bounds__(64 * NW) void k_router_split(const uint16_t* __restrict__ x, const float* __restrict__ G,

@@ -180,14 +180,15 @@ int mm_moe_decode_noalloc(const mm_layer_t* layer, const void* x, int x_dtype, i
 /* ------------------------------------------------------------------------------ fat experts (prefill) */
 
 /* Bytes of device workspace mm_grouped_gemm / mm_moe_prefill need for n routes over E experts (permutation,
- * per-expert records, transformed inputs, the down input and per-route outputs). */
+ * per-expert records, transformed inputs, the down input and per-route outputs): about 8 H + 2 I per route and, as an
+ * expert's inputs are held in groups of 32 rows, up to 32 (4 H + 2 I) for each of min(n, E) experts (250 MB at 384, H 4096). */
 size_t mm_prefill_workspace(int n, int E, int H, int I);
 
 /* Fat-expert grouped GEMM (replaces apply_exl3_batched_fat's per-expert reconstruct + 128x128 GEMM,
  * patches/vllm-exl3-host-dma.patch:182-201, and runtime/dma_gemm.py:5-26 run_batch, which feeds it): for every
  * route s < T*topk whose expert (0 <= ids[s] < E) has more than cap routes in the call, computes the expert
  * SwiGLU MLP and writes Y fp32 [T*topk][H] row s; other rows are left untouched. The weights are decoded into LDS
- * as fp16 (the reconstruct's rounding, ft_core.h:75-83) once per 96 or 256 routes and multiplied on MFMA; fp16
+ * as fp16 (the reconstruct's rounding, ft_core.h:75-83) once per 96, 128 or 256 routes and multiplied on MFMA; fp16
  * activations, fp32 accumulation, fp16 rounding at the reference's points. x, x_dtype as for mm_expert_gemv
  * (no rescale). Needs H a multiple of 256, I of 128, E <= 1024. */
 int mm_grouped_gemm(const mm_layer_t* layer, const void* x, int x_dtype, int T, int topk, const int64_t* ids, int cap,

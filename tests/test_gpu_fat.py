@@ -17,8 +17,8 @@ def _t(a, dev):
 
 
 def test_fat_expert_matches_reference_golden(dev):
-    """The two experts of the compiled reference's golden file, each fed 130 routes (one full 128-route tile and a
-    partial one), through the grouped GEMM: every route's row equals the reference's output."""
+    """The two experts of the compiled reference's golden file, each fed 130 routes (a tile of 96 and one of 34),
+    through the grouped GEMM: every route's row equals the reference's output."""
     import torch
     from mi355moe import moe
     g = np.load(os.path.join(GOLD, "expert_4096x2048.npz"), allow_pickle=False)
@@ -65,9 +65,8 @@ def test_fat_small_shapes_vs_oracle(dev, H, I, E, T, k):
 
 
 def test_fat_tile_boundaries(dev):
-    """Experts with 1, 128, 129, 192, 256 and 257 routes: 128-route tiles holding one route, 256-route tiles whose
-    second row half holds 1 or 64 routes (those waves skip their empty row blocks), a full tile, and a full tile
-    followed by a one-route tile."""
+    """Experts with 1, 128, 129, 192, 256 and 257 routes: tiles of up to 96 routes, full and with a remainder of one route or
+    of one or two row groups of 32 (the larger tiles: test_tiles_of_sorted_experts and the large-layer test)."""
     import torch
     from mi355moe import moe
     H, I, seed = 256, 128, 8080
@@ -120,7 +119,9 @@ def test_grouped_gemm_rows_of_fat_experts_only(dev):
 
 
 def test_threshold_split_matches_oracle(dev):
-    """moe_forward sends experts above the threshold to the grouped GEMM and the rest to the decode path."""
+    """moe_forward above the threshold, busy experts and experts with a few routes in one call of 240 routes (the decode
+    path takes it whole), and the same routes divided by the threshold over both paths: mm_moe_decode leaves out the experts
+    above max_rows, mm_moe_prefill with cap and accumulate adds them."""
     import torch
     from mi355moe import moe
     H, I, E, T, k = 512, 256, 8, 120, 2
@@ -135,9 +136,15 @@ def test_threshold_split_matches_oracle(dev):
     print(f"threshold split counts={counts.tolist()}", flush=True)
     assert (counts > 40).any() and ((counts > 0) & (counts <= 40)).any()
     out = moe.moe_forward(st, _t(x16, dev), _t(ids, dev), _t(w, dev), fat_threshold=40)
+    few = moe.decode_routes(st, _t(x16, dev), _t(ids, dev), _t(w, dev), 40)
+    split = moe.moe_prefill(st, _t(x16, dev), _t(ids, dev), _t(w, dev), cap=40, out=few.clone())
     torch.cuda.synchronize()
     ref = OracleLayer(st, seed).forward(x16.astype(np.float32), ids, w)
-    ok, m = within_tolerance(out.cpu().numpy(), ref)
+    for got in (out, split):
+        ok, m = within_tolerance(got.cpu().numpy(), ref)
+        assert ok, m
+    ok, m = within_tolerance(few.cpu().numpy(), OracleLayer(st, seed).forward(x16.astype(np.float32),
+                                                                              np.where(counts[ids] > 40, -1, ids), w))
     assert ok, m
 
 
@@ -198,9 +205,8 @@ def test_prefill_16k_tokens_deterministic_and_sampled(dev):
 
 @pytest.mark.parametrize("T,k,E,cap", [(600, 4, 40, 32), (90, 6, 24, 20)])
 def test_fused_moe_device_split_vs_oracle(dev, T, k, E, cap):
-    """mm_fused_moe: experts above cap on the grouped GEMM, the rest on the decode path, split on the device --
-    through the decode path's permutation (2,400 routes, positions bounded by E x cap) and its in-kernel routing
-    (540 routes)."""
+    """mm_fused_moe on the grouped GEMM (2,400 routes over 40 experts, 540 over 24), experts above and below cap, which
+    chooses nothing: two runs are bit-equal and match the oracle."""
     import torch
     from mi355moe import moe
     H, I = 512, 256

@@ -16,8 +16,8 @@ def _t(a, dev):
 
 
 def _tiles(c):
-    """Route tiles of an expert with c routes on the fat path: c // 256 tiles of 256, then a remainder above 128
-    in one more 256-route tile, else a 128-route tile. Returns [(first route, routes)]."""
+    """Route tiles of an expert with c routes in mm_moe_prefill of a layer this large: c // 256 tiles of 256, then a remainder
+    above 128 in one more 256-route tile, else one smaller tile (the fused call: from 193 on). Returns [(first route, routes)]."""
     out, r0 = [], 0
     for _ in range(c // 256):
         out.append((r0, 256))
@@ -29,9 +29,8 @@ def _tiles(c):
 
 def test_prefill_16k_skewed_routing_both_entries(dev):
     """The benchmark's 16k-token prefill routing (64 hot experts take 60 % of 131,072 routes, the others about
-    164 each), with one expert thinned to 20 routes so the decode path serves it at the image's threshold (32).
-    mm_moe_prefill (cap 32: fat experts only) and apply_exl3_fused_moe (threshold 32: fat GEMM + capped decode
-    path) are compared with the oracle on 16 sampled tokens: routes in the last tile of hot experts, routes in
+    164 each), with one expert thinned to 20 routes, below the image's threshold (32).
+    mm_moe_prefill (cap 32: fat experts only) and apply_exl3_fused_moe (the whole call on the grouped GEMM) are compared with the oracle on 16 sampled tokens: routes in the last tile of hot experts, routes in
     129-255-route tiles, routes of the thinned expert and random ones."""
     import torch
     from mi355moe import exl3, moe, workload
@@ -68,7 +67,7 @@ def test_prefill_16k_skewed_routing_both_entries(dev):
     cold = [e for e in range(E) if 128 < counts[e] < 256]
     for e in cold[:3]:
         pick += [tok_of(e, 0), tok_of(e, counts[e] - 1)]      # first and last route of a 129-255-route tile
-    pick += [tok_of(thin, 0), tok_of(thin, 19)]                # the thinned expert (decode path)
+    pick += [tok_of(thin, 0), tok_of(thin, 19)]                # the thinned expert
     rows = list(dict.fromkeys(pick))
     while len(rows) < 16:
         v = int(rng.integers(0, T))
@@ -244,8 +243,7 @@ def test_dsv41_shape_decode(dev, T):
 def test_dsv41_shape_prefill(dev):
     """DSV41 shape on the fat-expert path: 2048 tokens top-6 with skewed routing (hot experts about 115 routes,
     cold about 15): mm_moe_prefill with cap 0 (every expert on the grouped GEMM) and apply_exl3_fused_moe at the
-    image's threshold (hot experts on the GEMM, cold ones on the decode path), 6 sampled tokens against the
-    oracle."""
+    image's threshold (the whole call on the grouped GEMM), 6 sampled tokens against the oracle."""
     import torch
     from mi355moe import exl3, moe, workload
     H, I, E, T, K = 5120, 2304, 384, 2048, 6

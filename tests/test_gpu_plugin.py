@@ -1,5 +1,5 @@
 """GPU tests of the plugin entry points' argument handling: expert maps, the clamp switch, fp16 routing weights,
-fully masked calls, counts given as a device tensor, and the fat threshold split of the fused call."""
+fully masked calls, counts given as a device tensor, and fused calls above the fat threshold."""
 import numpy as np
 import pytest
 
@@ -54,8 +54,8 @@ def test_fused_moe_decode_call_semantics(dev):
 
 
 def test_fused_moe_fat_threshold_split(dev, monkeypatch):
-    """A prefill-sized call with the image's threshold (32): experts above it run on the grouped GEMM, the rest on
-    the decode path; the sum matches the oracle."""
+    """A call of more tokens than the image's threshold (32) with experts above and below it (240 routes: whole on the decode
+    path) matches the oracle."""
     import torch
     from mi355moe import exl3
     monkeypatch.setattr(exl3, "FAT_EXPERT_THRESHOLD", 32)
@@ -122,8 +122,8 @@ def test_expert_cache_synchronous_copies(dev):
 
 @pytest.mark.parametrize("T", [64, 200, 300])
 def test_fused_moe_captured_in_graph(dev, T):
-    """apply_exl3_fused_moe above the fat threshold (decode path with a cap plus the fat-expert GEMM, split on the
-    device) captures into a HIP graph; every replay, with eager work and synchronisations in between, equals the
+    """apply_exl3_fused_moe above the fat threshold (256 routes on the decode path, 800 and 1,200 on the grouped
+    GEMM) captures into a HIP graph; every replay, with eager work and synchronisations in between, equals the
     eager call bit for bit, and the eager call matches the oracle."""
     import torch
     from mi355moe import exl3
