@@ -300,7 +300,8 @@ __device__ __forceinline__ int fat_big_tiles(int c, int min_rest) { return c / F
 
 // Expert records, row groups and the tile lists of the experts with more than cap routes, one workgroup: thread a counts
 // expert a's tiles and groups, the lists are then filled by all threads, each entry finding its expert by a binary search
-// over the sums in LDS. totals = 256-route tiles, FT_MID-route tiles, row groups, 128-route tiles. The FT_MID-route list holds the tiles of
+// over the sums in LDS. totals = 256-route tiles, FT_MID-route tiles, row groups, 128-route tiles. The FT_MID-route list
+// holds the tiles of
 // three row groups first, then those of two, then those of one: the longest start first.
 // CHOICE (a fused call that either path may take, cap 0): the active experts and routed positions that the decode path is to
 // compute go to choice[0], [1]: all of them and no tile here, or none (see fused_path).
@@ -1554,8 +1555,8 @@ static void fat_plan(const mm_layer_t* L, int n, int cap, const FatWs& ws, hipSt
     const int E = L->E, na = n < E ? n : E;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(1), dim3(FT_PLAN_MAX), 0, s, ws.counts, ws.offsets, ws.active, ws.nactive, L->gate_ptr,
-                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.small, ws.mid, ws.groups, ws.totals, na, cap, mode.rule, layer_counts,
-                           choice, E, n);
+                           L->up_ptr, L->down_ptr, ws.rec, ws.big, ws.small, ws.mid, ws.groups, ws.totals, na, cap, mode.rule,
+                           layer_counts, choice, E, n);
     };
     if (choice) launch(k_fat_plan<true>);
     else launch(k_fat_plan<false>);

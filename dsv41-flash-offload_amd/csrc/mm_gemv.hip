@@ -3,9 +3,10 @@
 //
 // A layer runs as five launches on the caller's stream. Stream order is the only synchronisation (no fences,
 // no atomics between workgroups), so every result is deterministic:
-//   1. k_route_prep    one workgroup per (route, gate|up, 512 input rows), or per (route, gate|up) in larger calls: the
-//                      route's sorted position (stable by expert, then route index), the experts' records (one per active
-//                      expert, above 16 tokens one per 16 of its routes), and the route's transformed input xt = r16(FWHT128(x * suh) * HAD) in MFMA operand order, with its sums (the input
+//   1. k_route_prep    one workgroup per (route, gate|up, 512 input rows), or per (route, gate|up) in larger calls:
+//                      the route's sorted position (stable by expert, then route index), the experts' records (one
+//                      per active expert, above 16 tokens one per 16 of its routes), and the route's transformed
+//                      input xt = r16(FWHT128(x * suh) * HAD) in MFMA operand order, with its sums (the input
 //                      conversion and the optional unit-RMS rescale happen here too).
 //   2. k_partial<0>    gate/up partial sums, one launch that fills the GPU once: the work -- every
 //                      (record, matrix, 128 output columns) segment of 256 tile rows -- is cut into
@@ -35,11 +36,11 @@ namespace mm {
 constexpr int GV_WAVES = 4;
 constexpr int GV_THREADS = 64 * GV_WAVES;
 constexpr int GV_COLS = 128;          // output columns per segment (8 tiles)
-// Routes per record (one pass of a partial-sum wave) in calls of more than this many tokens. A segment costs
-// its waves one pass over its rows, whatever its routes, so equal runs of rows are equal work: with one record per expert
-// the waves of an expert with more than 16 routes took twice as long as the others and the launch waited for them (24
-// tokens, top-8 and the shared expert: 357 -> 304 us a call; 100 tokens on the decode path alone 741 us, against 884 with its
-// busy experts on the grouped GEMM). Fewer tokens keep one record per expert, found from a bitmap (the counts cost the
+// Routes per record (one pass of a partial-sum wave) in calls of more than this many tokens. A segment costs its waves one pass
+// over its rows, whatever its routes, so equal runs of rows are equal work: with one record per expert the waves of an expert with
+// more than 16 routes took twice as long as the others and the launch waited for them (24 tokens, top-8 and the shared expert:
+// 349 -> 296 us a call; 100 tokens on the decode path alone 741 us with route prep per 512 rows, 691 per row, against 884 with
+// its busy experts on the grouped GEMM). Fewer tokens keep one record per expert, found from a bitmap (the counts cost the
 // one-token layer 1 %); a token that picks an expert twice only makes a longer record.
 constexpr int REC_ROUTES = 16;
 constexpr int GV_RING = 4;            // tile rows in flight per wave (even: rows go through MFMA in pairs)
@@ -51,7 +52,8 @@ constexpr int PREP_WALK_MIN = 384;    // routes from which a permutation's route
 constexpr int SS_LOADS = 16;          // route prep: row elements per thread loaded at once for the rescale
 constexpr int MAX_TOPK = 16;
 
-// Rows of a partial launch: nseg (records x matrices x column blocks) segments of KT tile rows each (KT a multiple of 8), in segment order, cut into
+// Rows of a partial launch: nseg (records x matrices x column blocks) segments of KT tile rows each (KT a multiple of
+// 8), in segment order, cut into
 // nw runs of equal length (within 4 rows) that start and end on multiples of 4 rows, one per wave, so every wave
 // streams as many rows as every other. A run that reaches the end of a segment goes on in the next one; the wave
 // then computes one piece of each, and a segment's pieces are the runs that meet it, numbered from 0 in row

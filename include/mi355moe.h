@@ -138,10 +138,10 @@ size_t mm_gemv_workspace(int n, int E, int H, int I);
  * The expert input of token t is x[t] (x_dtype MM_DTYPE_*) converted to fp16: fp16 input is used as is, other
  * types go through bf16 (RNE); with rescale != 0 the row is first scaled to unit RMS (any type), as
  * mm_prepare_input does. Routes are found in-kernel from ids when offsets is NULL (n <= 1024); otherwise
- * offsets/order/active/nactive from mm_permute over the same routes are used, with the same results bit for bit. max_rows (>= 1) is the fat-expert
- * threshold of the call: an expert with more than max_rows routes is left to the fat-expert path (its rows stay
- * untouched here), so a caller can split a call between both paths without reading the counts on the host;
- * max_rows >= n computes every route. Any number of routes per expert is supported (the trellis is streamed once
+ * offsets/order/active/nactive from mm_permute over the same routes are used, with the same results bit for bit.
+ * max_rows (>= 1) is the fat-expert threshold of the call: an expert with more than max_rows routes is left to the
+ * fat-expert path (its rows stay untouched here), so a caller can split a call between both paths without reading
+ * the counts on the host; max_rows >= n computes every route. Any number of routes per expert is supported (the trellis is streamed once
  * per 16 routes of an expert). phases is a mask of the five launches, run in this order on the same workspace:
  * 1 = route prep and input transform, 2 = gate/up partial sums, 4 = gate/up epilogue (output transforms, SwiGLU,
  * down-input transform), 8 = down partial sums, 16 = down epilogue into Y; 31 = the whole expert MLP. */
