@@ -41,14 +41,15 @@ constexpr int FT_SMALL = 128;       // routes per tile of k_fat16<*, 2>
 //   a fused call: 256-route tiles where it has at least three rounds (FT_BIG_WORK workgroups) of them, the rest in FT_MID-route
 //     tiles. 3 tiles (48 workgroups) of a 512-token call took 214 us of its 1,540 where FT_MID-route tiles took 60; at 64 tiles
 //     (4,096 tokens) both GEMMs take 2.68 ms with them and 2.84 without, at 297 (16,384 tokens) 8.25 and 8.65.
-//   the other entry points, whose rows must have the same bits whichever experts of a layer a call computes (a layer in one call
-//     or in staging batches): by the expert's routes and the layer's. From 768 routes on 256-route tiles: a staging batch of 16 experts
-//     holds few (12 took 189 us of its 470, as FT_MID-route tiles 50). In layers of more than FT_LARGE routes and 200 per
-//     expert, from a remainder of 129 routes on, and remainders of 97 to 128 routes in 128-route tiles (k_mid costs more with
-//     rounded weights, 55 against 34 ns per 16 x 16 tile and SIMD); the shorter ones too where the layer has under one and a
-//     half rounds of them (a launch of a few k_mid workgroups takes 99 + 50 us). mm_moe_prefill of 16,384 tokens by the first / by this
-//     rule, ms: H 5120 10.91 / 10.35 (64 hot experts), 10.94 / 10.05 (even routing), H 4096 10.50 / 9.60 (even); 16 staged experts
-//     0.84 / 0.73. At 8,192 tokens staged experts take 0.48 ms by the first rule and 0.55 by this, the whole layer 5.5 and 5.3.
+//   the other entry points, whose rows must have the same bits whichever experts of a layer a call computes (a layer in one
+//     call or in staging batches): by the expert's routes and the layer's. From 768 routes on 256-route tiles: a staging batch
+//     of 16 experts holds few (12 took 189 us of its 470, as FT_MID-route tiles 50). In layers of at least FT_LARGE routes and
+//     200 per expert, from a remainder of 129 routes on, and remainders of 97 to 128 routes in 128-route tiles (two FT_MID-route
+//     tiles otherwise: 0.55 against 0.34 us per expert and column unit at H 5120); the shorter ones too where the layer has
+//     under one and a half rounds of them (a launch of a few k_mid workgroups takes 99 + 50 us). mm_moe_prefill of 16,384
+//     tokens by the first / by this rule, ms: H 5120 10.91 / 10.4 (64 hot experts), 10.94 / 10.05 (even routing), H 4096
+//     10.50 / 9.60 (even); 16 staged experts 0.84 / 0.73. At 8,192 tokens staged experts take 0.48 ms by the first rule and
+//     0.55 by this, the whole layer 5.5 and 5.3.
 struct TileRule
 {
     int min_tiles;      // 256-route tiles of the call
