@@ -1771,10 +1771,6 @@ int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int top
     MM_CHECK_ARG(w && out && cap >= 1, "mm_fused_moe: null pointer or cap < 1");
     MM_CHECK_ARG(topk <= 16, "mm_fused_moe: topk must be at most 16");
     const int n = T * topk, E = L->E;
-    // a limit of the interface: n, or E x cap for larger n, transformed inputs within 32-bit byte offsets
-    const size_t npos = n <= GV_ROUTE_MAX ? (size_t)n : (size_t)std::min<int64_t>(n, (int64_t)E * cap);
-    MM_CHECK_ARG(npos * 2 * std::max(L->H, L->I) * 2 < ((size_t)1 << 31),
-                 "mm_fused_moe: too many decode-path positions (%zu)", npos);
     const size_t need = fused_bytes(n, E, L->H, L->I);
     MM_CHECK_ARG(workspace && workspace_bytes >= need, "mm_fused_moe: workspace too small (%zu < %zu)", workspace_bytes,
                  need);

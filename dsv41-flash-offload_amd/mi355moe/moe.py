@@ -133,7 +133,7 @@ def moe_forward(store, x, ids, w, shared_expert=None, fat_threshold=FAT_THRESHOL
 
 def fused_moe(store, x, ids, w, cap, stream=None):
     """mm_fused_moe: out fp32 [T, H] over ids [T, k] / w [T, k], on the decode path (few routes, or few per expert) or the
-    grouped GEMM; `cap` is the reference's threshold between the two and only bounds the call's size."""
+    grouped GEMM; `cap` is the reference's threshold between the two and chooses nothing."""
     T, k = ids.shape
     x = x.contiguous()
     ids = ids.contiguous().long()

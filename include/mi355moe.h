@@ -207,12 +207,11 @@ int mm_moe_prefill(const mm_layer_t* layer, const void* x, int x_dtype, int T, i
  * group kernel): out fp32 [T][H] = sum_j w[t,j] * expert_{ids[t,j]}(x_t) over the valid routes, added in ascending
  * j. The call runs as a whole on the decode path or on the grouped GEMM: up to 1,024 routes by their number (384, or 10
  * per expert, and fewer on the decode path), above on the grouped GEMM unless the experts get few routes each, where the
- * device chooses from the routes' experts. cap, the reference's threshold between its two paths, chooses nothing and
- * bounds the call's size as before: n, or E x cap of more than 1,024, transformed inputs below 2 GiB. Weights follow the
- * layer's codebook evaluation (MM_LAYER_EXACT or not), except in tiles of 256 routes, which round them to fp16 as the
- * reference's reconstruct does. No host synchronisation: the call can be captured. ids int64 [T*topk], w fp32 [T*topk],
- * topk <= 16, cap >= 1; x as for mm_moe_prefill. Workspace: mm_fused_moe_workspace(T, topk, E, H, I, cap)
- * bytes, which also hold every call of fewer tokens. */
+ * device chooses from the routes' experts. cap, the reference's threshold between its two paths, is checked (at least
+ * 1) and chooses nothing. Weights follow the layer's codebook evaluation (MM_LAYER_EXACT or not), except in tiles of 256
+ * routes, which round them to fp16 as the reference's reconstruct does. No host synchronisation: the call can be
+ * captured. ids int64 [T*topk], w fp32 [T*topk], topk <= 16, cap >= 1; x as for mm_moe_prefill. Workspace:
+ * mm_fused_moe_workspace(T, topk, E, H, I, cap) bytes, which also hold every call of fewer tokens. */
 size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap);
 int mm_fused_moe(const mm_layer_t* layer, const void* x, int x_dtype, int T, int topk, const int64_t* ids,
                  const float* w, int cap, float* out, void* workspace, size_t workspace_bytes, mm_stream_t stream);

@@ -102,6 +102,24 @@ def test_fused_workspace_holds_every_smaller_call(E, H, I, k):
         had = ws
 
 
+@pytest.mark.parametrize("T,cap", [(16384, 32), (16384, 400), (16384, 1 << 30), (128, 400)])
+def test_fused_call_is_not_refused_by_its_threshold(T, cap):
+    """A fused call of 16,384 tokens, top-8 of 384 experts at H 4096 passes the argument checks whatever the threshold
+    (E x cap positions of 400 would pass 2 GiB of inputs, but no path holds them) and fails on the missing workspace; thresholds
+    below 1 and more routes than the decode path can address on it stay errors."""
+    import ctypes
+    from mi355moe import _lib
+    L = _lib.load()
+    lay = _lib.MMLayer(*([256] * 7), 384, 4096, 2048, 10.0, 0)
+    rc = L.mm_fused_moe(ctypes.byref(lay), 256, 0, T, 8, 256, 256, cap, 256, 256, 0, None)
+    assert rc == -1 and b"workspace too small" in L.mm_last_error(), L.mm_last_error()
+    rc = L.mm_fused_moe(ctypes.byref(lay), 256, 0, T, 8, 256, 256, 0, 256, 256, 1 << 40, None)
+    assert rc == -1 and b"cap < 1" in L.mm_last_error()
+    wide = _lib.MMLayer(*([256] * 7), 384, 1 << 19, 128, 10.0, 0)
+    rc = L.mm_fused_moe(ctypes.byref(wide), 256, 0, 128, 8, 256, 256, cap, 256, 256, 1 << 50, None)
+    assert rc == -1 and b"too many routes" in L.mm_last_error(), L.mm_last_error()
+
+
 def test_expert_seed_matches_oracle():
     import oracle as O
     from mi355moe import _lib
