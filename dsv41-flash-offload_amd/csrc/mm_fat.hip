@@ -1691,22 +1691,28 @@ static FatbWs fatb_carve(void* base, int n, int T, int E, int H, int I)
 //   E 128: n 800 470 / 535 u, 488 / 518 z; 1,024 488 / 532, 539 / 531; 1,600 586 / 552, 679 / 574
 //   E 256: n 1,024 861 / 957 u, 731 / 763 z; 2,048 932 / 993, 1,043 / 946; 3,200 1,104 / 1,002, 1,341 / 1,054
 //   E 384: n 1,024 1,141 / 1,326 u, 879 / 907 z, 249 / 174 8; 2,048 1,295 / 1,414, 1,252 / 1,146, 475 / 225
-// So up to GV_ROUTE_MAX routes the decode path (routed in-kernel) takes 384 routes or 10 per expert; what the host cannot see
-// is left there: tokens that agree on a few of many experts. Above, the permutation is needed in any case, and while experts
+//   H 2048, I 1024, E 64: n 800 109 / 119 u, 118 / 129 z; 1,024 134 / 121, 138 / 146.  H 1024, I 512, E 32: n 512 52 / 63 u
+// Both paths cost an expert's decode per record or tile, and the grouped GEMM about 40 us more in launches, which is 220
+// routes of the decode path at H 4096, I 2048. So up to GV_ROUTE_MAX routes the decode path (routed in-kernel) takes 10 routes
+// per expert and those, at least 384; what the host cannot see is left there: tokens that agree on a few of many experts. Above, the permutation is needed in any case, and while experts
 // get few routes (7 each on average; 9 to 1,280 routes) the plan kernel chooses on the device by records and tiles: decode path
 // 40 + 3.05 records + n / 33 us, grouped GEMM 80 + 3.45 tiles us, within 5 % of the above. The launches of the path not taken
 // find no work (25-30 us in all), so calls of small layers, in the end faster than that, are not given the choice (E H I below
 // 2^30: 512 experts, H 2048, I 512, 2,500 routes take 290 us on the grouped GEMM and 330 chosen). With more routes the experts
 // are busy enough for the grouped GEMM.
 enum class FusedPath { DECODE, CHOICE, GEMM };
-static int fused_most_decode(int E) { return std::min(GV_ROUTE_MAX, std::max(384, 10 * E)); }
+constexpr int64_t FUSED_LAUNCHES = (int64_t)220 * 4096 * 2048;
+static int fused_most_decode(int E, int H, int I)
+{
+    return (int)std::min<int64_t>(GV_ROUTE_MAX, std::max<int64_t>(384, 10 * E + FUSED_LAUNCHES / ((int64_t)H * I)));
+}
 static int fused_most_choice(int E, int H, int I)
 {
     return (int64_t)E * H * I >= (int64_t)1 << 30 ? std::min(9 * E, std::max(7 * E, 1280)) : 0;
 }
 static FusedPath fused_path(int n, int E, int H, int I)
 {
-    if (n <= GV_ROUTE_MAX) return n <= fused_most_decode(E) ? FusedPath::DECODE : FusedPath::GEMM;
+    if (n <= GV_ROUTE_MAX) return n <= fused_most_decode(E, H, I) ? FusedPath::DECODE : FusedPath::GEMM;
     return n <= fused_most_choice(E, H, I) && decode_fits(n, E, H, I) ? FusedPath::CHOICE : FusedPath::GEMM;
 }
 
@@ -1756,11 +1762,11 @@ size_t mm_fused_moe_workspace(int T, int topk, int E, int H, int I, int cap)
     if (T <= 0 || topk <= 0 || E <= 0 || H <= 0 || I <= 0 || cap < 0) return 0;
     const int n = T * topk;
     // enough for every smaller call too, whichever path it takes
-    size_t bytes = decode_workspace_upto(std::min(n, fused_most_decode(E)), E, H, I);
+    size_t bytes = decode_workspace_upto(std::min(n, fused_most_decode(E, H, I)), E, H, I);
     const int choice = std::min(n, fused_most_choice(E, H, I));
     if (choice > GV_ROUTE_MAX)
         bytes = std::max(bytes, fused_carve(nullptr, choice, E, H, I, decode_workspace_upto(choice, E, H, I)).bytes);
-    return n > fused_most_decode(E) ? std::max(bytes, fat_carve(nullptr, n, E, H, I).bytes) : bytes;
+    return n > fused_most_decode(E, H, I) ? std::max(bytes, fat_carve(nullptr, n, E, H, I).bytes) : bytes;
 }
 
 int mm_fused_moe(const mm_layer_t* L, const void* x, int x_dtype, int T, int topk, const int64_t* ids, const float* w,

@@ -206,7 +206,7 @@ int mm_moe_prefill(const mm_layer_t* layer, const void* x, int x_dtype, int T, i
  * the fat threshold routes through the fat-expert GEMM, patch:286-291,450-460, the others through the fused
  * group kernel): out fp32 [T][H] = sum_j w[t,j] * expert_{ids[t,j]}(x_t) over the valid routes, added in ascending
  * j. The call runs as a whole on the decode path or on the grouped GEMM: up to 1,024 routes by their number (384, or 10
- * per expert, and fewer on the decode path), above on the grouped GEMM unless the experts get few routes each, where the
+ * per expert and more in small layers, and fewer on the decode path), above on the grouped GEMM unless the experts get few routes each, where the
  * device chooses from the routes' experts. cap, the reference's threshold between its two paths, is checked (at least
  * 1) and chooses nothing. Weights follow the layer's codebook evaluation (MM_LAYER_EXACT or not), except in tiles of 256
  * routes, which round them to fp16 as the reference's reconstruct does. No host synchronisation: the call can be

@@ -122,8 +122,8 @@ def test_expert_cache_synchronous_copies(dev):
 
 @pytest.mark.parametrize("T", [64, 200, 300])
 def test_fused_moe_captured_in_graph(dev, T):
-    """apply_exl3_fused_moe above the fat threshold (256 routes on the decode path, 800 and 1,200 on the grouped
-    GEMM) captures into a HIP graph; every replay, with eager work and synchronisations in between, equals the
+    """apply_exl3_fused_moe above the fat threshold (256 and 800 routes on the decode path, 1,200 on the
+    grouped GEMM) captures into a HIP graph; every replay, with eager work and synchronisations in between, equals the
     eager call bit for bit, and the eager call matches the oracle."""
     import torch
     from mi355moe import exl3
